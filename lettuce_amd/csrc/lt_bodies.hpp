@@ -227,26 +227,13 @@ __device__ __forceinline__ double body_qdensity_site(const double2* __restrict__
 // spills; body_clover_deriv_all runs the halves as a loop with the running sum and one
 // partial product parked in LDS.
 
-// neighbour steps in a direction known only at run time (selects instead of indexing
-// the extents, which would put them in scratch)
-__device__ __forceinline__ int up_rt(const Geom& g, int s, int cm, int d)
-{
-    const int L = pick4(g.L, d), st = pick4(g.st, d);
-    return (cm + 1 < L) ? s + st : s - (L - 1) * st;
-}
-__device__ __forceinline__ int dn_rt(const Geom& g, int s, int cm, int d)
-{
-    const int L = pick4(g.L, d), st = pick4(g.st, d);
-    return (cm > 0) ? s - st : s + (L - 1) * st;
-}
-
 // Re tr of the plaquette U_mu(x) U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+ (plaquette.hpp:20-24)
 // as Re tr(A B^+) with A = U_mu(x) U_nu(x+mu), B = U_nu(x) U_mu(x+nu), both in SU(3), of
 // which only rows 0 and 1 are multiplied out (retr_su3_nd_r01).
 __device__ __forceinline__ double plaq_plane(const double2* __restrict__ U, const Geom& g, int s, const int c[4],
                                             int par, int mu, int nu)
 {
-    const int smu = up_rt(g, s, pick4(c, mu), mu), snu = up_rt(g, s, pick4(c, nu), nu);
+    const int smu = up(g, s, pick4(c, mu), mu), snu = up(g, s, pick4(c, nu), nu);
     const M3 A = mul_r01(ldu2(U, g, s, mu, par), ldu(U, g, smu, nu, par ^ 1));
     const M3 B = mul_r01(ldu2(U, g, s, nu, par), ldu(U, g, snu, mu, par ^ 1));
     return retr_su3_nd_r01(A, B);
@@ -291,7 +278,7 @@ __device__ __forceinline__ M3 cderiv_upper(const double2* __restrict__ U, const 
                                            double2* park, int n)
 {
     const int q = par ^ 1;
-    const int smu = up_rt(g, s, pick4(c, MU), MU), snu = up_rt(g, s, pick4(c, NU), NU);
+    const int smu = up(g, s, pick4(c, MU), MU), snu = up(g, s, pick4(c, NU), NU);
     const M3 Unu_x = ldu(U, g, s, NU, par);
     M3 tmp1, tmp2;
     {
@@ -304,7 +291,7 @@ __device__ __forceinline__ M3 cderiv_upper(const double2* __restrict__ U, const 
     M3 acc = mul(tmp1, S);
     if (park) park_store(park, n, acc);
     const M3 Unu_mu = ldu(U, g, smu, NU, q);
-    S = mul(Unu_mu, R_at(C, g, up_rt(g, smu, pick4(c, NU), NU), par, RHO, SIGMA));
+    S = mul(Unu_mu, R_at(C, g, up(g, smu, pick4(c, NU), NU), par, RHO, SIGMA));
     S = add(S, mul(R_at(C, g, smu, q, RHO, SIGMA), Unu_mu));
     const M3 second = mul(S, tmp2);
     if (park) acc = park_load(park, n);
@@ -316,8 +303,8 @@ __device__ __forceinline__ M3 cderiv_lower(const double2* __restrict__ U, const 
                                            double2* park, int n)
 {
     const int q = par ^ 1;
-    const int smu = up_rt(g, s, pick4(c, MU), MU);
-    const int snd = dn_rt(g, s, pick4(c, NU), NU), smu_nd = dn_rt(g, smu, pick4(c, NU), NU);
+    const int smu = up(g, s, pick4(c, MU), MU);
+    const int snd = dn(g, s, pick4(c, NU), NU), smu_nd = dn(g, smu, pick4(c, NU), NU);
     const M3 Unu_nd = ldu(U, g, snd, NU, q);
     const M3 Unu_mund = ldu(U, g, smu_nd, NU, par);
     M3 tmp3, tmp4;
@@ -463,13 +450,13 @@ __device__ __forceinline__ void body_sigma_all(const double2* __restrict__ U, do
     double2* fs_slot = lds + threadIdx.x;
     double2* st_slot = fs_slot + 9 * n;
     const int q = par ^ 1;
-    const int smu = up_rt(g, s, pick4(c, mu), mu);
+    const int smu = up(g, s, pick4(c, mu), mu);
 #pragma unroll 1
     for (int k = 0; k < 3; ++k) {
         const int nu = k < mu ? k : k + 1;
         const int cnu = pick4(c, nu);
-        const int snu = up_rt(g, s, cnu, nu), snd = dn_rt(g, s, cnu, nu);
-        const int smu_nd = dn_rt(g, smu, cnu, nu);
+        const int snu = up(g, s, cnu, nu), snd = dn(g, s, cnu, nu);
+        const int smu_nd = dn(g, smu, cnu, nu);
         const M3 Unu_x = ldu(U, g, s, nu, par);
         const M3 Unu_mu = ldu(U, g, smu, nu, q);
         M3 tmp1;

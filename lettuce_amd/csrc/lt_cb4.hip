@@ -44,19 +44,20 @@ __global__ void LT_LINK_KERNEL hb_cb4_graph_kernel(double2* __restrict__ U, Geom
     update_link<true>(U, g, s, c, mu, parity_of(c), prefactor, seed, state[0] + (uint64_t)k);
 }
 
-// Rectangular<R>(beta, c_plaq, c_rect) sweeps; the rectangle staple's sum waits in LDS
-// between its terms (9 x 16 bytes per lane: two waves per SIMD without spills, against
-// one wave and 22 spilled VGPRs when it stays in registers)
-template <bool HEATBATH>
-__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2)))
+// Six wavefronts per 64 links (update_links_action): three waves per SIMD, 20 spilled
+// VGPRs.  One lane per link with the sum parked in LDS ran about 9500 FP64 instructions in
+// a row at two waves per SIMD, and a 24^4 launch was 1296 waves on 1024 SIMDs: 186 us per
+// overrelaxation launch there, 322 us at 32^4; now 85 and 207 us (heatbath 195 -> 93 us at
+// 24^4).  What bounds it now is the latency of the twelve link loads of a part, about half
+// of whose lines miss the L2, at one load in flight ahead of the products.
+template <bool HEATBATH, bool RECT>
+__global__ void __launch_bounds__(ACT_BS) __attribute__((amdgpu_waves_per_eu(3)))
 sweep_action_kernel(double2* __restrict__ U, Geom g, int mu, int colour, double prefactor, uint64_t seed,
-                    uint64_t counter, double c_plaq, double c_rect)
+                    uint64_t counter, double c_plaq, double c_rect, int tc)
 {
-    extern __shared__ double2 lds[];
-    int c[4], s;
-    if (!cb4_site(g, mu, colour, xcd_block_dir(blockIdx.x, gridDim.x, colour & 1) * BS + threadIdx.x, c, s)) return;
-    update_link_action<HEATBATH>(U, g, s, c, mu, parity_of(c), prefactor, seed, counter, c_plaq, c_rect,
-                                 lds + threadIdx.x, BS);
+    __shared__ double2 lds[27 * ACT_LINKS];
+    update_links_action<HEATBATH, RECT>(U, g, mu, colour, xcd_block_dir(blockIdx.x, gridDim.x, colour & 1), prefactor, seed,
+                                  counter, c_plaq, c_rect, tc, lds);
 }
 
 // PlaquetteSum block partials of a captured four-colour update (the field is in the
@@ -115,13 +116,17 @@ void k_cb4_colour_graph_hb(lt_field u, int mu, int colour, double prefactor, con
 void k_cb4_colour_action(lt_field u, bool heatbath, int mu, int colour, double prefactor, uint64_t counter,
                          double c_plaq, double c_rect, const char* name)
 {
-    const dim3 grid(nblocks(u->g.V / 4, BS)), block(BS);
-    if (heatbath)
-        launch(u->ctx, name, sweep_action_kernel<true>, grid, block, 9 * BS * sizeof(double2), u->d, u->g, mu, colour,
-               prefactor, u->seed, counter, c_plaq, c_rect);
-    else
-        launch(u->ctx, name, sweep_action_kernel<false>, grid, block, 9 * BS * sizeof(double2), u->d, u->g, mu, colour,
-               prefactor, u->seed, counter, c_plaq, c_rect);
+    const dim3 grid(nblocks(u->g.V / 4, ACT_LINKS)), block(ACT_BS);
+    const bool rect = c_rect != 0.0;
+    const Geom& g = u->g;
+    // the largest divisor of Nt that leaves each of the eight XCDs a chunk of timeslices of its own
+    int tc = 1;
+    if ((g.V / g.L[0]) % (4 * ACT_LINKS) == 0)
+        for (int d = 2; d <= (g.L[0] + 7) / 8; ++d)
+            if (g.L[0] % d == 0) tc = d;
+    auto* k = heatbath ? (rect ? sweep_action_kernel<true, true> : sweep_action_kernel<true, false>)
+                       : (rect ? sweep_action_kernel<false, true> : sweep_action_kernel<false, false>);
+    launch(u->ctx, name, k, grid, block, 0, u->d, u->g, mu, colour, prefactor, u->seed, counter, c_plaq, c_rect, tc);
 }
 
 void k_cb4_plaq_partials(lt_field u, double* part)

@@ -695,6 +695,15 @@ __device__ __forceinline__ size_t slot_base(const Geom& g, int a, int nslot, int
 }
 __device__ __forceinline__ size_t slot_stride(const Geom& g) { return (size_t)g.Vh; }
 
+// v[i] for an index known only at run time, as four masked values: nested conditionals on
+// kernel arguments become a tree of branches, which cuts every kernel that works with
+// run-time directions into pieces that the compiler cannot schedule across.
+__device__ __forceinline__ int pick4(const int v[4], int i)
+{
+    const int a = v[0], b = v[1], c = v[2], d = v[3];
+    return (a & -(int)(i == 0)) | (b & -(int)(i == 1)) | (c & -(int)(i == 2)) | (d & -(int)(i == 3));
+}
+
 __device__ __forceinline__ void coords_of(const Geom& g, int s, int c[4])
 {
     c[3] = s % g.L[3];
@@ -707,11 +716,13 @@ __device__ __forceinline__ void coords_of(const Geom& g, int s, int c[4])
 // site index one step along +mu / -mu given the coordinate of that direction
 __device__ __forceinline__ int up(const Geom& g, int s, int cmu, int mu)
 {
-    return (cmu + 1 < g.L[mu]) ? s + g.st[mu] : s - (g.L[mu] - 1) * g.st[mu];
+    const int L = pick4(g.L, mu), st = pick4(g.st, mu);
+    return (cmu + 1 < L) ? s + st : s - (L - 1) * st;
 }
 __device__ __forceinline__ int dn(const Geom& g, int s, int cmu, int mu)
 {
-    return (cmu > 0) ? s - g.st[mu] : s + (g.L[mu] - 1) * g.st[mu];
+    const int L = pick4(g.L, mu), st = pick4(g.st, mu);
+    return (cmu > 0) ? s - st : s + (L - 1) * st;
 }
 
 // Element i of a buffer.  With LT_ADDR32 the byte offset is a 32-bit value added to
@@ -1118,7 +1129,7 @@ __device__ __forceinline__ int site_of_cb(const Geom& g, int cb, int par, int c[
 __device__ __forceinline__ M3 staple(const double2* __restrict__ U, const Geom& g, int s, const int c[4], int mu)
 {
     const int par = (c[0] + c[1] + c[2] + c[3]) & 1;
-    const int s_mu = up(g, s, c[mu], mu);
+    const int s_mu = up(g, s, pick4(c, mu), mu);
     M3 st;
 #pragma unroll
     for (int nu = 0, k = 0; nu < 4; ++nu) {
@@ -1126,7 +1137,7 @@ __device__ __forceinline__ M3 staple(const double2* __restrict__ U, const Geom& 
         const int cnu = c[nu];
         const int s_nu = up(g, s, cnu, nu);
         const int s_nd = dn(g, s, cnu, nu);
-        const int s_nd_mu = up(g, s_nd, c[mu], mu);
+        const int s_nd_mu = up(g, s_nd, pick4(c, mu), mu);
         {
             const M3 ab = mul_r01(ldu2(U, g, s, nu, par), ldu(U, g, s_nu, mu, par ^ 1));
             const M3 t = mul_nd_r01(ab, ldu(U, g, s_mu, nu, par ^ 1));
@@ -1171,8 +1182,6 @@ __device__ __forceinline__ M3 su3_of(const Raw6& r)
     third_row(a);
     return a;
 }
-__device__ __forceinline__ int pick4(const int v[4], int i) { return i == 0 ? v[0] : i == 1 ? v[1] : i == 2 ? v[2] : v[3]; }
-
 // The staple of staple() as six terms (upper and lower for each nu != mu, nu
 // ascending, the same products and summation order), software-pipelined: the
 // three links of term j+1 are loaded before term j is multiplied out, with
@@ -1182,7 +1191,7 @@ __device__ __forceinline__ M3 staple_pipelined(const double2* __restrict__ U, co
                                                int mu, int par, Raw6& own)
 {
     const int q = par ^ 1;
-    const int s_mu = up(g, s, c[mu], mu);
+    const int s_mu = up(g, s, pick4(c, mu), mu);
     int s_nu[3], s_nd[3], s_ndmu[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -1190,7 +1199,7 @@ __device__ __forceinline__ M3 staple_pipelined(const double2* __restrict__ U, co
         const int cnu = pick4(c, nu), L = pick4(g.L, nu), st = pick4(g.st, nu);
         s_nu[k] = (cnu + 1 < L) ? s + st : s - (L - 1) * st;
         s_nd[k] = (cnu > 0) ? s - st : s + (L - 1) * st;
-        s_ndmu[k] = up(g, s_nd[k], c[mu], mu);
+        s_ndmu[k] = up(g, s_nd[k], pick4(c, mu), mu);
     }
     // term j = 2k: a = U_nu(x) [rows 0, 1], b = U_mu(x+nu), cc = U_nu(x+mu):  (a b) cc^+
     // term j = 2k+1: a = U_mu(x-nu) [rows 0, 1], b = U_nu(x-nu+mu), cc = U_nu(x-nu):  cc^+ (a b)
@@ -1262,89 +1271,6 @@ __device__ __forceinline__ M3 park_load(const double2* park, int n)
 #pragma unroll
     for (int e = 0; e < 9; ++e) a.m[e] = cd{park[e * n].x, park[e * n].y};
     return a;
-}
-
-// Rectangular<2>::StapleRect (rectangular_action.hpp:186-225): for nu = mu+1, mu+2,
-// mu+3 (mod 4) the six 1x2 staples of link (x, mu) -- orthogonal to it (two), extending
-// it forward (two), backward (two) -- in the reference's grouping and order.  Every
-// rectangle is a product of five links, an SU(3) matrix, so only rows 0 and 1 are
-// carried along each chain and row 2 is added as conj(row0 x row1) (acc_su3_r01); the
-// forward pair is taken as a U^+ + b U^+ and the backward pair as U^+ a + U^+ b (the
-// reference's (a + b) U^+ and U^+ (a + b)), so every accumulated term is a unitary chain.
-__device__ __forceinline__ M3 staple_rect(const double2* __restrict__ U, const Geom& g, int s, const int c[4], int mu,
-                                          int par, double2* park = nullptr, int n = 0)
-{
-    const int q = par ^ 1;
-    M3 st = m3_zero();
-    // park (optional, see park_store): the sum waits in LDS between the terms, so that
-    // one term at a time holds registers; the same additions in the same order
-    if (park) park_store(park, n, st);
-    auto add_term = [&](const M3& r) {
-        if (park) st = park_load(park, n);
-        acc_su3_r01(st, r);
-        if (park) park_store(park, n, st);
-    };
-#pragma unroll 1
-    for (int off = 1; off < 4; ++off) {
-        const int nu = (mu + off) & 3;
-        auto at = [&](int a, int b) { return shift2(g, s, c, mu, a, nu, b); };
-        const int nup = at(0, 1), nupp = at(0, 2), mup_nup = at(1, 1), mup = at(1, 0);
-        const int nud = at(0, -1), nudd = at(0, -2), mup_nudd = at(1, -2), mup_nud = at(1, -1);
-        // orthogonal: U_nu(x) U_nu(x+nu) U_mu(x+2nu) U_nu(x+mu+nu)^+ U_nu(x+mu)^+ and its mirror
-        {
-            M3 r = mul_r01(ldu2(U, g, s, nu, par), ldu(U, g, nup, nu, q));
-            r = mul_r01(r, ldu(U, g, nupp, mu, par));
-            r = mul_nd_r01(r, ldu(U, g, mup_nup, nu, par));
-            r = mul_nd_r01(r, ldu(U, g, mup, nu, q));
-            add_term(r);
-            r = mul_dd_r01(ldu(U, g, nud, nu, q), ldu(U, g, nudd, nu, par));
-            r = mul_r01(r, ldu(U, g, nudd, mu, par));
-            r = mul_r01(r, ldu(U, g, mup_nudd, nu, q));
-            r = mul_r01(r, ldu(U, g, mup_nud, nu, par));
-            add_term(r);
-        }
-        // forward: [U_nu(x) U_mu(x+nu) U_mu(x+mu+nu) U_nu(x+2mu)^+ + mirror] U_mu(x+mu)^+
-        {
-            const int mupp = at(2, 0), mupp_nud = at(2, -1);
-            const M3 ump = ldu(U, g, mup, mu, q);
-            M3 r = mul_r01(ldu2(U, g, s, nu, par), ldu(U, g, nup, mu, q));
-            r = mul_r01(r, ldu(U, g, mup_nup, mu, par));
-            r = mul_nd_r01(r, ldu(U, g, mupp, nu, par));
-            r = mul_nd_r01(r, ump);
-            add_term(r);
-            r = mul_dn_r01(ldu(U, g, nud, nu, q), ldu(U, g, nud, mu, q));
-            r = mul_r01(r, ldu(U, g, mup_nud, mu, par));
-            r = mul_r01(r, ldu(U, g, mupp_nud, nu, q));
-            r = mul_nd_r01(r, ump);
-            add_term(r);
-        }
-        // backward: U_mu(x-mu)^+ [U_nu(x-mu) U_mu(x-mu+nu) U_mu(x+nu) U_nu(x+mu)^+ + mirror]
-        {
-            const int mud = at(-1, 0), mud_nup = at(-1, 1), mud_nud = at(-1, -1);
-            const M3 umd = ldu(U, g, mud, mu, q);
-            M3 r = mul_dn_r01(umd, ldu(U, g, mud, nu, q));
-            r = mul_r01(r, ldu(U, g, mud_nup, mu, par));
-            r = mul_r01(r, ldu(U, g, nup, mu, q));
-            r = mul_nd_r01(r, ldu(U, g, mup, nu, q));
-            add_term(r);
-            r = mul_dd_r01(umd, ldu(U, g, mud_nud, nu, par));
-            r = mul_r01(r, ldu(U, g, mud_nud, mu, par));
-            r = mul_r01(r, ldu(U, g, nud, mu, q));
-            r = mul_r01(r, ldu(U, g, mup_nud, nu, par));
-            add_term(r);
-        }
-    }
-    if (park) st = park_load(park, n);
-    return st;
-}
-
-// Rectangular<R>::Staple (rectangular_action.hpp:232-242)
-__device__ __forceinline__ M3 staple_action(const double2* __restrict__ U, const Geom& g, int s, const int c[4], int mu,
-                                            int par, double c_plaq, double c_rect, double2* park = nullptr, int n = 0)
-{
-    const M3 p = staple(U, g, s, c, mu);
-    if (c_rect == 0.0) return c_plaq == 1.0 ? p : scale(c_plaq, p);
-    return add(scale(c_plaq, p), scale(c_rect, staple_rect(U, g, s, c, mu, par, park, n)));
 }
 
 // Sum of the four clover leaves of plane (mu, nu) at site s (leaf orientation of

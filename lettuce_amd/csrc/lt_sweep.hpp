@@ -174,15 +174,11 @@ __device__ __forceinline__ void update_link(double2* __restrict__ U, const Geom&
     stu_stream(U, g, s, mu, par, L);
 }
 
-// Checkerboard4 sweeps with Rectangular<R>(beta, c_plaq, c_rect): the action enters
-// through the staple only (heatbath.hpp:110-129, overrelaxation.hpp:91-116)
+// SU(2) steps of one link with its staple at hand, reunitarisation and store
 template <bool HEATBATH>
-__device__ __forceinline__ void update_link_action(double2* __restrict__ U, const Geom& g, int s, const int c[4],
-                                                   int mu, int par, double prefactor, uint64_t seed, uint64_t counter,
-                                                   double c_plaq, double c_rect, double2* park = nullptr, int n = 0)
+__device__ __forceinline__ void update_link_with(double2* __restrict__ U, const Geom& g, int s, int mu, int par, M3 L,
+                                                 const M3& st, double prefactor, uint64_t seed, uint64_t counter)
 {
-    const M3 st = staple_action(U, g, s, c, mu, par, c_plaq, c_rect, park, n);
-    M3 L = ldu(U, g, s, mu, par);
 #pragma unroll
     for (int sub = 0; sub < 3; ++sub) {
         const int i = sub == 2 ? 1 : 0;
@@ -197,6 +193,155 @@ __device__ __forceinline__ void update_link_action(double2* __restrict__ U, cons
     }
     gram_schmidt(L);
     stu(U, g, s, mu, par, L);
+}
+
+// The part of Rectangular<R>::Staple (rectangular_action.hpp:103-242) of link (x, mu) that
+// lies on one side (UP: +nu, else -nu) of one direction nu: the plaquette term and its
+// three 1x2 rectangles.  With a, b, c the three links of the plaquette term (a b c^+ above,
+// a^+ b c below, x' = x - nu) each rectangle replaces one of them by its own three-link
+// staple:
+//   above: (c_p a b + c_r (Va b + a Vb)) c^+ + c_r a b Vc^+
+//     Va = U_mu(x-mu)^+ U_nu(x-mu) U_mu(x-mu+nu),  Vb = U_nu(x+nu) U_mu(x+2nu) U_nu(x+mu+nu)^+,
+//     Vc^+ = U_mu(x+mu+nu) U_nu(x+2mu)^+ U_mu(x+mu)^+
+//   below: (c_p a^+ b + c_r (Va^+ b + a^+ Vb)) c + c_r a^+ b Vc
+//     Va^+ = U_mu(x-mu)^+ U_nu(x'-mu)^+ U_mu(x'-mu),  Vb = U_nu(x'-nu)^+ U_mu(x'-nu) U_nu(x'+mu-nu),
+//     Vc = U_mu(x'+mu) U_nu(x'+2mu) U_mu(x+mu)^+
+// Eleven products instead of fourteen; every product but the last is a chain of links, an
+// SU(3) matrix, of which rows 0 and 1 are carried.  Each link is loaded while the product
+// before it is formed; the scheduling barriers keep the compiler from hoisting all twelve
+// link loads (which spills).
+template <bool UP, bool RECT>
+__device__ __forceinline__ M3 staple_action_side(const double2* __restrict__ U, const Geom& g, int s, const int c[4],
+                                                 int mu, int nu, int par, double c_plaq, double c_rect)
+{
+    const int q = par ^ 1;
+    constexpr int sg = UP ? 1 : -1;
+    auto at = [&](int a, int b) { return shift2(g, s, c, mu, a, nu, b); };
+    auto step = [&](int site, int dir, int parity, Raw6& into) {
+        ld_raw(U, g, site, dir, parity, into);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Raw6 l0, l1;
+    M3 ab, t, r;
+    // rows 0 and 1 of a^(+) b, and of a^(+) Vb's first product
+    {
+        Raw6 a;
+        ld_raw(U, g, UP ? s : at(0, -1), nu, UP ? par : q, a);
+        step(at(0, sg), mu, q, l0);
+        step(at(0, UP ? 1 : -2), nu, UP ? q : par, l1);
+        ab = UP ? mul_r01(rows01(a), su3_of(l0)) : mul_dn_r01(su3_of(a), su3_of(l0));
+        if (!RECT) {
+            ld_raw(U, g, at(1, UP ? 0 : -1), nu, UP ? q : par, l0);
+            t = UP ? mul_nd_r01(ab, su3_of(l0)) : mul_r01(ab, su3_of(l0));
+            third_row(t);
+            return scale(c_plaq, t);
+        }
+        step(at(0, 2 * sg), mu, par, l0);
+        t = UP ? mul_r01(rows01(a), su3_of(l1)) : mul_dd_r01(su3_of(a), su3_of(l1));
+    }
+    step(at(1, UP ? 1 : -2), nu, UP ? par : q, l1);
+    t = mul_r01(t, su3_of(l0));
+    step(at(-1, 0), mu, q, l0);
+    t = UP ? mul_nd_r01(t, su3_of(l1)) : mul_r01(t, su3_of(l1));
+    // Va^(+) b
+    step(at(-1, UP ? 0 : -1), nu, UP ? q : par, l1);
+    {
+        const M3 d = su3_of(l0);
+        step(at(-1, sg), mu, par, l0);
+        r = UP ? mul_dn_r01(d, su3_of(l1)) : mul_dd_r01(d, su3_of(l1));
+    }
+    step(at(0, sg), mu, q, l1);
+    r = mul_r01(r, su3_of(l0));
+    step(at(1, UP ? 0 : -1), nu, UP ? q : par, l0);
+    r = mul_r01(r, su3_of(l1));
+    // (c_p a^(+) b + c_r (a^(+) Vb + Va^(+) b)) c^(+)
+    M3 M = ab;
+    third_row(M);
+    third_row(t);
+    acc_su3_r01(t, r);
+#pragma unroll
+    for (int e = 0; e < 9; ++e) M.m[e] = c_plaq * M.m[e] + c_rect * t.m[e];
+    step(at(1, sg), mu, par, l1);
+    M = UP ? mul_nd(M, su3_of(l0)) : mul(M, su3_of(l0));
+    // a^(+) b Vc^(+)
+    step(at(2, UP ? 0 : -1), nu, UP ? par : q, l0);
+    r = mul_r01(ab, su3_of(l1));
+    step(at(1, 0), mu, q, l1);
+    r = UP ? mul_nd_r01(r, su3_of(l0)) : mul_r01(r, su3_of(l0));
+    __builtin_amdgcn_sched_barrier(0);
+    r = mul_nd_r01(r, su3_of(l1));
+    third_row(r);
+#pragma unroll
+    for (int e = 0; e < 9; ++e) M.m[e] += c_rect * r.m[e];
+    return M;
+}
+
+// Rectangular<R>::Staple (rectangular_action.hpp:232-242) of one link in one lane
+template <bool RECT>
+__device__ __forceinline__ M3 staple_action(const double2* __restrict__ U, const Geom& g, int s, const int c[4], int mu,
+                                            int par, double c_plaq, double c_rect)
+{
+    M3 st = m3_zero();
+#pragma unroll 1
+    for (int k = 0; k < 3; ++k) {
+        const int nu = k + (k >= mu);
+        acc(st, staple_action_side<true, RECT>(U, g, s, c, mu, nu, par, c_plaq, c_rect));
+        acc(st, staple_action_side<false, RECT>(U, g, s, c, mu, nu, par, c_plaq, c_rect));
+    }
+    return st;
+}
+
+// Checkerboard4 colour launches with Rectangular<R>(beta, c_plaq, c_rect): the action enters
+// through the staple only (heatbath.hpp:110-129, overrelaxation.hpp:91-116).  A block of six
+// wavefronts updates 64 links: wavefront w forms the part of the staple on side w & 1 of the
+// (w >> 1)-th direction nu != mu, the first one adds the parts in wavefront order through
+// LDS (lds: 27 x 64 entries) and applies the SU(2) steps.
+constexpr int ACT_WAVES = 6, ACT_LINKS = 64, ACT_BS = ACT_WAVES * ACT_LINKS;
+template <bool HEATBATH, bool RECT>
+__device__ __forceinline__ void update_links_action(double2* __restrict__ U, const Geom& g, int mu, int colour, int b,
+                                                    double prefactor, uint64_t seed, uint64_t counter, double c_plaq,
+                                                    double c_rect, int tc, double2* lds)
+{
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+    int c[4], s;
+    // tc > 1 (a timeslice is a whole number nbt of blocks): the tc timeslices of a chunk
+    // fastest, so that the t-neighbours of a block, two steps away, run in the same XCD at
+    // about the same time (24^4: 97 -> 85 us per overrelaxation launch with tc = 3)
+    if (tc > 1) {
+        const int nbt = (g.V / g.L[0]) / (4 * ACT_LINKS), per = tc * nbt;
+        const int ch = b / per, r = b - ch * per;
+        b = (ch * tc + r % tc) * nbt + r / tc;
+    }
+    const bool on = cb4_site(g, mu, colour, b * ACT_LINKS + lane, c, s);
+    M3 st = m3_zero();
+    int par = 0;
+    if (on) {
+        par = parity_of(c);
+        const int nu = (w >> 1) + ((w >> 1) >= mu);
+        st = (w & 1) ? staple_action_side<false, RECT>(U, g, s, c, mu, nu, par, c_plaq, c_rect)
+                     : staple_action_side<true, RECT>(U, g, s, c, mu, nu, par, c_plaq, c_rect);
+    }
+    auto put = [&](int slot) {
+#pragma unroll
+        for (int e = 0; e < 9; ++e) lds[(slot * 9 + e) * ACT_LINKS + lane] = make_double2(st.m[e].re, st.m[e].im);
+    };
+    auto add_from = [&](int slot) {
+#pragma unroll
+        for (int e = 0; e < 9; ++e) {
+            const double2 v = lds[(slot * 9 + e) * ACT_LINKS + lane];
+            st.m[e] += cd{v.x, v.y};
+        }
+    };
+    if (w >= 3) put(w - 3);
+    __syncthreads();
+    if (w < 3) add_from(w);
+    if (w == 1 || w == 2) put(w);
+    __syncthreads();
+    if (w || !on) return;
+    const M3 L = ldu(U, g, s, mu, par);
+    add_from(1);
+    add_from(2);
+    update_link_with<HEATBATH>(U, g, s, mu, par, L, st, prefactor, seed, counter);
 }
 
 }  // namespace lt

@@ -92,3 +92,29 @@ def test_overrelaxation_keeps_action_and_schedule_check(la, lto, gpu_ctx):
     with pytest.raises(la.LettuceError):
         la.Iterator.Checkerboard(la.OverrelaxationSubgroupKernel(f, action=act), 1)
     f.close()
+
+
+# extents: whole and partial blocks of 64 links, one and several timeslices per chunk, the
+# smallest lattice; actions with and without the rectangle
+@pytest.mark.parametrize("shape", [(4, 4, 4, 4), (4, 12, 8, 4), (16, 4, 8, 8), (8, 12, 4, 20)])
+@pytest.mark.parametrize("c_rect", [-1.0 / 12.0, 0.0])
+def test_split_staple_sweeps_match_oracle(la, lto, gpu_ctx, shape, c_rect):
+    """One overrelaxation and one heatbath sweep from identical links: per link 1e-12 and
+    1e-11, the bars of a sweep elsewhere (rounding of ~100 products, amplified by the SU(2)
+    projections of small staples)."""
+    flush(f"split staple {shape} {c_rect}")
+    cp = 1.0 - 8.0 * c_rect if c_rect else 0.7
+    U = lto.stout(lto.haar(shape, 9), shape, 0.1, 2)
+    f = make(la, gpu_ctx, shape, U)
+    act = la.RectangularAction(5.0, cp, c_rect)
+    la.Iterator.Checkerboard4(la.OverrelaxationSubgroupKernel(f, action=act), 1)
+    ref = U.copy()
+    lto.or_sweep_action(ref, shape, cp, c_rect, 1, 4)
+    assert np.max(np.abs(f.download() - ref)) <= 1e-12
+    f.upload(U)
+    f.set_rng(7, 5)
+    la.Iterator.Checkerboard4(la.HeatbathKernel(f, 5.0, action=act), 1)
+    ref = U.copy()
+    lto.hb_sweep_action(ref, shape, 5.0, cp, c_rect, 1, 4, 7, 5)
+    assert np.max(np.abs(f.download() - ref)) <= 1e-11
+    f.close()
