@@ -44,20 +44,23 @@ __global__ void LT_LINK_KERNEL hb_cb4_graph_kernel(double2* __restrict__ U, Geom
     update_link<true>(U, g, s, c, mu, parity_of(c), prefactor, seed, state[0] + (uint64_t)k);
 }
 
-// Six wavefronts per 64 links (update_links_action): three waves per SIMD, 20 spilled
-// VGPRs.  One lane per link with the sum parked in LDS ran about 9500 FP64 instructions in
-// a row at two waves per SIMD, and a 24^4 launch was 1296 waves on 1024 SIMDs: 186 us per
-// overrelaxation launch there, 322 us at 32^4; now 85 and 207 us (heatbath 195 -> 93 us at
+// Six wavefronts per 64 links (update_links_split), three waves per SIMD.  Rectangle staple:
+// one lane per link with the sum parked in LDS ran about 9500 FP64 instructions in a row at
+// two waves per SIMD, and a 24^4 launch was 1296 waves on 1024 SIMDs: 186 us per
+// overrelaxation launch there, 322 us at 32^4; now 85 and 207 us (heatbath 195 -> 94 us at
 // 24^4).  What bounds it now is the latency of the twelve link loads of a part, about half
 // of whose lines miss the L2, at one load in flight ahead of the products.
-template <bool HEATBATH, bool RECT>
-__global__ void __launch_bounds__(ACT_BS) __attribute__((amdgpu_waves_per_eu(3)))
-sweep_action_kernel(double2* __restrict__ U, Geom g, int mu, int colour, double prefactor, uint64_t seed,
-                    uint64_t counter, double c_plaq, double c_rect, int tc)
+template <bool HEATBATH, int KIND>
+__global__ void __launch_bounds__(SPLIT_BS) __attribute__((amdgpu_waves_per_eu(3)))
+split_cb4_kernel(double2* __restrict__ U, Geom g, int mu, int colour, double prefactor, uint64_t seed, uint64_t counter,
+                 const uint64_t* __restrict__ state, int k, double c_plaq, double c_rect, int tc)
 {
-    __shared__ double2 lds[27 * ACT_LINKS];
-    update_links_action<HEATBATH, RECT>(U, g, mu, colour, xcd_block_dir(blockIdx.x, gridDim.x, colour & 1), prefactor, seed,
-                                  counter, c_plaq, c_rect, tc, lds);
+    __shared__ SplitShared<HEATBATH> sh;
+    if (HEATBATH && state) counter = state[0] + (uint64_t)k;
+    int c[4], s = 0;
+    const int i = split_index((g.V / g.L[0]) >> 2, xcd_block_dir(blockIdx.x, gridDim.x, colour & 1), tc);
+    const bool on = i >= 0 && cb4_site(g, mu, colour, i, c, s);
+    update_links_split<HEATBATH, KIND>(U, g, mu, on, s, c, prefactor, seed, counter, c_plaq, c_rect, sh);
 }
 
 // PlaquetteSum block partials of a captured four-colour update (the field is in the
@@ -97,10 +100,37 @@ void k_cb_layout(lt_field u, int to_split)
     if (n) launch(u->ctx, "cb_layout", cb_layout_kernel, dim3(nblocks(n, RBS)), dim3(RBS), 0, u->d, u->g, to_split);
 }
 
+namespace {
+
+// Whether a Wilson colour launch uses the split kernel.  Rows of 32 z (or a multiple) give a
+// class whole 128-byte lines per row, and one lane per link is faster there once the launch
+// fills the GPU (32^4: overrelaxation 77 against 90 us, heatbath 90 against 102 us; 16^2 x
+// 32^2: 22.0 against 23.4 us).  Shorter rows leave half lines, which the six wavefronts of a
+// block share in the L1 (28^4: 76 -> 58 us, heatbath 89 -> 67 us), and launches below two
+// blocks per compute unit are bound by the latency of one link (8^4: 12.1 -> 8.3 us,
+// heatbath 21.7 -> 11.6 us; 16^4: 12.7 -> 9.6 and 21.3 -> 13.7 us).
+bool split_launches(const Geom& g) { return g.L[3] % 32 != 0 || g.V / 4 <= 32768; }
+
+template <bool HEATBATH, int KIND>
+void split_launch(lt_field u, const char* name, int mu, int colour, double prefactor, uint64_t counter,
+                  const uint64_t* state, int k, double c_plaq, double c_rect)
+{
+    const Geom& g = u->g;
+    launch(u->ctx, name, split_cb4_kernel<HEATBATH, KIND>, dim3((unsigned)g.L[0] * nblocks(g.V / g.L[0] / 4, SPLIT_LINKS)),
+           dim3(SPLIT_BS), 0, u->d, g, mu, colour, prefactor, u->seed, counter, state, k, c_plaq, c_rect, split_tc(g));
+}
+
+}  // namespace
+
 void k_cb4_colour(lt_field u, bool heatbath, int mu, int colour, double prefactor, uint64_t counter, const char* name)
 {
     const dim3 grid(nblocks(u->g.V / 4, BS)), block(BS);
-    if (heatbath)
+    const bool split = split_launches(u->g);
+    if (heatbath && split)
+        split_launch<true, SPLIT_WILSON>(u, name, mu, colour, prefactor, counter, nullptr, 0, 1.0, 0.0);
+    else if (split)
+        split_launch<false, SPLIT_WILSON>(u, name, mu, colour, prefactor, counter, nullptr, 0, 1.0, 0.0);
+    else if (heatbath)
         launch(u->ctx, name, sweep_cb4_kernel<true>, grid, block, 0, u->d, u->g, mu, colour, prefactor, u->seed, counter);
     else
         launch(u->ctx, name, sweep_cb4_kernel<false>, grid, block, 0, u->d, u->g, mu, colour, prefactor, u->seed,
@@ -109,24 +139,19 @@ void k_cb4_colour(lt_field u, bool heatbath, int mu, int colour, double prefacto
 
 void k_cb4_colour_graph_hb(lt_field u, int mu, int colour, double prefactor, const uint64_t* state, int k)
 {
-    launch(u->ctx, "hb_cb4", hb_cb4_graph_kernel, dim3(nblocks(u->g.V / 4, BS)), dim3(BS), 0, u->d, u->g, mu, colour,
-           prefactor, u->seed, state, k);
+    if (split_launches(u->g))
+        split_launch<true, SPLIT_WILSON>(u, "hb_cb4", mu, colour, prefactor, 0, state, k, 1.0, 0.0);
+    else
+        launch(u->ctx, "hb_cb4", hb_cb4_graph_kernel, dim3(nblocks(u->g.V / 4, BS)), dim3(BS), 0, u->d, u->g, mu, colour,
+               prefactor, u->seed, state, k);
 }
 
 void k_cb4_colour_action(lt_field u, bool heatbath, int mu, int colour, double prefactor, uint64_t counter,
                          double c_plaq, double c_rect, const char* name)
 {
-    const dim3 grid(nblocks(u->g.V / 4, ACT_LINKS)), block(ACT_BS);
-    const bool rect = c_rect != 0.0;
-    const Geom& g = u->g;
-    // the largest divisor of Nt that leaves each of the eight XCDs a chunk of timeslices of its own
-    int tc = 1;
-    if ((g.V / g.L[0]) % (4 * ACT_LINKS) == 0)
-        for (int d = 2; d <= (g.L[0] + 7) / 8; ++d)
-            if (g.L[0] % d == 0) tc = d;
-    auto* k = heatbath ? (rect ? sweep_action_kernel<true, true> : sweep_action_kernel<true, false>)
-                       : (rect ? sweep_action_kernel<false, true> : sweep_action_kernel<false, false>);
-    launch(u->ctx, name, k, grid, block, 0, u->d, u->g, mu, colour, prefactor, u->seed, counter, c_plaq, c_rect, tc);
+    auto* f = heatbath ? (c_rect != 0.0 ? split_launch<true, SPLIT_RECT> : split_launch<true, SPLIT_SCALED>)
+                       : (c_rect != 0.0 ? split_launch<false, SPLIT_RECT> : split_launch<false, SPLIT_SCALED>);
+    f(u, name, mu, colour, prefactor, counter, nullptr, 0, c_plaq, c_rect);
 }
 
 void k_cb4_plaq_partials(lt_field u, double* part)

@@ -182,6 +182,15 @@ void launch(lt_ctx ctx, const char* name, Kernel kernel, dim3 grid, dim3 block, 
 }
 
 inline unsigned nblocks(long long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
+// timeslices per chunk of a split colour launch (split_index): the largest divisor of Nt that
+// leaves each of the eight XCDs a chunk of its own
+inline int split_tc(const Geom& g)
+{
+    int tc = 1;
+    for (int d = 2; d <= (g.L[0] + 7) / 8; ++d)
+        if (g.L[0] % d == 0) tc = d;
+    return tc;
+}
 // grid size of a tiled link launch; refuses maps the kernels were not compiled for
 inline unsigned map_blocks(const LinkMap& m)
 {

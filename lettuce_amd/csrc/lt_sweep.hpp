@@ -51,11 +51,11 @@ __device__ __forceinline__ SU2 overrelax(SU2 A)
     return SU2{conj(VV.e11), -VV.e12};
 }
 
-// One Kennedy-Pendleton / Fabricius-Haan attempt k of the SU(2) sampler in the
-// reference's draw order: Philox blocks 2k (r1, r2) and 2k+1 (r3, r0) of the site;
-// coef = -0.25 prefactor / sqrt(det A).  Returns whether the attempt is accepted.
-__device__ __forceinline__ bool kp_attempt(uint64_t seed, uint32_t site, uint32_t sub, uint32_t mu, uint64_t counter,
-                                           int k, double coef, double& lambda_sq)
+// The draws of one Kennedy-Pendleton / Fabricius-Haan attempt k of the SU(2) sampler in the
+// reference's draw order: Philox blocks 2k (r1, r2) and 2k+1 (r3, r0) of the site.  They do
+// not depend on the link: y = log r1 + cos^2(2 pi r2) log r3, lambda^2 = coef * y.
+__device__ __forceinline__ void kp_draw(uint64_t seed, uint32_t site, uint32_t sub, uint32_t mu, uint64_t counter, int k,
+                                        double& y, double& r0)
 {
     double ua0, ua1, ub0, ub1;
     draw2(seed, site, RNG_HEATBATH, (uint32_t)(2 * k), sub, mu, counter, ua0, ua1);
@@ -63,26 +63,48 @@ __device__ __forceinline__ bool kp_attempt(uint64_t seed, uint32_t site, uint32_
     const double x1 = log(1.0 - ua0);
     const double x2 = cos(2.0 * 3.14159265358979323846 * (1.0 - ua1));
     const double x3 = log(1.0 - ub0);
-    lambda_sq = coef * (x1 + x2 * x2 * x3);
-    const double r0 = ub1;
+    y = x1 + x2 * x2 * x3;
+    r0 = ub1;
+}
+__device__ __forceinline__ bool kp_accept(double y, double r0, double coef, double& lambda_sq)
+{
+    lambda_sq = coef * y;
     return !(r0 * r0 + lambda_sq >= 1.0);
 }
+// One attempt; coef = -0.25 prefactor / sqrt(det A).  Returns whether it is accepted.
+__device__ __forceinline__ bool kp_attempt(uint64_t seed, uint32_t site, uint32_t sub, uint32_t mu, uint64_t counter,
+                                           int k, double coef, double& lambda_sq)
+{
+    double y, r0;
+    kp_draw(seed, site, sub, mu, counter, k, y, r0);
+    return kp_accept(y, r0, coef, lambda_sq);
+}
 
-// The accepted SU(2) draw X (direction from Philox block 0xFFFFF) times V^+, V = A / sqrt(det A)
-__device__ __forceinline__ SU2 kp_finish(SU2 V, double lambda_sq, uint64_t seed, uint32_t site, uint32_t sub,
-                                         uint32_t mu, uint64_t counter)
+// The direction of the accepted draw (Philox block 0xFFFFF): cos(theta), cos(phi), sin(phi)
+__device__ __forceinline__ void kp_direction(uint64_t seed, uint32_t site, uint32_t sub, uint32_t mu, uint64_t counter,
+                                             double& cos_theta, double& cp, double& sp)
+{
+    double phi, ct;
+    draw2(seed, site, RNG_HEATBATH, 0xFFFFFu, sub, mu, counter, phi, ct);
+    cos_theta = 1.0 - 2.0 * ct;
+    sincos(2.0 * 3.14159265358979323846 * phi, &sp, &cp);
+}
+// The accepted SU(2) draw X times V^+, V = A / sqrt(det A)
+__device__ __forceinline__ SU2 kp_element(SU2 V, double lambda_sq, double cos_theta, double cp, double sp)
 {
     double x0 = 1.0 - 2.0 * lambda_sq;
     double abs_x = sqrt(1.0 - x0 * x0);
-    double phi, ct;
-    draw2(seed, site, RNG_HEATBATH, 0xFFFFFu, sub, mu, counter, phi, ct);
-    double cos_theta = 1.0 - 2.0 * ct;
     double vec_norm = abs_x * sqrt(1.0 - cos_theta * cos_theta);
-    double sp, cp;
-    sincos(2.0 * 3.14159265358979323846 * phi, &sp, &cp);
     SU2 X{cd{x0, vec_norm * cp}, cd{vec_norm * sp, abs_x * cos_theta}};
     SU2 Vd{conj(V.e11), -V.e12};
     return su2_mul(X, Vd);
+}
+__device__ __forceinline__ SU2 kp_finish(SU2 V, double lambda_sq, uint64_t seed, uint32_t site, uint32_t sub,
+                                         uint32_t mu, uint64_t counter)
+{
+    double ct, cp, sp;
+    kp_direction(seed, site, sub, mu, counter, ct, cp, sp);
+    return kp_element(V, lambda_sq, ct, cp, sp);
 }
 
 // Kennedy-Pendleton / Fabricius-Haan SU(2) sampler in the reference's draw order: the
@@ -172,27 +194,6 @@ __device__ __forceinline__ void update_link(double2* __restrict__ U, const Geom&
     // the updated link is not read again in this launch: a streaming store keeps the
     // L2 for the neighbour links (-0.3 % overrelaxation, -0.8 % heatbath launch at 32^4)
     stu_stream(U, g, s, mu, par, L);
-}
-
-// SU(2) steps of one link with its staple at hand, reunitarisation and store
-template <bool HEATBATH>
-__device__ __forceinline__ void update_link_with(double2* __restrict__ U, const Geom& g, int s, int mu, int par, M3 L,
-                                                 const M3& st, double prefactor, uint64_t seed, uint64_t counter)
-{
-#pragma unroll
-    for (int sub = 0; sub < 3; ++sub) {
-        const int i = sub == 2 ? 1 : 0;
-        const int j = sub == 0 ? 1 : 2;
-        SU2 A = extract(L, st, i, j);
-        SU2 X;
-        if (HEATBATH)
-            X = heatbath_su2(A, prefactor, seed, (uint32_t)s, (uint32_t)sub, (uint32_t)mu, counter);
-        else
-            X = overrelax(A);
-        embed_mul(L, X, i, j);
-    }
-    gram_schmidt(L);
-    stu(U, g, s, mu, par, L);
 }
 
 // The part of Rectangular<R>::Staple (rectangular_action.hpp:103-242) of link (x, mu) that
@@ -291,44 +292,87 @@ __device__ __forceinline__ M3 staple_action(const double2* __restrict__ U, const
     return st;
 }
 
-// Checkerboard4 colour launches with Rectangular<R>(beta, c_plaq, c_rect): the action enters
-// through the staple only (heatbath.hpp:110-129, overrelaxation.hpp:91-116).  A block of six
-// wavefronts updates 64 links: wavefront w forms the part of the staple on side w & 1 of the
-// (w >> 1)-th direction nu != mu, the first one adds the parts in wavefront order through
-// LDS (lds: 27 x 64 entries) and applies the SU(2) steps.
-constexpr int ACT_WAVES = 6, ACT_LINKS = 64, ACT_BS = ACT_WAVES * ACT_LINKS;
-template <bool HEATBATH, bool RECT>
-__device__ __forceinline__ void update_links_action(double2* __restrict__ U, const Geom& g, int mu, int colour, int b,
-                                                    double prefactor, uint64_t seed, uint64_t counter, double c_plaq,
-                                                    double c_rect, int tc, double2* lds)
+// A colour launch with the staple split over wavefronts.  A block of six wavefronts updates
+// 64 links: wavefront w forms the part of the staple on side w & 1 of the (w >> 1)-th
+// direction nu != mu; the parts are added through LDS and the first wavefront applies the
+// SU(2) steps.  The heatbath's random numbers do not depend on the link: wavefront w also
+// draws attempt w / 3 of subgroup w % 3, the first three the directions, while the links of
+// their parts are on the way; only the rare third attempts are drawn in the SU(2) steps.
+// The action enters through the staple only (heatbath.hpp:110-129, overrelaxation.hpp:91-116):
+// SPLIT_WILSON, SPLIT_SCALED (c_plaq times the plaquette staple), SPLIT_RECT.
+enum SplitKind { SPLIT_WILSON = 0, SPLIT_SCALED = 1, SPLIT_RECT = 2 };
+constexpr int SPLIT_WAVES = 6, SPLIT_LINKS = 64, SPLIT_BS = SPLIT_WAVES * SPLIT_LINKS;
+template <bool HEATBATH>
+struct SplitShared {
+    double2 part[27 * SPLIT_LINKS];
+    double draw[HEATBATH ? 21 * SPLIT_LINKS : 1];   // y, r0 of (subgroup, attempt); cos, cos, sin of the directions
+};
+
+// one side of the Wilson staple for one direction, rows 0 and 1 and the third from them
+template <bool UP, typename Between>
+__device__ __forceinline__ M3 staple_wilson_side(const double2* __restrict__ U, const Geom& g, int s, const int c[4],
+                                                 int mu, int nu, int par, Between between)
+{
+    const int q = par ^ 1;
+    const int x1 = UP ? s : shift2(g, s, c, mu, 0, nu, -1);
+    Raw6 a, b, e;
+    ld_raw(U, g, x1, nu, UP ? par : q, a);
+    ld_raw(U, g, UP ? shift2(g, s, c, mu, 0, nu, 1) : x1, mu, q, b);
+    ld_raw(U, g, shift2(g, s, c, mu, 1, nu, UP ? 0 : -1), nu, UP ? q : par, e);
+    __builtin_amdgcn_sched_barrier(0);
+    between();
+    __builtin_amdgcn_sched_barrier(0);
+    M3 t = UP ? mul_nd_r01(mul_r01(rows01(a), su3_of(b)), su3_of(e)) : mul_r01(mul_dn_r01(su3_of(a), su3_of(b)), su3_of(e));
+    third_row(t);
+    return t;
+}
+
+// on: whether this lane holds a link (s, mu) of the launch
+template <bool HEATBATH, int KIND>
+__device__ __forceinline__ void update_links_split(double2* __restrict__ U, const Geom& g, int mu, bool on, int s,
+                                                   const int c[4], double prefactor, uint64_t seed, uint64_t counter,
+                                                   double c_plaq, double c_rect, SplitShared<HEATBATH>& sh)
 {
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
-    int c[4], s;
-    // tc > 1 (a timeslice is a whole number nbt of blocks): the tc timeslices of a chunk
-    // fastest, so that the t-neighbours of a block, two steps away, run in the same XCD at
-    // about the same time (24^4: 97 -> 85 us per overrelaxation launch with tc = 3)
-    if (tc > 1) {
-        const int nbt = (g.V / g.L[0]) / (4 * ACT_LINKS), per = tc * nbt;
-        const int ch = b / per, r = b - ch * per;
-        b = (ch * tc + r % tc) * nbt + r / tc;
-    }
-    const bool on = cb4_site(g, mu, colour, b * ACT_LINKS + lane, c, s);
     M3 st = m3_zero();
     int par = 0;
+    auto draws = [&]() {
+        if (HEATBATH) {
+            const uint32_t sub = (uint32_t)(w % 3);
+            double y, r0;
+            kp_draw(seed, (uint32_t)s, sub, (uint32_t)mu, counter, w / 3, y, r0);
+            sh.draw[(2 * w) * SPLIT_LINKS + lane] = y;
+            sh.draw[(2 * w + 1) * SPLIT_LINKS + lane] = r0;
+            if (w < 3) {
+                double ct, cp, sp;
+                kp_direction(seed, (uint32_t)s, sub, (uint32_t)mu, counter, ct, cp, sp);
+                sh.draw[(12 + 3 * w) * SPLIT_LINKS + lane] = ct;
+                sh.draw[(13 + 3 * w) * SPLIT_LINKS + lane] = cp;
+                sh.draw[(14 + 3 * w) * SPLIT_LINKS + lane] = sp;
+            }
+        }
+    };
     if (on) {
         par = parity_of(c);
         const int nu = (w >> 1) + ((w >> 1) >= mu);
-        st = (w & 1) ? staple_action_side<false, RECT>(U, g, s, c, mu, nu, par, c_plaq, c_rect)
-                     : staple_action_side<true, RECT>(U, g, s, c, mu, nu, par, c_plaq, c_rect);
+        if (KIND == SPLIT_RECT) {
+            draws();
+            st = (w & 1) ? staple_action_side<false, true>(U, g, s, c, mu, nu, par, c_plaq, c_rect)
+                         : staple_action_side<true, true>(U, g, s, c, mu, nu, par, c_plaq, c_rect);
+        } else {
+            st = (w & 1) ? staple_wilson_side<false>(U, g, s, c, mu, nu, par, draws)
+                         : staple_wilson_side<true>(U, g, s, c, mu, nu, par, draws);
+            if (KIND == SPLIT_SCALED) st = scale(c_plaq, st);
+        }
     }
     auto put = [&](int slot) {
 #pragma unroll
-        for (int e = 0; e < 9; ++e) lds[(slot * 9 + e) * ACT_LINKS + lane] = make_double2(st.m[e].re, st.m[e].im);
+        for (int e = 0; e < 9; ++e) sh.part[(slot * 9 + e) * SPLIT_LINKS + lane] = make_double2(st.m[e].re, st.m[e].im);
     };
     auto add_from = [&](int slot) {
 #pragma unroll
         for (int e = 0; e < 9; ++e) {
-            const double2 v = lds[(slot * 9 + e) * ACT_LINKS + lane];
+            const double2 v = sh.part[(slot * 9 + e) * SPLIT_LINKS + lane];
             st.m[e] += cd{v.x, v.y};
         }
     };
@@ -338,10 +382,49 @@ __device__ __forceinline__ void update_links_action(double2* __restrict__ U, con
     if (w == 1 || w == 2) put(w);
     __syncthreads();
     if (w || !on) return;
-    const M3 L = ldu(U, g, s, mu, par);
+    M3 L = ldu(U, g, s, mu, par);
     add_from(1);
     add_from(2);
-    update_link_with<HEATBATH>(U, g, s, mu, par, L, st, prefactor, seed, counter);
+#pragma unroll
+    for (int sub = 0; sub < 3; ++sub) {
+        const int i = sub == 2 ? 1 : 0;
+        const int j = sub == 0 ? 1 : 2;
+        const SU2 A = extract(L, st, i, j);
+        SU2 X;
+        if (HEATBATH) {
+            const double an = 1.0 / sqrt(su2_det(A));
+            const SU2 V{an * A.e11, an * A.e12};
+            const double coef = -0.25 * prefactor * an;
+            const double* d = sh.draw + lane;
+            double lambda_sq;
+            bool found = kp_accept(d[2 * sub * SPLIT_LINKS], d[(2 * sub + 1) * SPLIT_LINKS], coef, lambda_sq);
+            if (!found) found = kp_accept(d[(6 + 2 * sub) * SPLIT_LINKS], d[(7 + 2 * sub) * SPLIT_LINKS], coef, lambda_sq);
+            for (int k = 2; !found && k <= KP_MAX_ITER; ++k)
+                found = kp_attempt(seed, (uint32_t)s, (uint32_t)sub, (uint32_t)mu, counter, k, coef, lambda_sq);
+            X = found ? kp_element(V, lambda_sq, d[(12 + 3 * sub) * SPLIT_LINKS], d[(13 + 3 * sub) * SPLIT_LINKS],
+                                   d[(14 + 3 * sub) * SPLIT_LINKS])
+                      : SU2{cd{1.0, 0.0}, cd{0.0, 0.0}};
+        } else {
+            X = overrelax(A);
+        }
+        embed_mul(L, X, i, j);
+    }
+    gram_schmidt(L);
+    stu(U, g, s, mu, par, L);
+}
+
+// Index (in the class's order, t slowest) of the link of this lane in block b of a split
+// launch with nt links per timeslice; -1 for none.  Every timeslice is covered by its own
+// blocks of 64 links (the last one partly); the tc timeslices of a chunk are walked fastest,
+// so that the t-neighbours of a block run in the same XCD at about the same time (24^4,
+// Luescher-Weisz staple: 97 -> 85 us per overrelaxation launch with tc = 3; 20^4, four
+// colours, Wilson staple: 25 -> 20 us with tc = 2).
+__device__ __forceinline__ int split_index(int nt, int b, int tc)
+{
+    const int nbt = (nt + SPLIT_LINKS - 1) / SPLIT_LINKS, per = tc * nbt;
+    const int ch = b / per, q = b - ch * per;
+    const int r = (q / tc) * SPLIT_LINKS + (threadIdx.x & (SPLIT_LINKS - 1));
+    return r < nt ? (ch * tc + q % tc) * nt + r : -1;
 }
 
 }  // namespace lt

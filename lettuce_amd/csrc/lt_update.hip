@@ -48,111 +48,29 @@ hb_cb2_graph_kernel(double2* __restrict__ U, Geom g, LinkMap m, int mu, int par,
 }
 
 // ---- small lattices ---------------------------------------------------------------
-// A colour launch of a few thousand links leaves most of the GPU idle, and its duration
-// is one wavefront's serial work: about 2400 VALU instructions for an overrelaxation
-// link, twice that with the heatbath sampler (8^4: 7.8 and 17.8 us per launch).  Up to
-// SMALL_VH links per colour launch, four lanes share a link: lane j < 3 builds the upper
-// and the lower staple term of the j-th direction nu != mu, a two-step sum inside the
-// quad (DPP quad permutations; every lane ends with the same ((t0 + t1) + (t2 + 0)),
-// since a + b = b + a) gives all four lanes the staple, all four apply the SU(2) steps
-// -- the heatbath's attempts base + j run side by side and the first accepted one is
-// taken, exactly the attempt the sequential loop would take -- and lane 0 stores.
+// A colour launch of a few thousand links leaves most of the GPU idle, and its duration is
+// the serial work of one link.  Up to SMALL_VH links per colour launch the staple of a link
+// is split over six wavefronts (update_links_split): 8^4 overrelaxation 8.0 us a launch and
+// heatbath 11.9 us between two events, of which about 6 us are the launch itself (four lanes
+// per link: 8.9 and 13.4 us; one lane: 10 and 20 us).  From 16^4 on (32768 links) the launch
+// fills the GPU and one lane per link is as fast or faster (16^4: 11.5 against 12.8 us; 32^4:
+// 96 against 124 us).
 #ifndef LT_SMALL_VH
 #define LT_SMALL_VH 16384
 #endif
 constexpr int SMALL_VH = LT_SMALL_VH;
-constexpr int SBS = 256;
 
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
-    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
-}
-// a <- a + a of lane (lane ^ 1) (CTRL 0xB1) or (lane ^ 2) (CTRL 0x4E)
-template <int CTRL>
-__device__ __forceinline__ void quad_add(M3& a)
-{
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-        a.m[k].re += dpp_f64<CTRL>(a.m[k].re);
-        a.m[k].im += dpp_f64<CTRL>(a.m[k].im);
-    }
-}
-
-// upper + lower staple term of direction nu for link (s, mu)
-__device__ __forceinline__ M3 staple_pair(const double2* __restrict__ U, const Geom& g, int s, const int c[4], int mu,
-                                          int par, int nu)
-{
-    const int q = par ^ 1;
-    const int cnu = pick4(c, nu), Ln = pick4(g.L, nu), stn = pick4(g.st, nu);
-    const int s_nu = (cnu + 1 < Ln) ? s + stn : s - (Ln - 1) * stn;
-    const int s_nd = (cnu > 0) ? s - stn : s + (Ln - 1) * stn;
-    const int cmu = pick4(c, mu), Lm = pick4(g.L, mu), stm = pick4(g.st, mu);
-    const int dmu = (cmu + 1 < Lm) ? stm : -(Lm - 1) * stm;   // site step +mu
-    const int s_mu = s + dmu, s_nd_mu = s_nd + dmu;
-    M3 t = mul_nd_r01(mul_r01(ldu2(U, g, s, nu, par), ldu(U, g, s_nu, mu, q)), ldu(U, g, s_mu, nu, q));
-    third_row(t);
-    M3 ef = mul_r01(ldu2(U, g, s_nd, mu, q), ldu(U, g, s_nd_mu, nu, par));
-    third_row(ef);
-    mul_dn_acc(t, ldu(U, g, s_nd, nu, q), ef);
-    return t;
-}
-
-// One colour launch (mu, parity) of a small lattice, four lanes per link; the heatbath
-// draws with counter state[0] + k when state is given (captured updates), else counter.
 template <bool HEATBATH>
-__global__ void __launch_bounds__(SBS) sweep_small_kernel(double2* __restrict__ U, Geom g, int mu, int par,
-                                                          double prefactor, uint64_t seed, uint64_t counter,
-                                                          const uint64_t* __restrict__ state, int k)
+__global__ void __launch_bounds__(SPLIT_BS) __attribute__((amdgpu_waves_per_eu(3)))
+split_cb2_kernel(double2* __restrict__ U, Geom g, int mu, int par, double prefactor, uint64_t seed, uint64_t counter,
+                 const uint64_t* __restrict__ state, int k, int tc)
 {
-    const int tid = blockIdx.x * SBS + threadIdx.x;
-    const int l = tid >> 2, j = tid & 3;
-    if (l >= g.Vh) return;   // whole quads (4 Vh threads)
+    __shared__ SplitShared<HEATBATH> sh;
     if (HEATBATH && state) counter = state[0] + (uint64_t)k;
-    int c[4];
-    const int s = site_of_cb(g, l, par, c);
-    M3 st = j < 3 ? staple_pair(U, g, s, c, mu, par, j + (j >= mu)) : m3_zero();
-    quad_add<0xB1>(st);
-    quad_add<0x4E>(st);
-    M3 L = ldu(U, g, s, mu, par);
-    const int lane = __lane_id();
-#pragma unroll
-    for (int sub = 0; sub < 3; ++sub) {
-        const int i = sub == 2 ? 1 : 0;
-        const int jj = sub == 0 ? 1 : 2;
-        const SU2 A = extract(L, st, i, jj);
-        SU2 X;
-        if (HEATBATH) {
-            const double an = 1.0 / sqrt(su2_det(A));
-            const SU2 V{an * A.e11, an * A.e12};
-            const double coef = -0.25 * prefactor * an;
-            double lambda_sq = 0.0;
-            bool found = false;
-            for (int base = 0; base <= KP_MAX_ITER; base += 4) {
-                double lsq = 0.0;
-                const int kk = base + j;
-                const bool acc = kk <= KP_MAX_ITER &&
-                                 kp_attempt(seed, (uint32_t)s, (uint32_t)sub, (uint32_t)mu, counter, kk, coef, lsq);
-                const int qbits = (int)((__ballot(acc) >> (lane & ~3)) & 0xFull);
-                const double first = __shfl(lsq, qbits ? (lane & ~3) + __ffs(qbits) - 1 : lane);
-                if (qbits) {
-                    lambda_sq = first;
-                    found = true;
-                    break;
-                }
-            }
-            X = found ? kp_finish(V, lambda_sq, seed, (uint32_t)s, (uint32_t)sub, (uint32_t)mu, counter)
-                      : SU2{cd{1.0, 0.0}, cd{0.0, 0.0}};
-        } else {
-            X = overrelax(A);
-        }
-        embed_mul(L, X, i, jj);
-    }
-    gram_schmidt(L);
-    if (j == 0) stu(U, g, s, mu, par, L);
+    int c[4] = {0, 0, 0, 0}, s = 0;
+    const int i = split_index((g.V / g.L[0]) >> 1, xcd_block_dir(blockIdx.x, gridDim.x, par), tc);
+    if (i >= 0) s = site_of_cb(g, i, par, c);
+    update_links_split<HEATBATH, SPLIT_WILSON>(U, g, mu, i >= 0, s, c, prefactor, seed, counter, 1.0, 0.0, sh);
 }
 
 // PlaquetteSum of the captured update: per-block sums (the block tree of the HMC
@@ -233,6 +151,15 @@ LinkMap sweep_map(const LinkMap& m)
     return r;
 }
 
+template <bool HEATBATH>
+void split_cb2(lt_field u, const char* name, int mu, int par, double prefactor, uint64_t counter, const uint64_t* state,
+               int k)
+{
+    const Geom& g = u->g;
+    launch(u->ctx, name, split_cb2_kernel<HEATBATH>, dim3((unsigned)g.L[0] * nblocks(g.Vh / g.L[0], SPLIT_LINKS)),
+           dim3(SPLIT_BS), 0, u->d, g, mu, par, prefactor, u->seed, counter, state, k, split_tc(g));
+}
+
 // n sweeps; the four-colour ones (split) expect the field in the split order
 template <bool HEATBATH>
 void sweep_launches(lt_field u, int n, int schedule, double prefactor, const char* name)
@@ -246,8 +173,7 @@ void sweep_launches(lt_field u, int n, int schedule, double prefactor, const cha
                 for (int col = 0; col < 4; ++col) k_cb4_colour(u, HEATBATH, mu, col, prefactor, counter, name);
             } else if (g.Vh <= SMALL_VH) {
                 for (int par = 0; par < 2; ++par)
-                    launch(ctx, name, sweep_small_kernel<HEATBATH>, dim3(nblocks(4LL * g.Vh, SBS)), dim3(SBS), 0, u->d, g,
-                           mu, par, prefactor, u->seed, counter, (const uint64_t*)nullptr, 0);
+                    split_cb2<HEATBATH>(u, name, mu, par, prefactor, counter, nullptr, 0);
             } else {
                 const LinkMap m = sweep_map(u->map);
                 for (int par = 0; par < 2; ++par)
@@ -362,9 +288,7 @@ void enqueue_update(lt_field u, UpdateGraph& G, double prefactor)
             if (G.schedule == LT_CB4) {
                 for (int col = 0; col < 4; ++col) k_cb4_colour_graph_hb(u, mu, col, prefactor, G.state, k);
             } else if (g.Vh <= SMALL_VH) {
-                for (int par = 0; par < 2; ++par)
-                    launch(ctx, "hb_cb2", sweep_small_kernel<true>, dim3(nblocks(4LL * g.Vh, SBS)), dim3(SBS), 0, u->d, g,
-                           mu, par, prefactor, u->seed, (uint64_t)0, (const uint64_t*)G.state, k);
+                for (int par = 0; par < 2; ++par) split_cb2<true>(u, "hb_cb2", mu, par, prefactor, 0, G.state, k);
             } else {
                 for (int par = 0; par < 2; ++par)
                     launch(ctx, "hb_cb2", hb_cb2_graph_kernel, dim3(map_blocks(m)), dim3(m.nthreads), 0, u->d, g, m,

@@ -329,3 +329,38 @@ def test_update_sweeps_graph_equals_eager(la, gpu_ctx, schedule, shape):
     assert np.array_equal(a.download(), c.download())
     for f in (a, b, c):
         f.close()
+
+
+def one_rounding(U):
+    """U with every entry moved by one rounding, either way."""
+    return U * (1.0 + np.where(np.random.default_rng(3).random(U.shape) < 0.5, -1.0, 1.0) * 2.0 ** -52)
+
+
+# split colour launches: whole and partial blocks of 64 links, one and several timeslices per
+# chunk, both sides of the switch to one lane per link (32768 links of rows of 32, 16384 links
+# with two colours); beta = 0.7 rejects most draws, so third and later attempts occur
+@pytest.mark.parametrize("schedule,shape", [(2, (2, 2, 2, 2)), (2, (6, 10, 4, 14)), (2, (16, 4, 8, 4)), (2, (8, 16, 16, 18)),
+                                            (4, (4, 4, 4, 4)), (4, (16, 12, 4, 20)), (4, (4, 4, 8, 32)),
+                                            (4, (20, 16, 16, 32))])
+def test_split_launches_match_oracle(la, lto, gpu_ctx, schedule, shape):
+    """One overrelaxation and one heatbath sweep from identical links against the oracle.  The
+    SU(2) projections of small staples amplify rounding by a factor that the links decide, so
+    the bar is what the oracle itself moves by when its links move by one rounding, times the
+    40 roundings of a staple and its projections."""
+    flush(f"split {schedule} {shape}")
+    U = lto.stout(lto.haar(shape, 6), shape, 0.1, 1)
+    f = field(la, gpu_ctx, shape, U)
+    it = la.Iterator.Checkerboard if schedule == 2 else la.Iterator.Checkerboard4
+    sweeps = [(lambda: it(la.OverrelaxationSubgroupKernel(f), 1), lambda W: lto.or_sweep(W, shape, 1, schedule))]
+    for beta in (6.0, 0.7):
+        sweeps.append((lambda beta=beta: it(la.HeatbathKernel(f, beta), 1),
+                       lambda W, beta=beta: lto.hb_sweep(W, shape, beta, 1, schedule, 13, 1 << 33)))
+    for gpu, cpu in sweeps:
+        f.upload(U)
+        f.set_rng(13, 1 << 33)
+        gpu()
+        ref, near = U.copy(), one_rounding(U)
+        cpu(ref)
+        cpu(near)
+        assert np.max(np.abs(f.download() - ref)) <= 1e-13 + 40.0 * np.max(np.abs(near - ref))
+    f.close()
