@@ -187,6 +187,53 @@ double* lt_ctx_s::host_for(size_t n)
     return host;
 }
 
+double2* lt_ctx_s::links_for(size_t n)
+{
+    if (n > links_n) {
+        if (links) {
+            LT_HIP_CHECK(hipStreamSynchronize(stream));
+            LT_HIP_CHECK(hipFree(links));
+        }
+        links = nullptr;
+        links_n = 0;
+        if (hipMalloc(&links, n * sizeof(double2)) != hipSuccess) {
+            (void)hipGetLastError();
+            links = nullptr;
+            throw lt::LtError{LT_ENOMEM, "link buffer allocation failed"};
+        }
+        links_n = n;
+    }
+    return links;
+}
+
+void lt_ctx_s::links_release()
+{
+    std::lock_guard<std::mutex> lock(links_mutex);
+    if (!links) return;
+    (void)hipStreamSynchronize(stream);
+    (void)hipFree(links);
+    links = nullptr;
+    links_n = 0;
+}
+
+void* lt_ctx_s::device_alloc(size_t bytes)
+{
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    links_release();
+    p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
+void lt_ctx_s::handle_gone()
+{
+    live -= 1;
+    if (live == 0) links_release();
+}
+
 void lt_ctx_s::collect_profile()
 {
     if (pending.empty()) return;
@@ -216,11 +263,10 @@ bool same_shape(lt_field a, lt_field b)
     return true;
 }
 
-double2* alloc_links(const lt::Geom& g)
+double2* alloc_links(lt_ctx ctx, const lt::Geom& g)
 {
-    double2* p = nullptr;
-    if (hipMalloc(&p, (size_t)72 * g.Vh * sizeof(double2)) != hipSuccess)
-        throw lt::LtError{LT_ENOMEM, "link buffer allocation failed"};
+    auto* p = (double2*)ctx->device_alloc((size_t)72 * g.Vh * sizeof(double2));
+    if (!p) throw lt::LtError{LT_ENOMEM, "link buffer allocation failed"};
     return p;
 }
 
@@ -273,6 +319,7 @@ int lt_ctx_destroy(lt_ctx ctx)
             (void)hipEventDestroy(p.second);
         }
         if (ctx->scratch) (void)hipFree(ctx->scratch);
+        ctx->links_release();
         if (ctx->host) (void)hipHostFree(ctx->host);
         (void)hipStreamDestroy(ctx->stream);
         delete ctx;
@@ -394,7 +441,7 @@ int lt_field_create(lt_ctx ctx, int nt, int nx, int ny, int nz, lt_field* out)
         f->g = lt::make_geom(nt, nx, ny, nz);
         f->map = lt::default_linkmap(f->g);
         try {
-            f->d = alloc_links(f->g);
+            f->d = alloc_links(ctx, f->g);
         } catch (...) {
             delete f;
             throw;
@@ -414,7 +461,7 @@ int lt_field_destroy(lt_field f)
         LT_HIP_CHECK(hipStreamSynchronize(f->ctx->stream));
         lt::drop_update_graph(f);
         if (f->d) LT_HIP_CHECK(hipFree(f->d));
-        f->ctx->live -= 1;
+        f->ctx->handle_gone();
         delete f;
         return LT_OK;
     });
@@ -433,8 +480,8 @@ int lt_field_upload(lt_field f, const double* aos)
     return guarded([&] {
         use_device(f->ctx);
         size_t bytes = (size_t)4 * f->g.V * 18 * sizeof(double);
-        double* stage = nullptr;
-        if (hipMalloc(&stage, bytes) != hipSuccess) throw lt::LtError{LT_ENOMEM, "upload staging allocation failed"};
+        auto* stage = (double*)f->ctx->device_alloc(bytes);
+        if (!stage) throw lt::LtError{LT_ENOMEM, "upload staging allocation failed"};
         hipError_t e = hipMemcpyAsync(stage, aos, bytes, hipMemcpyHostToDevice, f->ctx->stream);
         if (e == hipSuccess) {
             try {
@@ -458,8 +505,8 @@ int lt_field_download(lt_field f, double* aos)
     return guarded([&] {
         use_device(f->ctx);
         size_t bytes = (size_t)4 * f->g.V * 18 * sizeof(double);
-        double* stage = nullptr;
-        if (hipMalloc(&stage, bytes) != hipSuccess) throw lt::LtError{LT_ENOMEM, "download staging allocation failed"};
+        auto* stage = (double*)f->ctx->device_alloc(bytes);
+        if (!stage) throw lt::LtError{LT_ENOMEM, "download staging allocation failed"};
         hipError_t e = hipSuccess;
         try {
             lt::k_unpack(f, stage);
@@ -859,21 +906,18 @@ int lt_stout(lt_field in, lt_field out, double rho, int n_levels)
             if (in != out) lt::k_copy(ctx, in->d, out->d, (size_t)72 * in->g.Vh);
             return LT_OK;
         }
-        // ping-pong so that the last level lands in out->d
-        double2* tmp = alloc_links(in->g);
+        // ping-pong so that the last level lands in out->d; a single level into another
+        // field needs no second buffer
+        std::lock_guard<std::mutex> lock(ctx->links_mutex);
+        double2* tmp = n_levels > 1 || in == out ? ctx->links_for((size_t)72 * in->g.Vh) : nullptr;
         const double2* src = in->d;
         for (int k = 0; k < n_levels; ++k) {
-            const bool last = k == n_levels - 1;
-            double2* dst;
-            if (last) dst = (src == out->d) ? tmp : out->d;
-            else dst = (src == tmp) ? out->d : tmp;
-            if (dst == src) dst = (dst == tmp) ? out->d : tmp;
+            double2* dst = (n_levels - 1 - k) % 2 == 0 ? out->d : tmp;
+            if (dst == src) dst = dst == tmp ? out->d : tmp;
             lt::k_stout(ctx, in->g, in->map, src, dst, rho);
             src = dst;
         }
         if (src != out->d) lt::k_copy(ctx, src, out->d, (size_t)72 * in->g.Vh);
-        LT_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-        LT_HIP_CHECK(hipFree(tmp));
         return LT_OK;
     });
 }
@@ -893,11 +937,9 @@ int lt_flow_create(lt_field unflowed, lt_field flowed, int integrator, double ep
         fl->eps = eps;
         try {
             // Z is an su(3) field: 8 reals per link (4 complex doubles)
-            if (hipMalloc(&fl->z, (size_t)32 * flowed->g.Vh * sizeof(double2)) != hipSuccess) {
-                fl->z = nullptr;
-                throw lt::LtError{LT_ENOMEM, "flow Z allocation failed"};
-            }
-            fl->tmp = alloc_links(flowed->g);
+            fl->z = (double2*)flowed->ctx->device_alloc((size_t)32 * flowed->g.Vh * sizeof(double2));
+            if (!fl->z) throw lt::LtError{LT_ENOMEM, "flow Z allocation failed"};
+            fl->tmp = alloc_links(flowed->ctx, flowed->g);
         } catch (...) {
             if (fl->z) (void)hipFree(fl->z);
             delete fl;
@@ -917,7 +959,7 @@ int lt_flow_destroy(lt_flow fl)
         LT_HIP_CHECK(hipStreamSynchronize(fl->flowed->ctx->stream));
         (void)hipFree(fl->z);
         (void)hipFree(fl->tmp);
-        fl->flowed->ctx->live -= 1;
+        fl->flowed->ctx->handle_gone();
         delete fl;
         return LT_OK;
     });

@@ -35,11 +35,11 @@ struct StepKey {
 };
 
 template <typename T>
-T* dev_alloc(size_t n)
+T* dev_alloc(lt_ctx ctx, size_t n)
 {
-    T* p = nullptr;
     if (n == 0) n = 1;
-    if (hipMalloc(&p, n * sizeof(T)) != hipSuccess) throw lt::LtError{LT_ENOMEM, "batch device allocation failed"};
+    auto* p = (T*)ctx->device_alloc(n * sizeof(T));
+    if (!p) throw lt::LtError{LT_ENOMEM, "batch device allocation failed"};
     return p;
 }
 
@@ -131,7 +131,7 @@ void ensure_samples(lt_batch b, int n_sub)
     b->drop_graph();
     if (b->st.samples) LT_HIP_CHECK(hipFree(b->st.samples));
     b->st.samples = nullptr;
-    b->st.samples = dev_alloc<double>((size_t)b->n * n_sub);
+    b->st.samples = dev_alloc<double>(b->ctx, (size_t)b->n * n_sub);
     b->n_sub_cap = n_sub;
 }
 
@@ -258,30 +258,30 @@ int lt_batch_create(lt_ctx ctx, int n_rep, const int* shapes, int n_levels, doub
             b->total_kb = (int)kb;
             b->total_cb = (int)cb;
 
-            b->d_reps = dev_alloc<lt::BatchRep>(n_rep);
+            b->d_reps = dev_alloc<lt::BatchRep>(b->ctx, n_rep);
             upload(b->d_reps, b->reps.data(), sizeof(lt::BatchRep) * n_rep);
-            b->d_pre = dev_alloc<int>(b->pre.size());
+            b->d_pre = dev_alloc<int>(b->ctx, b->pre.size());
             upload(b->d_pre, b->pre.data(), sizeof(int) * b->pre.size());
 
             const size_t nl = (size_t)b->total;
-            b->U = dev_alloc<double2>(nl);
-            b->Ucopy = dev_alloc<double2>(nl);
-            b->P = dev_alloc<double2>(nl);
-            b->F = dev_alloc<double2>(nl);
-            b->lambda[0] = dev_alloc<double2>((size_t)lt::alg_offset(b->total));
-            b->lambda[1] = dev_alloc<double2>((size_t)lt::alg_offset(b->total));
-            b->clover = dev_alloc<double2>((size_t)lt::clover_offset(b->total));
+            b->U = dev_alloc<double2>(b->ctx, nl);
+            b->Ucopy = dev_alloc<double2>(b->ctx, nl);
+            b->P = dev_alloc<double2>(b->ctx, nl);
+            b->F = dev_alloc<double2>(b->ctx, nl);
+            b->lambda[0] = dev_alloc<double2>(b->ctx, (size_t)lt::alg_offset(b->total));
+            b->lambda[1] = dev_alloc<double2>(b->ctx, (size_t)lt::alg_offset(b->total));
+            b->clover = dev_alloc<double2>(b->ctx, (size_t)lt::clover_offset(b->total));
             b->levels.push_back(b->U);
             for (int l = 0; l < n_levels; ++l) {
-                b->levels.push_back(dev_alloc<double2>(nl));
-                b->tapes.push_back(dev_alloc<double2>((size_t)lt::alg_offset(b->total)));
+                b->levels.push_back(dev_alloc<double2>(b->ctx, nl));
+                b->tapes.push_back(dev_alloc<double2>(b->ctx, (size_t)lt::alg_offset(b->total)));
             }
-            b->part = dev_alloc<double>((size_t)std::max(b->total_sb, b->total_kb));
+            b->part = dev_alloc<double>(b->ctx, (size_t)std::max(b->total_sb, b->total_kb));
 
             // per-replica scalar state, one allocation
             const size_t n = (size_t)n_rep;
             const size_t bytes = n * (8 + 4 + 8 * 10 + 4) + 2 * n * 8 + 3 * 8 + 64;
-            b->state_mem = dev_alloc<char>(bytes);
+            b->state_mem = dev_alloc<char>(b->ctx, bytes);
             size_t o = 0;
             auto take = [&](size_t sz) {
                 char* p = b->state_mem + o;
@@ -351,7 +351,7 @@ int lt_batch_destroy(lt_batch b)
         LT_HIP_CHECK(hipSetDevice(b->ctx->device));
         LT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
         b->release();
-        b->ctx->live -= 1;
+        b->ctx->handle_gone();
         delete b;
         return LT_OK;
     });
@@ -427,7 +427,7 @@ int lt_batch_set_bias(lt_batch b, lt_bias bias)
             b->drop_graph();
             if (b->bias.grid) LT_HIP_CHECK(hipFree(b->bias.grid));
             b->bias.grid = nullptr;
-            b->bias.grid = dev_alloc<double>(ng);
+            b->bias.grid = dev_alloc<double>(b->ctx, ng);
             b->grid_cap = ng;
         }
         lt::DevBias d{};

@@ -84,11 +84,10 @@ bool same_shape(const lt::Geom& a, const lt::Geom& b)
     return true;
 }
 
-double2* alloc_buf(size_t n_double2)
+double2* alloc_buf(lt_ctx ctx, size_t n_double2)
 {
-    double2* p = nullptr;
-    if (hipMalloc(&p, n_double2 * sizeof(double2)) != hipSuccess)
-        throw lt::LtError{LT_ENOMEM, "device allocation failed"};
+    auto* p = (double2*)ctx->device_alloc(n_double2 * sizeof(double2));
+    if (!p) throw lt::LtError{LT_ENOMEM, "device allocation failed"};
     return p;
 }
 
@@ -520,7 +519,7 @@ int lt_cv_create_checkpointed(lt_ctx ctx, int nt, int nx, int ny, int nz, int n_
         cv->interval = interval > 0 ? std::min(interval, std::max(n_levels, 1)) : 0;
         const size_t nl = (size_t)72 * cv->g.Vh, na = (size_t)32 * cv->g.Vh;
         auto take = [&](size_t n) {
-            double2* p = alloc_buf(n);
+            double2* p = alloc_buf(ctx, n);
             cv->bytes += n * sizeof(double2);
             return p;
         };
@@ -555,7 +554,7 @@ int lt_clover_derivative(lt_field U, lt_field F, double scale)
         return fail(LT_EINVAL, "lt_clover_derivative: bad arguments");
     return guarded([&] {
         LT_HIP_CHECK(hipSetDevice(U->ctx->device));
-        double2* clover = alloc_buf((size_t)12 * lt::R_SLOTS * U->g.Vh);
+        double2* clover = alloc_buf(U->ctx, (size_t)12 * lt::R_SLOTS * U->g.Vh);
         try {
             (void)lt::k_clover_charge(U->ctx, U->g, U->d, clover);
             lt::k_clover_deriv(U->ctx, U->g, U->map, U->d, clover, F->d, scale);
@@ -588,7 +587,7 @@ int lt_cv_destroy(lt_cv cv)
     return guarded([&] {
         LT_HIP_CHECK(hipStreamSynchronize(cv->ctx->stream));
         cv->release();
-        cv->ctx->live -= 1;
+        cv->ctx->handle_gone();
         delete cv;
         return LT_OK;
     });

@@ -10,6 +10,7 @@
 #include <exception>
 #include <functional>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -75,8 +76,22 @@ struct lt_ctx_s {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> event_pool;
     std::map<std::string, lt::ProfEntry> prof;
 
+    // second link buffer of multi-level smearing, grown on demand and kept: allocating and
+    // freeing 382 MB in every call took 9 ms where two stout levels of that field take 0.65 ms.
+    // One buffer per context, of the largest field smeared so far; given back with the
+    // context's last handle, and when another allocation of the context fails.  A caller
+    // holds links_mutex while it enqueues the launches that use the buffer (they are ordered
+    // by the stream), so threads sharing a context do not interleave on it.
+    std::mutex links_mutex;
+    double2* links = nullptr;
+    size_t links_n = 0;
+
     double* scratch_for(size_t n);
     double* host_for(size_t n);
+    double2* links_for(size_t n);   // with links_mutex held
+    void links_release();           // takes links_mutex
+    void* device_alloc(size_t bytes);   // null when out of memory
+    void handle_gone();             // a handle was destroyed (its stream work is done)
     void collect_profile();
 };
 
