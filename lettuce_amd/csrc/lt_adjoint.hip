@@ -20,10 +20,12 @@ namespace {
 
 constexpr int CBS = 256;
 
+template <bool KEEP>
 __global__ void LT_LINK_KERNEL stout_tape_kernel(const double2* __restrict__ Uin, double2* __restrict__ Uout,
-                                                 double2* __restrict__ T, Geom g, LinkMap m, double rho)
+                                                 double2* __restrict__ T, Geom g, LinkMap m, double rho,
+                                                 double2* __restrict__ keep)
 {
-    body_stout_tape(Uin, Uout, T, g, m, link_block(m, blockIdx.x, gridDim.x), rho);
+    body_stout_tape<KEEP>(Uin, Uout, T, g, m, link_block(m, blockIdx.x, gridDim.x), rho, keep);
 }
 
 // one thread per (site, plane): the clover term of that plane.  Block b (XCD-remapped)
@@ -77,9 +79,12 @@ __global__ void LT_LINK_KERNEL sigma_all_kernel(const double2* __restrict__ U, d
 
 }  // namespace
 
-void k_stout_tape(lt_ctx ctx, const Geom& g, const LinkMap& m, const double2* in, double2* out, double2* tape, double rho)
+void k_stout_tape(lt_ctx ctx, const Geom& g, const LinkMap& m, const double2* in, double2* out, double2* tape, double rho,
+                  double2* keep)
 {
-    launch(ctx, "stout_tape", stout_tape_kernel, dim3(8 * map_blocks(m)), dim3(m.nthreads), 0, in, out, tape, g, m, rho);
+    auto* k = keep ? stout_tape_kernel<true> : stout_tape_kernel<false>;
+    launch(ctx, "stout_tape", k, dim3(8 * map_blocks(m)), dim3(m.nthreads), 0, in, out, tape, g, m, rho,
+           keep);
 }
 
 double k_clover_charge(lt_ctx ctx, const Geom& g, const double2* U, double2* C)

@@ -965,14 +965,21 @@ int lt_flow_destroy(lt_flow fl)
     });
 }
 
-// One integrator step on fl->flowed; each stage writes the other buffer and the
-// buffers are exchanged, so the flowed field always owns the newest links.
-static void flow_steps(lt_flow fl, int n)
+// n integrator steps on fl->flowed; each stage writes the other buffer and the buffers are
+// exchanged, so the flowed field always owns the newest links.  start (optional): the links
+// of the first stage's field, which then writes the flowed field's own buffer -- a flow from
+// the unflowed field without a copy of it first (604 MB at 32^4, 0.2 ms).
+static void flow_steps(lt_flow fl, int n, const double2* start)
 {
     lt_field u = fl->flowed;
     lt_ctx ctx = u->ctx;
     const double e = fl->eps;
     auto stage = [&](double c_old, double c_new, double c_exp, int read_z, int write_z) {
+        if (start) {
+            lt::k_flow_stage(ctx, u->g, u->map, start, u->d, fl->z, c_old, c_new, c_exp, read_z, write_z);
+            start = nullptr;
+            return;
+        }
         lt::k_flow_stage(ctx, u->g, u->map, u->d, fl->tmp, fl->z, c_old, c_new, c_exp, read_z, write_z);
         std::swap(u->d, fl->tmp);
     };
@@ -992,8 +999,11 @@ int lt_flow_run(lt_flow fl, int n_steps)
     if (!fl || n_steps < 0) return fail(LT_EINVAL, "lt_flow_run: bad argument");
     return guarded([&] {
         use_device(fl->flowed->ctx);
-        lt::k_copy(fl->flowed->ctx, fl->unflowed->d, fl->flowed->d, (size_t)72 * fl->flowed->g.Vh);
-        flow_steps(fl, n_steps);
+        // fields of general matrices keep the copy: their third rows are data of their own
+        const bool direct = n_steps > 0 && fl->unflowed->su3 && fl->flowed->su3;
+        if (!direct)
+            lt::k_copy(fl->flowed->ctx, fl->unflowed->d, fl->flowed->d, (size_t)72 * fl->flowed->g.Vh);
+        flow_steps(fl, n_steps, direct ? fl->unflowed->d : nullptr);
         return LT_OK;
     });
 }
@@ -1003,7 +1013,7 @@ int lt_flow_resume(lt_flow fl, int n_steps)
     if (!fl || n_steps < 0) return fail(LT_EINVAL, "lt_flow_resume: bad argument");
     return guarded([&] {
         use_device(fl->flowed->ctx);
-        flow_steps(fl, n_steps);
+        flow_steps(fl, n_steps, nullptr);
         return LT_OK;
     });
 }

@@ -69,7 +69,7 @@ __global__ void LT_LINK_KERNEL bk_stout_tape(const double2* __restrict__ Uin, do
                                              double2* __restrict__ T, BatchGrid bg, double rho)
 {
     LT_BATCH_LINK_PROLOGUE
-    body_stout_tape(Uin + off, Uout + off, T + alg_offset(off), g, m, lb, rho);
+    body_stout_tape<false>(Uin + off, Uout + off, T + alg_offset(off), g, m, lb, rho, nullptr);
 }
 
 template <bool LAMBDA>

@@ -157,10 +157,13 @@ __device__ __forceinline__ M3 R_at(const double2* __restrict__ C, const Geom& g,
     return rho < sigma ? r : scale(-1.0, r);
 }
 
-// stout level with tape: Q = -i rho Algebra(st U^+), U' = exp(iQ) U, Gram-Schmidt
+// stout level with tape: Q = -i rho Algebra(st U^+), U' = exp(iQ) U, Gram-Schmidt.
+// KEEP: the link read is also stored in keep, which keeps level 0 of a stack without a copy
+// of the field beforehand (a template: tested at run time the branch cost 224 spilled VGPRs).
+template <bool KEEP>
 __device__ __forceinline__ void body_stout_tape(const double2* __restrict__ Uin, double2* __restrict__ Uout,
                                                 double2* __restrict__ T, const Geom& g, const LinkMap& m, int b,
-                                                double rho)
+                                                double rho, double2* __restrict__ keep)
 {
     int mu, par, c[4], s;
     if (!map_link_b(g, m, b, mu, par, c, s)) return;
@@ -179,6 +182,7 @@ __device__ __forceinline__ void body_stout_tape(const double2* __restrict__ Uin,
     Q = her8_round(Q);   // forward and adjoint use exactly the stored exponent
     st_her8(T, g, s, mu, par, Q);
     M3 W = mul(su3_exp(Q), L);
+    if (KEEP) stu_stream(keep, g, s, mu, par, L);
     gram_schmidt(W);
     stu(Uout, g, s, mu, par, W);
 }
