@@ -104,7 +104,7 @@ void k_clover_deriv(lt_ctx ctx, const Geom& g, const LinkMap& m, const double2* 
                     double scale_factor, const SigmaNext* next)
 {
     const dim3 grid(8 * map_blocks(m)), block(m.nthreads);
-    const size_t lds = 18 * m.nthreads * sizeof(double2);
+    const size_t lds = CDERIV_SLOTS * m.nthreads * sizeof(double2);
     if (next)
         launch(ctx, "clover_deriv", clover_deriv_all_kernel<true>, grid, block, lds, U, C, F, g, m, scale_factor, *next);
     else

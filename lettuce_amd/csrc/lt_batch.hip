@@ -398,7 +398,7 @@ void kb_clover_deriv(lt_ctx ctx, const BatchGrid& bg, int total_lb, const double
                      const double* scale, const SigmaNext* next)
 {
     const dim3 grid(total_lb), block(link_threads(bg, total_lb));
-    const size_t lds = 18 * block.x * sizeof(double2);
+    const size_t lds = CDERIV_SLOTS * block.x * sizeof(double2);
     if (next)
         launch(ctx, "batch_clover_deriv", bk_clover_deriv_all<true>, grid, block, lds, U, C, F, bg, scale, *next);
     else

@@ -137,6 +137,13 @@ __device__ __forceinline__ M3 ld_plane(const double2* __restrict__ R, const Geom
     r.m[7] = cd{-a12.x, a12.y};
     return r;
 }
+__device__ __forceinline__ Tri ld_plane_tri(const double2* __restrict__ R, const Geom& g, int s, int plane, int par)
+{
+    const double2* p = R + slot_base(g, plane * 2 + par, R_SLOTS, cbi(g, s));
+    const double2 a01 = p[0], a02 = p[slot_stride(g)], a12 = p[(size_t)2 * slot_stride(g)];
+    const double2 d01 = p[(size_t)3 * slot_stride(g)], d2 = p[(size_t)4 * slot_stride(g)];
+    return Tri{d01.x, d01.y, d2.x, cd{a01.x, a01.y}, cd{a02.x, a02.y}, cd{a12.x, a12.y}};
+}
 // stores R = C - C^+ of the clover term C
 __device__ __forceinline__ void st_plane(double2* __restrict__ R, const Geom& g, int s, int plane, int par, const M3& c)
 {
@@ -218,19 +225,6 @@ __device__ __forceinline__ double body_qdensity_site(const double2* __restrict__
          + retr_mul(R_at(C, g, s, par, 0, 3), R_at(C, g, s, par, 1, 2));
 }
 
-// Clover-charge derivative for link (x, mu) (CloverDerivativeComponent,
-// LettuceGauge/observables/clover.hpp:238-321): for each of the three nu != mu,
-// with (rho, sigma) the remaining directions and s = eps(mu, nu, rho, sigma),
-//   upper: tmp1 (U_nu(x)^+ R(x) + R(x+nu) U_nu(x)^+) + (U_nu(x+mu) R(x+mu+nu) + R(x+mu) U_nu(x+mu)) tmp2
-//   lower: tmp3 (U_nu(x-nu) R(x) + R(x-nu) U_nu(x-nu)) + (U_nu(x+mu-nu)^+ R(x+mu-nu) + R(x+mu) U_nu(x+mu-nu)^+) tmp4
-// with tmp1 = U_nu(x+mu) U_mu(x+nu)^+, tmp2 = U_mu(x+nu)^+ U_nu(x)^+,
-//      tmp3 = U_nu(x+mu-nu)^+ U_mu(x-nu)^+, tmp4 = U_mu(x-nu)^+ U_nu(x-nu),
-// accumulate sum_nu s (upper - lower) and end with
-//   F(x, mu) = scale * (-2/(512 pi^2)) Algebra(U_mu(x) * sum).
-// One half-term alone needs ~210 VGPRs, so the whole sum straight through one thread
-// spills; body_clover_deriv_all runs the halves as a loop with the running sum and one
-// partial product parked in LDS.
-
 // Re tr of the plaquette U_mu(x) U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+ (plaquette.hpp:20-24)
 // as Re tr(A B^+) with A = U_mu(x) U_nu(x+mu), B = U_nu(x) U_mu(x+nu), both in SU(3), of
 // which only rows 0 and 1 are multiplied out (retr_su3_nd_r01).
@@ -271,84 +265,41 @@ __device__ __forceinline__ void plaq_link_partials(const double2* __restrict__ U
     }
 }
 
-// Parking slot (park_store / park_load): the first of the two products of a half waits
-// in LDS while the second is formed, so it holds no registers meanwhile.  park is never
-// null in the kernels: testing it anyway puts the parking in a branch of its own, and the
-// compiler does not hoist the second product's link loads above a branch (19 spilled
-// VGPRs in clover_deriv_all_kernel without the tests, 2 with them).
-
-__device__ __forceinline__ M3 cderiv_upper(const double2* __restrict__ U, const double2* __restrict__ C, const Geom& g,
-                                           int s, const int c[4], int par, int MU, int NU, int RHO, int SIGMA,
-                                           double2* park, int n)
+// Running sums in LDS (entries e * n of a per-lane slot, e < 9): a sum waits there between the
+// directions, so that one half term at a time has the registers; the empty asm statements with
+// memory clobbers keep the compiler from carrying it in registers anyway.
+template <int SG>
+__device__ __forceinline__ void park_acc(double2* slot, int n, const M3& a, bool first)
 {
-    const int q = par ^ 1;
-    const int smu = up(g, s, pick4(c, MU), MU), snu = up(g, s, pick4(c, NU), NU);
-    const M3 Unu_x = ldu(U, g, s, NU, par);
-    M3 tmp1, tmp2;
-    {
-        const M3 Umu_nu = ldu(U, g, snu, MU, q);
-        tmp2 = mul_nd(dag(Umu_nu), Unu_x);
-        tmp1 = mul_nd(ldu(U, g, smu, NU, q), Umu_nu);
-    }
-    M3 S = mul_dn(Unu_x, R_at(C, g, s, par, RHO, SIGMA));
-    S = add(S, mul_nd(R_at(C, g, snu, q, RHO, SIGMA), Unu_x));
-    M3 acc = mul(tmp1, S);
-    if (park) park_store(park, n, acc);
-    const M3 Unu_mu = ldu(U, g, smu, NU, q);
-    S = mul(Unu_mu, R_at(C, g, up(g, smu, pick4(c, NU), NU), par, RHO, SIGMA));
-    S = add(S, mul(R_at(C, g, smu, q, RHO, SIGMA), Unu_mu));
-    const M3 second = mul(S, tmp2);
-    if (park) acc = park_load(park, n);
-    return add(acc, second);
-}
-
-__device__ __forceinline__ M3 cderiv_lower(const double2* __restrict__ U, const double2* __restrict__ C, const Geom& g,
-                                           int s, const int c[4], int par, int MU, int NU, int RHO, int SIGMA,
-                                           double2* park, int n)
-{
-    const int q = par ^ 1;
-    const int smu = up(g, s, pick4(c, MU), MU);
-    const int snd = dn(g, s, pick4(c, NU), NU), smu_nd = dn(g, smu, pick4(c, NU), NU);
-    const M3 Unu_nd = ldu(U, g, snd, NU, q);
-    const M3 Unu_mund = ldu(U, g, smu_nd, NU, par);
-    M3 tmp3, tmp4;
-    {
-        const M3 Umu_nd = ldu(U, g, snd, MU, q);
-        tmp3 = mul_nd(dag(Unu_mund), Umu_nd);
-        tmp4 = mul_dn(Umu_nd, Unu_nd);
-    }
-    M3 S = mul(Unu_nd, R_at(C, g, s, par, RHO, SIGMA));
-    S = add(S, mul(R_at(C, g, snd, q, RHO, SIGMA), Unu_nd));
-    M3 acc = mul(tmp3, S);
-    if (park) park_store(park, n, acc);
-    S = mul_dn(Unu_mund, R_at(C, g, smu_nd, par, RHO, SIGMA));
-    S = add(S, mul_nd(R_at(C, g, smu, q, RHO, SIGMA), Unu_mund));
-    const M3 second = mul(S, tmp4);
-    if (park) acc = park_load(park, n);
-    return add(acc, second);
-}
-
-// All six half terms of link (x, mu) in one pass: upper then lower half of the k-th
-// direction nu != mu, k = 0, 1, 2, summed in that order.  The running sum waits in LDS
-// (acc: entries e * nthreads + lane, e < 9) and the first product of each half in the
-// parking slot after it (acc + 9 * nthreads), so that each half has the registers to
-// itself; the empty asm statements with memory clobbers keep the compiler from carrying
-// them in registers instead.  The directions are loop variables (one copy of the code
-// for every mu and k).  LDS: 18 x 16 bytes per lane of the block.
-__device__ __forceinline__ void lds_acc(double2* acc, int n, const M3& a, int first, int negate)
-{
+    asm volatile("" ::: "memory");
 #pragma unroll
     for (int e = 0; e < 9; ++e) {
-        const cd v = a.m[e];
+        const cd v = SG > 0 ? a.m[e] : -a.m[e];
         if (first) {
-            acc[e * n] = make_double2(v.re, v.im);
+            slot[e * n] = make_double2(v.re, v.im);
         } else {
-            const double2 o = acc[e * n];
-            acc[e * n] = negate ? make_double2(o.x - v.re, o.y - v.im) : make_double2(o.x + v.re, o.y + v.im);
+            const double2 o = slot[e * n];
+            slot[e * n] = make_double2(o.x + v.re, o.y + v.im);
         }
     }
     asm volatile("" ::: "memory");
 }
+
+// Clover-charge derivative for link (x, mu) (CloverDerivativeComponent,
+// LettuceGauge/observables/clover.hpp:238-321): for each of the three nu != mu, with (rho,
+// sigma) the remaining directions, R their clover plane and s = eps(mu, nu, rho, sigma), the
+// reference's eight products per half regroup to
+//   upper = S R(x) + R(x+mu) S + c (b^+ R(x+nu) + R(x+mu+nu) b^+) a^+,  S = c b^+ a^+
+//   lower = T R(x) + R(x+mu) T + f^+ (e^+ R(x-nu) + R(x+mu-nu) e^+) d,  T = f^+ e^+ d
+// with a = U_nu(x), b = U_mu(x+nu), c = U_nu(x+mu), d = U_nu(x-nu), e = U_mu(x-nu),
+// f = U_nu(x+mu-nu), so that the terms with R(x) and R(x+mu) are taken once, of S - T, and
+// the staples S, T are SU(3) matrices of which two rows are multiplied out.  The sum of
+// s (upper - lower) over nu ends with
+//   F(x, mu) = scale * (-2/(512 pi^2)) Algebra(U_mu(x) * sum).
+// The running sum waits in LDS, as do S's two rows while the lower half is formed.  About
+// 1500 FP64 instructions per nu instead of 1900.
+// LDS: 15 x 16 bytes per lane of the block.
+constexpr int CDERIV_SLOTS = 15;
 __device__ __forceinline__ void lambda_link(const double2* __restrict__ U, const M3& Lprev, const M3& sig,
                                             double2* __restrict__ Sig, const double2* __restrict__ T,
                                             double2* __restrict__ Lam, const Geom& g, int s, int mu, int par);
@@ -358,11 +309,14 @@ __device__ __forceinline__ void lambda_link(const double2* __restrict__ U, const
 template <bool LAMBDA>
 __device__ __forceinline__ void body_clover_deriv_all(const double2* __restrict__ U, const double2* __restrict__ C,
                                                       double2* __restrict__ F, const Geom& g, const LinkMap& m, int b,
-                                                      double scale_factor, double2* acc, const SigmaNext& next)
+                                                      double scale_factor, double2* lds, const SigmaNext& next)
 {
     int mu, par, c[4], s;
     if (!map_link_b(g, m, b, mu, par, c, s)) return;
-    acc += threadIdx.x;
+    const int n = m.nthreads, q = par ^ 1;
+    double2* sum = lds + threadIdx.x;
+    double2* wait = sum + 9 * n;
+    const int smu = up(g, s, pick4(c, mu), mu);
 #pragma unroll 1
     for (int k = 0; k < 3; ++k) {
         const int nu = k < mu ? k : k + 1;
@@ -370,15 +324,46 @@ __device__ __forceinline__ void body_clover_deriv_all(const double2* __restrict_
         const int sigma = (mu != 3 && nu != 3) ? 3 : ((mu != 2 && nu != 2) ? 2 : 1);
         const int inv = (mu > nu) + (mu > rho) + (mu > sigma) + (nu > rho) + (nu > sigma) + (rho > sigma);
         const double sign = (inv & 1) ? -1.0 : 1.0;
-        double2* park = acc + 9 * m.nthreads;
-        lds_acc(acc, m.nthreads, scale(sign, cderiv_upper(U, C, g, s, c, par, mu, nu, rho, sigma, park, m.nthreads)),
-                k == 0, 0);
-        lds_acc(acc, m.nthreads, scale(sign, cderiv_lower(U, C, g, s, c, par, mu, nu, rho, sigma, park, m.nthreads)), 0,
-                1);
-    }
-    M3 a;
+        const int plane = plane_of(rho, sigma);
+        const int cnu = pick4(c, nu);
+        {
+            const int snu = up(g, s, cnu, nu);
+            const M3 bd = dag(ldu(U, g, snu, mu, q));
+            const M3 cc = ldu(U, g, smu, nu, q);
+            const M3 a = ldu(U, g, s, nu, par);
+            const M3 S = mul_nd_r01(mul_r01(cc, bd), a);
+            asm volatile("" ::: "memory");
 #pragma unroll
-    for (int e = 0; e < 9; ++e) a.m[e] = cd{acc[e * m.nthreads].x, acc[e * m.nthreads].y};
+            for (int e = 0; e < 6; ++e) wait[e * n] = make_double2(S.m[e].re, S.m[e].im);
+            asm volatile("" ::: "memory");
+            M3 K = m3_zero();
+            mul_tri_acc<true, 1>(K, bd, ld_plane_tri(C, g, snu, plane, q));
+            tri_mul_acc<true, 1>(K, ld_plane_tri(C, g, up(g, smu, cnu, nu), plane, par), bd);
+            park_acc<1>(sum, n, scale(sign, mul_nd(mul(cc, K), a)), k == 0);
+        }
+        {
+            const int snd = dn(g, s, cnu, nu), smu_nd = dn(g, smu, cnu, nu);
+            const M3 ed = dag(ldu(U, g, snd, mu, q));
+            const M3 f = ldu(U, g, smu_nd, nu, par);
+            const M3 d = ldu(U, g, snd, nu, q);
+            M3 D = mul_r01(mul_dn_r01(f, ed), d);
+            third_row(D);
+            M3 K = m3_zero();
+            mul_tri_acc<true, 1>(K, ed, ld_plane_tri(C, g, snd, plane, q));
+            tri_mul_acc<true, 1>(K, ld_plane_tri(C, g, smu_nd, plane, par), ed);
+            M3 X = mul(mul_dn(f, K), d);
+            asm volatile("" ::: "memory");
+            M3 S;
+#pragma unroll
+            for (int e = 0; e < 6; ++e) S.m[e] = cd{wait[e * n].x, wait[e * n].y};
+            third_row(S);
+            D = sub(D, S);   // T - S
+            mul_tri_acc<true, 1>(X, D, ld_plane_tri(C, g, s, plane, par));
+            tri_mul_acc<true, 1>(X, ld_plane_tri(C, g, smu, plane, q), D);
+            park_acc<-1>(sum, n, scale(sign, X), false);
+        }
+    }
+    M3 a = park_load(sum, n);
     const double pref = -2.0 / (512.0 * 3.14159265358979323846 * 3.14159265358979323846);
     const M3 L = ldu(U, g, s, mu, par);
     a = scale(scale_factor * pref, algebra(mul(L, a)));
@@ -421,12 +406,15 @@ __device__ __forceinline__ void body_lambda(const double2* __restrict__ U, const
     lambda_link(U, ldu(Uprev, g, s, mu, par), ld(Sig, g, s, mu, par), Sig, T, Lam, g, s, mu, par);
 }
 
-// body_sigma_fs and body_sigma in one pass: the six-term sum and the staple st are
-// built in the same loop over nu != mu from the same neighbour links (the staple with
-// the products of staple(), in its order), each waiting in LDS between the directions
-// (fs at lds + lane, st after it: entries e * nthreads, e < 9), then the sigma update.
-// The same operations in the same order as the two launches: the same Sigma bit for
-// bit, without the scratch field Fs and the second reading of the neighbours.
+// The six-term sum and the staple st are formed in one loop over nu != mu from the same
+// neighbour links, each waiting in LDS between the halves (fs at lds + lane, st after it:
+// entries e * nthreads, e < 9), then the sigma update.  With a = U_nu(x), b = U_mu(x+nu),
+// c = U_nu(x+mu), d = U_nu(x-nu), e = U_mu(x-nu), f = U_nu(x+mu-nu), t = a b c^+ and
+// d^+ e f the two staple terms and L the Lambda fields, the reference's products regroup to
+//   upper: t^+ L_nu(x) - L_nu(x+mu) t^+ + c b^+ L_mu(x+nu) a^+
+//   lower: f^+ (e^+ (L_mu(x-nu) - L_nu(x-nu)) + L_nu(x+mu-nu) e^+) d
+// The products with a Lambda use that it is hermitian (mul_tri_acc).  About 1250 FP64
+// instructions per nu instead of 1450.
 // LDS: 18 x 16 bytes per lane of the block.
 // MODE SIGMA_STORE stores the result in Sig.  SIGMA_LAMBDA goes on with the Lambda of the
 // level below for the same link (lambda_link: its Uprev is this level's U, whose link is
@@ -461,51 +449,35 @@ __device__ __forceinline__ void body_sigma_all(const double2* __restrict__ U, do
         const int cnu = pick4(c, nu);
         const int snu = up(g, s, cnu, nu), snd = dn(g, s, cnu, nu);
         const int smu_nd = dn(g, smu, cnu, nu);
-        const M3 Unu_x = ldu(U, g, s, nu, par);
-        const M3 Unu_mu = ldu(U, g, smu, nu, q);
-        M3 tmp1;
         {
-            const M3 Umu_nu = ldu(U, g, snu, mu, q);
-            // staple, upper term: U_nu(x) U_mu(x+nu) U_nu(x+mu)^+
-            const M3 t = mul_nd_r01(mul_r01(Unu_x, Umu_nu), Unu_mu);
-            M3 st;
-            if (k == 0) {
-                st = t;
-                third_row(st);
-            } else {
-                st = park_load(st_slot, n);
-                acc_su3_r01(st, t);
-            }
-            park_store(st_slot, n, st);
-            tmp1 = mul_nd(Unu_mu, Umu_nu);
+            const M3 a = ldu(U, g, s, nu, par);
+            const M3 b = ldu(U, g, snu, mu, q);
+            const M3 cc = ldu(U, g, smu, nu, q);
+            M3 t = mul_nd_r01(mul_r01(a, b), cc);   // staple, upper term
+            third_row(t);
+            park_acc<1>(st_slot, n, t, k == 0);
+            M3 K = m3_zero();
+            mul_tri_acc<false, 1>(K, dag(b), ld_her8_tri(Lam, g, snu, mu, q));
+            M3 X = mul_nd(mul(cc, K), a);
+            t = dag(t);
+            mul_tri_acc<false, 1>(X, t, ld_her8_tri(Lam, g, s, nu, par));
+            tri_mul_acc<false, -1>(X, ld_her8_tri(Lam, g, smu, nu, q), t);
+            park_acc<1>(fs_slot, n, X, k == 0);
         }
-        {   // six-term sum: + tmp1 (U_nu(x)^+ L_nu(x) + L_mu(x+nu) U_nu(x)^+) - L_nu(x+mu) tmp1 U_nu(x)^+
-            const M3 x1 = mul(tmp1, add(mul_dn(Unu_x, ld_her8(Lam, g, s, nu, par)), mul_nd(ld_her8(Lam, g, snu, mu, q), Unu_x)));
-            M3 fs = k == 0 ? m3_zero() : park_load(fs_slot, n);
-            acc(fs, x1);
-            park_store(fs_slot, n, fs);
-            const M3 x2 = mul_nd(mul(ld_her8(Lam, g, smu, nu, q), tmp1), Unu_x);
-            fs = park_load(fs_slot, n);
-            fs = sub(fs, x2);
-            park_store(fs_slot, n, fs);
-        }
-        const M3 Umu_nd = ldu(U, g, snd, mu, q);
-        const M3 Unu_mund = ldu(U, g, smu_nd, nu, par);
-        const M3 Unu_nd = ldu(U, g, snd, nu, q);
-        {   // staple, lower term: U_nu(x-nu)^+ U_mu(x-nu) U_nu(x-nu+mu)
-            M3 ef = mul_r01(Umu_nd, Unu_mund);
-            third_row(ef);
-            M3 st = park_load(st_slot, n);
-            mul_dn_acc(st, Unu_nd, ef);
-            park_store(st_slot, n, st);
-        }
-        {   // + U_nu(x+mu-nu)^+ (U_mu(x-nu)^+ (L_mu(x-nu) - L_nu(x-nu)) + L_nu(x+mu-nu) U_mu(x-nu)^+) U_nu(x-nu)
-            M3 tmp2 = mul_dn(Umu_nd, sub(ld_her8(Lam, g, snd, mu, q), ld_her8(Lam, g, snd, nu, q)));
-            M3 inner = add(tmp2, mul_nd(ld_her8(Lam, g, smu_nd, nu, par), Umu_nd));
-            const M3 x3 = mul(mul_dn(Unu_mund, inner), Unu_nd);
-            M3 fs = park_load(fs_slot, n);
-            acc(fs, x3);
-            park_store(fs_slot, n, fs);
+        {
+            const M3 e = ldu(U, g, snd, mu, q);
+            const M3 f = ldu(U, g, smu_nd, nu, par);
+            const M3 d = ldu(U, g, snd, nu, q);
+            M3 t = mul_r01(e, f);
+            third_row(t);
+            t = mul_dn_r01(d, t);                   // staple, lower term
+            third_row(t);
+            park_acc<1>(st_slot, n, t, false);
+            const M3 ed = dag(e);
+            M3 K = m3_zero();
+            mul_tri_acc<false, 1>(K, ed, ld_her8_tri(Lam, g, snd, mu, q) - ld_her8_tri(Lam, g, snd, nu, q));
+            tri_mul_acc<false, 1>(K, ld_her8_tri(Lam, g, smu_nd, nu, par), ed);
+            park_acc<1>(fs_slot, n, mul(mul_dn(f, K), d), false);
         }
     }
     M3 cl = mul_dn(park_load(st_slot, n), ld_her8(Lam, g, s, mu, par));   // st^+ Lambda

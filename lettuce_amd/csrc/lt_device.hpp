@@ -929,6 +929,83 @@ __device__ __forceinline__ M3 her8_round(const M3& q)
     r.m[7] = conj(q.m[5]);
     return r;
 }
+// Hermitian or anti-hermitian 3x3 matrices in 9 reals: the diagonal (d, or i d where AH) and
+// the upper triangle; the lower triangle is conj (-conj where AH) of the upper one.
+struct Tri {
+    double d0, d1, d2;
+    cd r01, r02, r12;
+};
+__device__ __forceinline__ Tri ld_her8_tri(const double2* __restrict__ Z, const Geom& g, int s, int mu, int par)
+{
+    const double2* p = Z + slot_base(g, mu * 2 + par, 4, cbi(g, s));
+    const double2 v0 = p[0], v1 = p[slot_stride(g)], v2 = p[(size_t)2 * slot_stride(g)], v3 = p[(size_t)3 * slot_stride(g)];
+    return Tri{v0.x, v0.y, -(v0.x + v0.y), cd{v1.x, v1.y}, cd{v2.x, v2.y}, cd{v3.x, v3.y}};
+}
+__device__ __forceinline__ Tri operator-(const Tri& a, const Tri& b)
+{
+    return Tri{a.d0 - b.d0, a.d1 - b.d1, a.d2 - b.d2, a.r01 - b.r01, a.r02 - b.r02, a.r12 - b.r12};
+}
+// c += SG a d (i a d where AH), SG = +-1
+template <bool AH, int SG>
+__device__ __forceinline__ void diag_acc(cd& c, cd a, double d)
+{
+    if (AH) {
+        c.re = fma(SG > 0 ? -a.im : a.im, d, c.re);
+        c.im = fma(SG > 0 ? a.re : -a.re, d, c.im);
+    } else {
+        c.re = fma(SG > 0 ? a.re : -a.re, d, c.re);
+        c.im = fma(SG > 0 ? a.im : -a.im, d, c.im);
+    }
+}
+// c += SG a b
+template <int SG>
+__device__ __forceinline__ void cmul_acc(cd& c, cd a, cd b)
+{
+    const double s = SG > 0 ? 1.0 : -1.0;
+    c.re = fma(s * a.re, b.re, c.re);
+    c.re = fma(-s * a.im, b.im, c.re);
+    c.im = fma(s * a.re, b.im, c.im);
+    c.im = fma(s * a.im, b.re, c.im);
+}
+// C += SG A R and C += SG R A for R hermitian (AH: anti-hermitian): 10 FP64 instructions per
+// complex entry instead of 12, the zero parts of the diagonal left out
+template <bool AH, int SG>
+__device__ __forceinline__ void mul_tri_acc(M3& C, const M3& A, const Tri& R)
+{
+    constexpr int LO = AH ? -SG : SG;   // sign of the conjugated lower triangle
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const cd x = A.m[3 * i], y = A.m[3 * i + 1], z = A.m[3 * i + 2];
+        diag_acc<AH, SG>(C.m[3 * i], x, R.d0);
+        cmul_acc<LO>(C.m[3 * i], y, conj(R.r01));
+        cmul_acc<LO>(C.m[3 * i], z, conj(R.r02));
+        cmul_acc<SG>(C.m[3 * i + 1], x, R.r01);
+        diag_acc<AH, SG>(C.m[3 * i + 1], y, R.d1);
+        cmul_acc<LO>(C.m[3 * i + 1], z, conj(R.r12));
+        cmul_acc<SG>(C.m[3 * i + 2], x, R.r02);
+        cmul_acc<SG>(C.m[3 * i + 2], y, R.r12);
+        diag_acc<AH, SG>(C.m[3 * i + 2], z, R.d2);
+    }
+}
+template <bool AH, int SG>
+__device__ __forceinline__ void tri_mul_acc(M3& C, const Tri& R, const M3& A)
+{
+    constexpr int LO = AH ? -SG : SG;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const cd x = A.m[j], y = A.m[3 + j], z = A.m[6 + j];
+        diag_acc<AH, SG>(C.m[j], x, R.d0);
+        cmul_acc<SG>(C.m[j], R.r01, y);
+        cmul_acc<SG>(C.m[j], R.r02, z);
+        cmul_acc<LO>(C.m[3 + j], conj(R.r01), x);
+        diag_acc<AH, SG>(C.m[3 + j], y, R.d1);
+        cmul_acc<SG>(C.m[3 + j], R.r12, z);
+        cmul_acc<LO>(C.m[6 + j], conj(R.r02), x);
+        cmul_acc<LO>(C.m[6 + j], conj(R.r12), y);
+        diag_acc<AH, SG>(C.m[6 + j], z, R.d2);
+    }
+}
+
 // complex-double offset of a replica's 8-real field given its link-field offset
 __host__ __device__ constexpr long long alg_offset(long long link_off) { return link_off / 72 * 32; }
 
