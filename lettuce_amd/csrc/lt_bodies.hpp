@@ -186,9 +186,8 @@ __device__ __forceinline__ void body_stout_tape(const double2* __restrict__ Uin,
     M3 Q;
 #pragma unroll
     for (int k = 0; k < 9; ++k) Q.m[k] = cd{rho * A.m[k].im, -rho * A.m[k].re};
-    Q = her8_round(Q);   // forward and adjoint use exactly the stored exponent
     st_her8(T, g, s, mu, par, Q);
-    M3 W = mul(su3_exp(Q), L);
+    M3 W = mul(exp_her(Tri{Q.m[0].re, Q.m[4].re, -(Q.m[0].re + Q.m[4].re), Q.m[1], Q.m[2], Q.m[5]}), L);
     if (KEEP) stu_stream(keep, g, s, mu, par, L);
     gram_schmidt(W);
     stu(Uout, g, s, mu, par, W);
@@ -269,18 +268,14 @@ __device__ __forceinline__ void plaq_link_partials(const double2* __restrict__ U
 // directions, so that one half term at a time has the registers; the empty asm statements with
 // memory clobbers keep the compiler from carrying it in registers anyway.
 template <int SG>
-__device__ __forceinline__ void park_acc(double2* slot, int n, const M3& a, bool first)
+__device__ __forceinline__ void park_acc(double2* slot, int n, const M3& a)
 {
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int e = 0; e < 9; ++e) {
-        const cd v = SG > 0 ? a.m[e] : -a.m[e];
-        if (first) {
-            slot[e * n] = make_double2(v.re, v.im);
-        } else {
-            const double2 o = slot[e * n];
-            slot[e * n] = make_double2(o.x + v.re, o.y + v.im);
-        }
+        const double2 o = slot[e * n];
+        slot[e * n] = SG > 0 ? make_double2(o.x + a.m[e].re, o.y + a.m[e].im)
+                             : make_double2(o.x - a.m[e].re, o.y - a.m[e].im);
     }
     asm volatile("" ::: "memory");
 }
@@ -316,6 +311,7 @@ __device__ __forceinline__ void body_clover_deriv_all(const double2* __restrict_
     const int n = m.nthreads, q = par ^ 1;
     double2* sum = lds + threadIdx.x;
     double2* wait = sum + 9 * n;
+    park_store(sum, n, m3_zero());
     const int smu = up(g, s, pick4(c, mu), mu);
 #pragma unroll 1
     for (int k = 0; k < 3; ++k) {
@@ -339,7 +335,7 @@ __device__ __forceinline__ void body_clover_deriv_all(const double2* __restrict_
             M3 K = m3_zero();
             mul_tri_acc<true, 1>(K, bd, ld_plane_tri(C, g, snu, plane, q));
             tri_mul_acc<true, 1>(K, ld_plane_tri(C, g, up(g, smu, cnu, nu), plane, par), bd);
-            park_acc<1>(sum, n, scale(sign, mul_nd(mul(cc, K), a)), k == 0);
+            park_acc<1>(sum, n, scale(sign, mul_nd(mul(cc, K), a)));
         }
         {
             const int snd = dn(g, s, cnu, nu), smu_nd = dn(g, smu, cnu, nu);
@@ -360,7 +356,7 @@ __device__ __forceinline__ void body_clover_deriv_all(const double2* __restrict_
             D = sub(D, S);   // T - S
             mul_tri_acc<true, 1>(X, D, ld_plane_tri(C, g, s, plane, par));
             tri_mul_acc<true, 1>(X, ld_plane_tri(C, g, smu, plane, q), D);
-            park_acc<-1>(sum, n, scale(sign, X), false);
+            park_acc<-1>(sum, n, scale(sign, X));
         }
     }
     M3 a = park_load(sum, n);
@@ -382,20 +378,38 @@ __device__ __forceinline__ void lambda_link(const double2* __restrict__ U, const
 {
     M3 sp = mul_dn(Lprev, sig);
     st_link(Sig, g, s, mu, par, sp);
-    M3 Q = ld_her8(T, g, s, mu, par);
-    M3 Q2 = mul(Q, Q);
-    ExpC e;
-    exp_constants(Q, Q2, e);
-    M3 B1, B2;
-    cd f1, f2;
-    exp_deriv(e, Q, Q2, B1, B2, f1, f2);
-    M3 G = mul(ldu(U, g, s, mu, par), sp);
-    cd t1 = trace(mul(B1, G)), t2 = trace(mul(B2, G));
-    M3 QG = add(mul(Q, G), mul(G, Q));
+    const Tri Q = ld_her8_tri(T, g, s, mu, par);
+    const M3 G = mul(ldu(U, g, s, mu, par), sp);
+    M3 QG = m3_zero();   // Q G + G Q, of trace 2 tr(Q G)
+    mul_tri_acc<false, 1>(QG, G, Q);
+    tri_mul_acc<false, 1>(QG, Q, G);
+    const Tri Q2 = her_square(Q);
+    ExpDeriv d;
+    exp_deriv(her_det(Q), 0.5 * (Q2.d0 + Q2.d1 + Q2.d2), d);
+    // tr(B_i G) = b_i0 tr G + b_i1 tr(Q G) + b_i2 tr(Q^2 G)
+    const cd tg = trace(G), tqg = 0.5 * trace(QG);
+    cd tq2g = Q2.d0 * G.m[0] + Q2.d1 * G.m[4] + Q2.d2 * G.m[8];
+    cmul_acc<1>(tq2g, Q2.r01, G.m[3]);
+    cmul_acc<1>(tq2g, Q2.r02, G.m[6]);
+    cmul_acc<1>(tq2g, Q2.r12, G.m[7]);
+    cmul_acc<1>(tq2g, conj(Q2.r01), G.m[1]);
+    cmul_acc<1>(tq2g, conj(Q2.r02), G.m[2]);
+    cmul_acc<1>(tq2g, conj(Q2.r12), G.m[5]);
+    const cd t1 = d.b10 * tg + d.b11 * tqg + d.b12 * tq2g;
+    const cd t2 = d.b20 * tg + d.b21 * tqg + d.b22 * tq2g;
+    // traceless hermitian part of t1 Q + t2 Q^2 + f1 G + f2 (Q G + G Q): Q and Q^2 are
+    // hermitian, so only the real parts of t1 and t2 stay
     M3 Gam;
 #pragma unroll
-    for (int k = 0; k < 9; ++k) Gam.m[k] = t1 * Q.m[k] + t2 * Q2.m[k] + f1 * G.m[k] + f2 * QG.m[k];
-    st_her8(Lam, g, s, mu, par, tl_herm(Gam));
+    for (int k = 0; k < 9; ++k) Gam.m[k] = d.f1 * G.m[k] + d.f2 * QG.m[k];
+    Gam.m[0].re += t1.re * Q.d0 + t2.re * Q2.d0;
+    Gam.m[4].re += t1.re * Q.d1 + t2.re * Q2.d1;
+    Gam.m[8].re += t1.re * Q.d2 + t2.re * Q2.d2;
+    Gam = tl_herm(Gam);
+    Gam.m[1] += t1.re * Q.r01 + t2.re * Q2.r01;
+    Gam.m[2] += t1.re * Q.r02 + t2.re * Q2.r02;
+    Gam.m[5] += t1.re * Q.r12 + t2.re * Q2.r12;
+    st_her8(Lam, g, s, mu, par, Gam);
 }
 __device__ __forceinline__ void body_lambda(const double2* __restrict__ U, const double2* __restrict__ Uprev,
                                             double2* __restrict__ Sig, const double2* __restrict__ T,
@@ -441,6 +455,8 @@ __device__ __forceinline__ void body_sigma_all(const double2* __restrict__ U, do
     const int n = m.nthreads;
     double2* fs_slot = lds + threadIdx.x;
     double2* st_slot = fs_slot + 9 * n;
+    park_store(fs_slot, n, m3_zero());
+    park_store(st_slot, n, m3_zero());
     const int q = par ^ 1;
     const int smu = up(g, s, pick4(c, mu), mu);
 #pragma unroll 1
@@ -455,14 +471,14 @@ __device__ __forceinline__ void body_sigma_all(const double2* __restrict__ U, do
             const M3 cc = ldu(U, g, smu, nu, q);
             M3 t = mul_nd_r01(mul_r01(a, b), cc);   // staple, upper term
             third_row(t);
-            park_acc<1>(st_slot, n, t, k == 0);
+            park_acc<1>(st_slot, n, t);
             M3 K = m3_zero();
             mul_tri_acc<false, 1>(K, dag(b), ld_her8_tri(Lam, g, snu, mu, q));
             M3 X = mul_nd(mul(cc, K), a);
             t = dag(t);
             mul_tri_acc<false, 1>(X, t, ld_her8_tri(Lam, g, s, nu, par));
             tri_mul_acc<false, -1>(X, ld_her8_tri(Lam, g, smu, nu, q), t);
-            park_acc<1>(fs_slot, n, X, k == 0);
+            park_acc<1>(fs_slot, n, X);
         }
         {
             const M3 e = ldu(U, g, snd, mu, q);
@@ -472,17 +488,18 @@ __device__ __forceinline__ void body_sigma_all(const double2* __restrict__ U, do
             third_row(t);
             t = mul_dn_r01(d, t);                   // staple, lower term
             third_row(t);
-            park_acc<1>(st_slot, n, t, false);
+            park_acc<1>(st_slot, n, t);
             const M3 ed = dag(e);
             M3 K = m3_zero();
             mul_tri_acc<false, 1>(K, ed, ld_her8_tri(Lam, g, snd, mu, q) - ld_her8_tri(Lam, g, snd, nu, q));
             tri_mul_acc<false, 1>(K, ld_her8_tri(Lam, g, smu_nd, nu, par), ed);
-            park_acc<1>(fs_slot, n, mul(mul_dn(f, K), d), false);
+            park_acc<1>(fs_slot, n, mul(mul_dn(f, K), d));
         }
     }
-    M3 cl = mul_dn(park_load(st_slot, n), ld_her8(Lam, g, s, mu, par));   // st^+ Lambda
+    M3 cl = m3_zero();   // st^+ Lambda
+    mul_tri_acc<false, 1>(cl, dag(park_load(st_slot, n)), ld_her8_tri(Lam, g, s, mu, par));
     const M3 fs = park_load(fs_slot, n);
-    M3 inner = mul(ld(Sig, g, s, mu, par), su3_exp(ld_her8(T, g, s, mu, par)));
+    M3 inner = mul(ld(Sig, g, s, mu, par), exp_her(ld_her8_tri(T, g, s, mu, par)));
 #pragma unroll
     for (int e = 0; e < 9; ++e) {
         cd d = cl.m[e] - fs.m[e];

@@ -468,73 +468,132 @@ __device__ __forceinline__ void exp_constants_c(double c0s, double c1, ExpC& e)
     e.h2 = h2;
 }
 
-// Q2 = Q*Q must be supplied by the caller (it is needed again for the exponential).
-__device__ __forceinline__ void exp_constants(const M3& Q, const M3& Q2, ExpC& e)
-{
-    exp_constants_c((1.0 / 3.0) * retr_mul(Q, Q2), 0.5 * (Q2.m[0].re + Q2.m[4].re + Q2.m[8].re), e);
-}
+// exp(iQ) = f0 + f1 Q + f2 Q^2 by the power series reduced with Cayley-Hamilton: with
+// Q^3 = c1 Q + c0 (c1 = tr Q^2 / 2, c0 = det Q) every power is Q^k = c0 G_{k-1} + G_{k+1} Q +
+// G_k Q^2 where G_{k+1} = c1 G_{k-1} + c0 G_{k-2}, G_0 = G_1 = 0, G_2 = 1, so
+//   f0 = 1 + c0 sum_k i^k/k! G_{k-1},  f1 = sum_k i^k/k! G_{k+1},  f2 = sum_k i^k/k! G_k:
+// five FP64 instructions per term, no branches and no transcendental functions (the closed
+// form above takes an arc cosine and three sine-cosine pairs).  The derivatives of G with
+// respect to c1 and c0 are H_k and H_{k-1} with H_{k+1} = G_{k-1} + c1 H_{k-1} + c0 H_{k-2}
+// (both have the generating function z^4 / (1 - c1 z^2 - c0 z^3)^2 up to a power of z), so
+// the derivatives of f0, f1, f2 follow from one more sequence.
+// The largest omitted terms of all eight coefficients are below 6e-18 with k <= 12 for
+// c1 <= 0.02 (the Wilson flow's exponents) and 2e-18 with k <= 20 for c1 <= 1 (a stout step:
+// c1 <= (6 rho)^2 3/2, 0.78 for rho = 0.12; the closed form loses digits to its denominator
+// 9 u^2 - w^2 there).
+constexpr double EXP_SERIES_SMALL = 0.02, EXP_SERIES_C1 = 1.0;
+constexpr int EXP_TERMS_SMALL = 12, EXP_TERMS = 20;
 
-__device__ __forceinline__ M3 exp_from(const ExpC& e, const M3& Q, const M3& Q2)
+// z += i^k x
+template <int K4>
+__device__ __forceinline__ void acc_ik(cd& z, double t, double x)
 {
-    M3 r;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) r.m[i] = e.denom * (e.h1 * Q.m[i] + e.h2 * Q2.m[i]);
-    r.m[0] += e.denom * e.h0;
-    r.m[4] += e.denom * e.h0;
-    r.m[8] += e.denom * e.h0;
-    return r;
+    if (K4 == 0) z.re = fma(t, x, z.re);
+    if (K4 == 1) z.im = fma(t, x, z.im);
+    if (K4 == 2) z.re = fma(-t, x, z.re);
+    if (K4 == 3) z.im = fma(-t, x, z.im);
 }
-
-// exp(iQ) = f0 + f1 Q + f2 Q^2 for small Q by the power series reduced with
-// Cayley-Hamilton, Q^3 = c1 Q + c0 (c1 = tr Q^2 / 2, c0 = det Q): with
-// Q^k / k! = a_k + b_k Q + g_k Q^2,
-//   a_{k+1} = g_k c0 / (k+1),  b_{k+1} = (a_k + g_k c1) / (k+1),  g_{k+1} = b_k / (k+1),
-// f_j = sum_k i^k (a_k, b_k, g_k).  For c1 <= EXP_SERIES_C1 (|Q|_F <= 0.2) the 13
-// terms k = 0..12 leave a remainder below 0.2^13 / 13! ~ 1e-19; no transcendental
-// functions are needed (the Wilson-flow exponents are always this small).
-constexpr double EXP_SERIES_C1 = 0.02;
-__device__ __forceinline__ void exp_series_coeffs(double c0, double c1, cd& f0, cd& f1, cd& f2)
+__device__ __forceinline__ void acc_ik(cd& z, int k, double t, double x)
 {
-    double a = 1.0, b = 0.0, gg = 0.0;
-    double f0r = 0.0, f0i = 0.0, f1r = 0.0, f1i = 0.0, f2r = 0.0, f2i = 0.0;
-#pragma unroll
-    for (int k = 0; k <= 12; ++k) {
-        switch (k & 3) {   // i^k
-            case 0: f0r += a; f1r += b; f2r += gg; break;
-            case 1: f0i += a; f1i += b; f2i += gg; break;
-            case 2: f0r -= a; f1r -= b; f2r -= gg; break;
-            default: f0i -= a; f1i -= b; f2i -= gg; break;
-        }
-        const double inv = 1.0 / (double)(k + 1);
-        const double an = gg * c0 * inv, bn = fma(gg, c1, a) * inv, gn = b * inv;
-        a = an;
-        b = bn;
-        gg = gn;
+    switch (k & 3) {
+        case 0: acc_ik<0>(z, t, x); break;
+        case 1: acc_ik<1>(z, t, x); break;
+        case 2: acc_ik<2>(z, t, x); break;
+        default: acc_ik<3>(z, t, x); break;
     }
-    f0 = cd{f0r, f0i};
-    f1 = cd{f1r, f1i};
-    f2 = cd{f2r, f2i};
+}
+template <int K>
+__device__ __forceinline__ void exp_series(double c0, double c1, cd& f0, cd& f1, cd& f2)
+{
+    cd s0 = cd{0.0, 0.0};
+    f1 = cd{0.0, 1.0};        // k = 1: G_2 = 1
+    f2 = cd{0.0, 0.0};
+    double gm = 0.0, g = 0.0, gp = 1.0;   // G_{k-1}, G_k, G_{k+1} at k = 1
+    double t = 1.0;                       // 1/k!
+#pragma unroll
+    for (int k = 2; k <= K; ++k) {
+        const double next = k == 2 ? 0.0 : fma(c1, g, c0 * gm);   // G_{k+1}
+        gm = g;
+        g = gp;
+        gp = next;
+        t /= (double)k;
+        if (k >= 3) acc_ik(s0, k, t, gm);
+        acc_ik(f2, k, t, g);
+        if (k >= 3) acc_ik(f1, k, t, gp);
+    }
+    f0 = cd{fma(c0, s0.re, 1.0), c0 * s0.im};
+}
+// f1, f2 and the derivatives b1j = df_j/dc1, b2j = df_j/dc0 (the b_ij of Morningstar-Peardon)
+struct ExpDeriv {
+    cd f1, f2, b10, b11, b12, b20, b21, b22;
+};
+template <int K>
+__device__ __forceinline__ void exp_series_deriv(double c0, double c1, ExpDeriv& d)
+{
+    cd s0 = cd{0.0, 0.0}, h2 = cd{0.0, 0.0}, h1 = cd{0.0, 0.0}, h0 = cd{0.0, 0.0}, hm = cd{0.0, 0.0};
+    cd f1 = cd{0.0, 1.0}, f2 = cd{0.0, 0.0};
+    double gm = 0.0, g = 0.0, gp = 1.0;
+    double hmm = 0.0, hk1 = 0.0, hk = 0.0, hp = 0.0;   // H_{k-2}, H_{k-1}, H_k, H_{k+1}
+    double t = 1.0;
+#pragma unroll
+    for (int k = 2; k <= K; ++k) {
+        const double gnext = k == 2 ? 0.0 : fma(c1, g, c0 * gm);
+        const double hnext = k <= 2 ? 0.0 : (k == 3 ? 1.0 : fma(c1, hk, fma(c0, hk1, g)));   // H_{k+1}
+        gm = g;
+        g = gp;
+        gp = gnext;
+        hmm = hk1;
+        hk1 = hk;
+        hk = hp;
+        hp = hnext;
+        t /= (double)k;
+        acc_ik(f2, k, t, g);
+        if (k >= 3) {
+            acc_ik(s0, k, t, gm);
+            acc_ik(f1, k, t, gp);
+            acc_ik(h2, k, t, hp);    // sum i^k/k! H_{k+1}
+        }
+        if (k >= 4) acc_ik(h1, k, t, hk);
+        if (k >= 5) acc_ik(h0, k, t, hk1);
+        if (k >= 6) acc_ik(hm, k, t, hmm);
+    }
+    d.f1 = f1;
+    d.f2 = f2;
+    d.b10 = c0 * h0;
+    d.b11 = h2;
+    d.b12 = h1;
+    d.b20 = cd{fma(c0, hm.re, s0.re), fma(c0, hm.im, s0.im)};
+    d.b21 = h1;
+    d.b22 = h0;
+}
+__device__ __forceinline__ void exp_coeffs(double c0, double c1, cd& f0, cd& f1, cd& f2)
+{
+    if (c1 <= EXP_SERIES_SMALL) {
+        exp_series<EXP_TERMS_SMALL>(c0, c1, f0, f1, f2);
+    } else if (c1 <= EXP_SERIES_C1) {
+        exp_series<EXP_TERMS>(c0, c1, f0, f1, f2);
+    } else {
+        ExpC e;
+        exp_constants_c(c0, c1, e);
+        f0 = e.denom * e.h0;
+        f1 = e.denom * e.h1;
+        f2 = e.denom * e.h2;
+    }
 }
 
 // exp(iQ)
 __device__ __forceinline__ M3 su3_exp(const M3& Q)
 {
     M3 Q2 = mul(Q, Q);
-    const double c1 = 0.5 * (Q2.m[0].re + Q2.m[4].re + Q2.m[8].re);
-    if (c1 <= EXP_SERIES_C1) {
-        cd f0, f1, f2;
-        exp_series_coeffs((1.0 / 3.0) * retr_mul(Q, Q2), c1, f0, f1, f2);
-        M3 r;
+    cd f0, f1, f2;
+    exp_coeffs((1.0 / 3.0) * retr_mul(Q, Q2), 0.5 * (Q2.m[0].re + Q2.m[4].re + Q2.m[8].re), f0, f1, f2);
+    M3 r;
 #pragma unroll
-        for (int i = 0; i < 9; ++i) r.m[i] = f1 * Q.m[i] + f2 * Q2.m[i];
-        r.m[0] += f0;
-        r.m[4] += f0;
-        r.m[8] += f0;
-        return r;
-    }
-    ExpC e;
-    exp_constants(Q, Q2, e);
-    return exp_from(e, Q, Q2);
+    for (int i = 0; i < 9; ++i) r.m[i] = f1 * Q.m[i] + f2 * Q2.m[i];
+    r.m[0] += f0;
+    r.m[4] += f0;
+    r.m[8] += f0;
+    return r;
 }
 
 // exp(c * A) for traceless anti-hermitian A: exp(i * (-i c A))
@@ -815,47 +874,6 @@ __device__ __forceinline__ void st_alg8(double2* __restrict__ Z, const Geom& g, 
     p[(size_t)3 * slot_stride(g)] = make_double2(z.a12.re, z.a12.im);
 }
 
-// exp(c Z) for Z anti-hermitian traceless in the 8-real form (the flow's Z):
-// exp(cZ) = exp(iQ) with Q = -i c Z hermitian traceless.  Q^2 is built from its six
-// independent entries and c0 = det Q, c1 = tr(Q^2)/2 directly from Q's entries.
-__device__ __forceinline__ M3 exp_alg8(const Alg8& z, double c)
-{
-    const double q0 = c * z.d0, q1 = c * z.d1, q2 = -(q0 + q1);
-    const cd q01 = cd{c * z.a01.im, -c * z.a01.re}, q02 = cd{c * z.a02.im, -c * z.a02.re},
-             q12 = cd{c * z.a12.im, -c * z.a12.re};
-    const double n01 = q01.re * q01.re + q01.im * q01.im, n02 = q02.re * q02.re + q02.im * q02.im,
-                 n12 = q12.re * q12.re + q12.im * q12.im;
-    // Q^2: diagonal and upper triangle
-    const double s00 = fma(q0, q0, n01 + n02), s11 = fma(q1, q1, n01 + n12), s22 = fma(q2, q2, n02 + n12);
-    const cd s01 = (q0 + q1) * q01 + mul_c(q02, q12);   // q02 conj(q12)
-    const cd s02 = (q0 + q2) * q02 + q01 * q12;
-    const cd s12 = (q1 + q2) * q12 + cmul(q01, q02);    // conj(q01) q02
-    const double c1 = 0.5 * (s00 + s11 + s22);
-    const cd t = q01 * q12;
-    const double c0s = q0 * q1 * q2 - q0 * n12 - q1 * n02 - q2 * n01 + 2.0 * (t.re * q02.re + t.im * q02.im);
-    cd f0, f1, f2;
-    if (c1 <= EXP_SERIES_C1) {
-        exp_series_coeffs(c0s, c1, f0, f1, f2);
-    } else {
-        ExpC e;
-        exp_constants_c(c0s, c1, e);
-        f0 = e.denom * e.h0;
-        f1 = e.denom * e.h1;
-        f2 = e.denom * e.h2;
-    }
-    M3 r;
-    r.m[0] = f0 + q0 * f1 + s00 * f2;
-    r.m[4] = f0 + q1 * f1 + s11 * f2;
-    r.m[8] = f0 + q2 * f1 + s22 * f2;
-    r.m[1] = f1 * q01 + f2 * s01;
-    r.m[2] = f1 * q02 + f2 * s02;
-    r.m[5] = f1 * q12 + f2 * s12;
-    r.m[3] = f1 * conj(q01) + f2 * conj(s01);
-    r.m[6] = f1 * conj(q02) + f2 * conj(s02);
-    r.m[7] = f1 * conj(q12) + f2 * conj(s12);
-    return r;
-}
-
 // Streaming (non-temporal) accesses for data touched once per launch, so that it
 // does not displace the L2-resident neighbourhood of the link reads.
 typedef double lt_d2v __attribute__((ext_vector_type(2)));
@@ -890,22 +908,6 @@ __device__ __forceinline__ void st_alg8_stream(double2* __restrict__ Z, const Ge
 // Lambda) in 8 reals, slots as above:
 //   c: 0 = (Re q00, Re q11), 1 = q01, 2 = q02, 3 = q12;
 // Im q_ii = 0, q_22 = -(q_00 + q_11) and q_ji = conj(q_ij) are implied.
-__device__ __forceinline__ M3 ld_her8(const double2* __restrict__ Z, const Geom& g, int s, int mu, int par)
-{
-    const double2* p = Z + slot_base(g, mu * 2 + par, 4, cbi(g, s));
-    const double2 v0 = p[0], v1 = p[slot_stride(g)], v2 = p[(size_t)2 * slot_stride(g)], v3 = p[(size_t)3 * slot_stride(g)];
-    M3 r;
-    r.m[0] = cd{v0.x, 0.0};
-    r.m[4] = cd{v0.y, 0.0};
-    r.m[8] = cd{-(v0.x + v0.y), 0.0};
-    r.m[1] = cd{v1.x, v1.y};
-    r.m[2] = cd{v2.x, v2.y};
-    r.m[5] = cd{v3.x, v3.y};
-    r.m[3] = cd{v1.x, -v1.y};
-    r.m[6] = cd{v2.x, -v2.y};
-    r.m[7] = cd{v3.x, -v3.y};
-    return r;
-}
 __device__ __forceinline__ void st_her8(double2* __restrict__ Z, const Geom& g, int s, int mu, int par, const M3& q)
 {
     double2* p = Z + slot_base(g, mu * 2 + par, 4, cbi(g, s));
@@ -914,27 +916,58 @@ __device__ __forceinline__ void st_her8(double2* __restrict__ Z, const Geom& g, 
     p[(size_t)2 * slot_stride(g)] = make_double2(q.m[2].re, q.m[2].im);
     p[(size_t)3 * slot_stride(g)] = make_double2(q.m[5].re, q.m[5].im);
 }
-// the matrix that st_her8 followed by ld_her8 reproduces
-__device__ __forceinline__ M3 her8_round(const M3& q)
-{
-    M3 r;
-    r.m[0] = cd{q.m[0].re, 0.0};
-    r.m[4] = cd{q.m[4].re, 0.0};
-    r.m[8] = cd{-(q.m[0].re + q.m[4].re), 0.0};
-    r.m[1] = q.m[1];
-    r.m[2] = q.m[2];
-    r.m[5] = q.m[5];
-    r.m[3] = conj(q.m[1]);
-    r.m[6] = conj(q.m[2]);
-    r.m[7] = conj(q.m[5]);
-    return r;
-}
 // Hermitian or anti-hermitian 3x3 matrices in 9 reals: the diagonal (d, or i d where AH) and
 // the upper triangle; the lower triangle is conj (-conj where AH) of the upper one.
 struct Tri {
     double d0, d1, d2;
     cd r01, r02, r12;
 };
+// Q^2 of a hermitian Q from its six independent entries
+__device__ __forceinline__ Tri her_square(const Tri& q)
+{
+    const double n01 = q.r01.re * q.r01.re + q.r01.im * q.r01.im, n02 = q.r02.re * q.r02.re + q.r02.im * q.r02.im,
+                 n12 = q.r12.re * q.r12.re + q.r12.im * q.r12.im;
+    return Tri{fma(q.d0, q.d0, n01 + n02),
+               fma(q.d1, q.d1, n01 + n12),
+               fma(q.d2, q.d2, n02 + n12),
+               (q.d0 + q.d1) * q.r01 + mul_c(q.r02, q.r12),
+               (q.d0 + q.d2) * q.r02 + q.r01 * q.r12,
+               (q.d1 + q.d2) * q.r12 + cmul(q.r01, q.r02)};
+}
+__device__ __forceinline__ double her_det(const Tri& q)
+{
+    const cd t = q.r01 * q.r12;
+    const double n01 = q.r01.re * q.r01.re + q.r01.im * q.r01.im, n02 = q.r02.re * q.r02.re + q.r02.im * q.r02.im,
+                 n12 = q.r12.re * q.r12.re + q.r12.im * q.r12.im;
+    return q.d0 * q.d1 * q.d2 - q.d0 * n12 - q.d1 * n02 - q.d2 * n01 + 2.0 * (t.re * q.r02.re + t.im * q.r02.im);
+}
+// exp(iQ) for Q hermitian traceless: Q^2 from its six independent entries, c0 = det Q and
+// c1 = tr(Q^2)/2 from Q's entries
+__device__ __forceinline__ M3 exp_her(const Tri& q)
+{
+    const Tri s = her_square(q);
+    cd f0, f1, f2;
+    exp_coeffs(her_det(q), 0.5 * (s.d0 + s.d1 + s.d2), f0, f1, f2);
+    M3 r;
+    r.m[0] = f0 + q.d0 * f1 + s.d0 * f2;
+    r.m[4] = f0 + q.d1 * f1 + s.d1 * f2;
+    r.m[8] = f0 + q.d2 * f1 + s.d2 * f2;
+    r.m[1] = f1 * q.r01 + f2 * s.r01;
+    r.m[2] = f1 * q.r02 + f2 * s.r02;
+    r.m[5] = f1 * q.r12 + f2 * s.r12;
+    r.m[3] = f1 * conj(q.r01) + f2 * conj(s.r01);
+    r.m[6] = f1 * conj(q.r02) + f2 * conj(s.r02);
+    r.m[7] = f1 * conj(q.r12) + f2 * conj(s.r12);
+    return r;
+}
+// exp(c Z) for Z anti-hermitian traceless in the 8-real form (the flow's Z): exp(iQ) with
+// Q = -i c Z hermitian traceless
+__device__ __forceinline__ M3 exp_alg8(const Alg8& z, double c)
+{
+    const double q0 = c * z.d0, q1 = c * z.d1;
+    return exp_her(Tri{q0, q1, -(q0 + q1), cd{c * z.a01.im, -c * z.a01.re}, cd{c * z.a02.im, -c * z.a02.re},
+                       cd{c * z.a12.im, -c * z.a12.re}});
+}
 __device__ __forceinline__ Tri ld_her8_tri(const double2* __restrict__ Z, const Geom& g, int s, int mu, int par)
 {
     const double2* p = Z + slot_base(g, mu * 2 + par, 4, cbi(g, s));
@@ -1393,10 +1426,9 @@ __device__ __forceinline__ M3 clover_plane(const double2* __restrict__ U, const 
 }
 
 
-// Derivative constants of the Cayley-Hamilton exponential (Morningstar-Peardon
-// r_ij, b_ij, B_1, B_2 with the sign-flip conjugation rules); returns B1, B2 and
-// f1, f2 for the stout-force Lambda.
-__device__ __forceinline__ void exp_deriv(const ExpC& e, const M3& Q, const M3& Q2, M3& B1, M3& B2, cd& f1, cd& f2)
+// Derivative constants of the Cayley-Hamilton exponential (Morningstar-Peardon r_ij, b_ij
+// with the sign-flip conjugation rules) from the closed form
+__device__ __forceinline__ void exp_deriv_closed(const ExpC& e, ExpDeriv& out)
 {
     const double u = e.u, u2 = e.u2, w2 = e.w2;
     const double xi0 = e.xi0, xi1 = xi1_of(e.w), cw = e.cosw;
@@ -1404,8 +1436,7 @@ __device__ __forceinline__ void exp_deriv(const ExpC& e, const M3& Q, const M3& 
     const cd ix = cd{0.0, xi0};
     const cd I = cd{0.0, 1.0};
     const cd f0 = e.denom * e.h0;
-    f1 = e.denom * e.h1;
-    f2 = e.denom * e.h2;
+    const cd f1 = e.denom * e.h1, f2 = e.denom * e.h2;
     const cd r10 = 2.0 * (cd{u, u2 - w2} * e2)
                  + 2.0 * (em * ((4.0 * u) * cd{2.0, -u} * cw + ix * cd{9.0 * u2 + w2, -u * (3.0 * u2 + w2)}));
     const cd r11 = 2.0 * (cd{1.0, 2.0 * u} * e2) + em * (-2.0 * cd{1.0, -u} * cw + ix * cd{6.0 * u, w2 - 3.0 * u2});
@@ -1437,17 +1468,18 @@ __device__ __forceinline__ void exp_deriv(const ExpC& e, const M3& Q, const M3& 
             b22 = bd * (r12 - (3.0 * u) * r22 - (24.0 * u) * f2);
         }
     }
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-        B1.m[k] = b11 * Q.m[k] + b12 * Q2.m[k];
-        B2.m[k] = b21 * Q.m[k] + b22 * Q2.m[k];
+    out = ExpDeriv{f1, f2, b10, b11, b12, b20, b21, b22};
+}
+// f1, f2 and the b_ij of exp(iQ) from c0 = det Q, c1 = tr(Q^2)/2
+__device__ __forceinline__ void exp_deriv(double c0, double c1, ExpDeriv& d)
+{
+    if (c1 <= EXP_SERIES_C1) {
+        exp_series_deriv<EXP_TERMS>(c0, c1, d);
+    } else {
+        ExpC e;
+        exp_constants_c(c0, c1, e);
+        exp_deriv_closed(e, d);
     }
-    B1.m[0] += b10;
-    B1.m[4] += b10;
-    B1.m[8] += b10;
-    B2.m[0] += b20;
-    B2.m[4] += b20;
-    B2.m[8] += b20;
 }
 
 }  // namespace lt
