@@ -29,6 +29,9 @@ Geom make_geom(int nt, int nx, int ny, int nz)
     g.st[0] = nx * ny * nz;
     g.V = nt * nx * ny * nz;
     g.Vh = g.V / 2;
+    g.dx = make_div(nx);
+    g.dy = make_div(ny);
+    g.dz = make_div(nz);
     return g;
 }
 
@@ -45,6 +48,7 @@ bool make_linkmap(const Geom& g, int tt, int tx, int ty, int tz, LinkMap& m)
         m.N[1] = m.N[2] = m.N[3] = 1;
         m.tc = m.yc = m.ycs = 1;
         m.xr = LT_XCD_REMAP;
+        finish_map(m);
         return true;
     }
     const int ext[4] = {g.L[0], g.L[1], g.L[2], g.L[3] / 2};
@@ -75,6 +79,7 @@ bool make_linkmap(const Geom& g, int tt, int tx, int ty, int tz, LinkMap& m)
     // the colour sweeps walk all y tiles of an x step in one chunk
     m.ycs = m.N[2];
     m.xr = LT_XCD_REMAP;
+    finish_map(m);
     return true;
 }
 

@@ -53,12 +53,12 @@ __global__ void LT_LINK_KERNEL hb_cb4_graph_kernel(double2* __restrict__ U, Geom
 template <bool HEATBATH, int KIND>
 __global__ void __launch_bounds__(SPLIT_BS) __attribute__((amdgpu_waves_per_eu(3)))
 split_cb4_kernel(double2* __restrict__ U, Geom g, int mu, int colour, double prefactor, uint64_t seed, uint64_t counter,
-                 const uint64_t* __restrict__ state, int k, double c_plaq, double c_rect, int tc)
+                 const uint64_t* __restrict__ state, int k, double c_plaq, double c_rect, SplitMap map)
 {
     __shared__ SplitShared<HEATBATH> sh;
     if (HEATBATH && state) counter = state[0] + (uint64_t)k;
     int c[4], s = 0;
-    const int i = split_index((g.V / g.L[0]) >> 2, xcd_block_dir(blockIdx.x, gridDim.x, colour & 1), tc);
+    const int i = split_index(map, xcd_block_dir(blockIdx.x, gridDim.x, colour & 1));
     const bool on = i >= 0 && cb4_site(g, mu, colour, i, c, s);
     update_links_split<HEATBATH, KIND>(U, g, mu, on, s, c, prefactor, seed, counter, c_plaq, c_rect, sh);
 }
@@ -115,9 +115,9 @@ template <bool HEATBATH, int KIND>
 void split_launch(lt_field u, const char* name, int mu, int colour, double prefactor, uint64_t counter,
                   const uint64_t* state, int k, double c_plaq, double c_rect)
 {
-    const Geom& g = u->g;
-    launch(u->ctx, name, split_cb4_kernel<HEATBATH, KIND>, dim3((unsigned)g.L[0] * nblocks(g.V / g.L[0] / 4, SPLIT_LINKS)),
-           dim3(SPLIT_BS), 0, u->d, g, mu, colour, prefactor, u->seed, counter, state, k, c_plaq, c_rect, split_tc(g));
+    const SplitMap m = split_map(u->g, 4);
+    launch(u->ctx, name, split_cb4_kernel<HEATBATH, KIND>, dim3(split_blocks(u->g, m)), dim3(SPLIT_BS), 0, u->d, u->g, mu,
+           colour, prefactor, u->seed, counter, state, k, c_plaq, c_rect, m);
 }
 
 }  // namespace

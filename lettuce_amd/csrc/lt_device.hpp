@@ -705,6 +705,41 @@ __device__ __forceinline__ void gauss2(double u0, double u1, double& g0, double&
     g1 = r * s;
 }
 
+// Division of 0 <= n < 2^31 by d as one high product and a shift: with sh = ceil(log2 d) - 1
+// and m = ceil(2^(32 + sh) / d), m d - 2^(32 + sh) < d <= 2^(sh + 1), so n m / 2^(32 + sh)
+// exceeds n / d by less than 1/d and the quotient is exact.  A division by a kernel argument
+// is about twenty VALU instructions otherwise, also where the operands are uniform; the maps
+// from a thread to its site take eight to ten of them (OR + HB updates of a 16^4 lattice 462 ->
+// 448 us, four colours at 20^4 2025 -> 1968 us, the heatbath launch at 32^4 128 -> 124 us).
+struct Div {
+    uint32_t m;
+    int sh;
+    int d;
+};
+inline Div make_div(int d)
+{
+    Div v{0u, 0, d};
+    if (d > 1) {
+        int bits = 0;   // ceil(log2 d)
+        while ((1ll << bits) < d) ++bits;
+        v.sh = bits - 1;
+        v.m = (uint32_t)(((1ull << (32 + v.sh)) + (uint64_t)d - 1) / (uint64_t)d);
+    }
+    return v;
+}
+__host__ __device__ __forceinline__ int div_by(int n, const Div& v)
+{
+    const int q = (int)((uint32_t)(((uint64_t)(uint32_t)n * v.m) >> 32) >> v.sh);
+    return v.d == 1 ? n : q;
+}
+// n <- n / d, returns n % d
+__host__ __device__ __forceinline__ int mod_div(int& n, const Div& v)
+{
+    const int q = div_by(n, v), r = n - q * v.d;
+    n = q;
+    return r;
+}
+
 // ---------------------------------------------------------------------------
 // Lattice geometry.  Sites are lexicographic s = ((t*Nx+x)*Ny+y)*Nz+z; the parity
 // of a site is (t+x+y+z)&1 and, because Nz is even, its checkerboard index is s>>1.
@@ -716,6 +751,7 @@ struct Geom {
     int L[4];       // Nt, Nx, Ny, Nz
     int st[4];      // lexicographic strides of t, x, y, z
     int V, Vh;
+    Div dx, dy, dz; // division by Nx, Ny, Nz
 };
 
 // Storage slot of site s in its parity array.  Plain order: cb = s>>1.  Split order
@@ -765,12 +801,10 @@ __device__ __forceinline__ int pick4(const int v[4], int i)
 
 __device__ __forceinline__ void coords_of(const Geom& g, int s, int c[4])
 {
-    c[3] = s % g.L[3];
-    int r = s / g.L[3];
-    c[2] = r % g.L[2];
-    r /= g.L[2];
-    c[1] = r % g.L[1];
-    c[0] = r / g.L[1];
+    c[3] = mod_div(s, g.dz);
+    c[2] = mod_div(s, g.dy);
+    c[1] = mod_div(s, g.dx);
+    c[0] = s;
 }
 // site index one step along +mu / -mu given the coordinate of that direction
 __device__ __forceinline__ int up(const Geom& g, int s, int cmu, int mu)
@@ -1145,6 +1179,31 @@ struct LinkMap {
     int lin;      // linear map: block b covers checkerboard sites [b * nthreads, (b + 1) * nthreads)
     int ycs;      // y tiles per chunk of the colour sweeps
     int xr;       // spread the block index over the XCDs (xcd_block)
+    // divisions of map_site_b, from the numbers above (finish_map)
+    Div dtx, dty, dtz, dtc, dnz, dyc, dnx, dny;
+};
+// to be called after any change of T, N, tc or yc
+inline void finish_map(LinkMap& m)
+{
+    m.dtx = make_div(m.T[1]);
+    m.dty = make_div(m.T[2]);
+    m.dtz = make_div(m.T[3]);
+    m.dtc = make_div(m.tc);
+    m.dnz = make_div(m.N[3]);
+    m.dyc = make_div(m.yc);
+    m.dnx = make_div(m.N[1]);
+    m.dny = make_div(m.N[2] / m.yc);
+}
+
+// Blocks of the split colour launches (64 links each): every timeslice of the class, nt
+// links, is covered by its own blocks, the last one partly; the tc timeslices of a chunk are
+// walked fastest, so that the t-neighbours of a block run in the same XCD at about the same
+// time (24^4, Luescher-Weisz staple: 97 -> 85 us per overrelaxation launch with tc = 3; 20^4,
+// four colours, Wilson staple: 25 -> 20 us with tc = 2).
+constexpr int SPLIT_LINKS = 64;
+struct SplitMap {
+    int nt;
+    Div dtc, dper;   // by tc, and by the blocks of a chunk
 };
 
 // Block index of a link kernel in its map's order: spread over the XCDs when m.xr is
@@ -1166,29 +1225,22 @@ __device__ __forceinline__ bool map_site_b(const Geom& g, const LinkMap& m, int 
         s = site_of_cb(g, cb, par, c);
         return true;
     }
-    const int bt_lo = b % m.tc;
-    b /= m.tc;
-    int bz = b % m.N[3];
-    b /= m.N[3];
-    const int by_lo = b % m.yc;
-    b /= m.yc;
-    int bx = b % m.N[1];
-    b /= m.N[1];
-    const int ny_hi = m.N[2] / m.yc;
-    int by = (b % ny_hi) * m.yc + by_lo;
-    int bt = (b / ny_hi) * m.tc + bt_lo;
+    const int bt_lo = mod_div(b, m.dtc);
+    const int bz = mod_div(b, m.dnz);
+    const int by_lo = mod_div(b, m.dyc);
+    const int bx = mod_div(b, m.dnx);
+    const int by = mod_div(b, m.dny) * m.yc + by_lo;
+    const int bt = b * m.tc + bt_lo;
     if (bt >= m.N[0] || tid >= m.nthreads) return false;
-    int dz = tid % m.T[3];
-    tid /= m.T[3];
-    int dy = tid % m.T[2];
-    tid /= m.T[2];
-    int dx = tid % m.T[1];
-    int dt = tid / m.T[1];
+    const int dz = mod_div(tid, m.dtz);
+    const int dy = mod_div(tid, m.dty);
+    const int dx = mod_div(tid, m.dtx);
+    const int dt = tid;
     c[0] = bt * m.T[0] + dt;
     c[1] = bx * m.T[1] + dx;
     c[2] = by * m.T[2] + dy;
-    int zc = bz * m.T[3] + dz;
-    int flip = (c[0] + c[1] + c[2] + par) & 1;
+    const int zc = bz * m.T[3] + dz;
+    const int flip = (c[0] + c[1] + c[2] + par) & 1;
     c[3] = 2 * zc + flip;
     s = ((c[0] * g.L[1] + c[1]) * g.L[2] + c[2]) * g.L[3] + c[3];
     return true;

@@ -197,15 +197,20 @@ void launch(lt_ctx ctx, const char* name, Kernel kernel, dim3 grid, dim3 block, 
 }
 
 inline unsigned nblocks(long long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
-// timeslices per chunk of a split colour launch (split_index): the largest divisor of Nt that
-// leaves each of the eight XCDs a chunk of its own
-inline int split_tc(const Geom& g)
+// map of a split colour launch over 1/colours of the sites; tc is the largest divisor of Nt
+// that leaves each of the eight XCDs a chunk of its own
+inline SplitMap split_map(const Geom& g, int colours)
 {
     int tc = 1;
     for (int d = 2; d <= (g.L[0] + 7) / 8; ++d)
         if (g.L[0] % d == 0) tc = d;
-    return tc;
+    SplitMap m;
+    m.nt = g.V / g.L[0] / colours;
+    m.dtc = make_div(tc);
+    m.dper = make_div(tc * (int)nblocks(m.nt, SPLIT_LINKS));
+    return m;
 }
+inline unsigned split_blocks(const Geom& g, const SplitMap& m) { return (unsigned)g.L[0] * nblocks(m.nt, SPLIT_LINKS); }
 // grid size of a tiled link launch; refuses maps the kernels were not compiled for
 inline unsigned map_blocks(const LinkMap& m)
 {

@@ -136,23 +136,19 @@ __device__ __forceinline__ bool cb4_site(const Geom& g, int mu, int k, int i, in
 {
     if (i >= (g.V >> 2)) return false;
     if (mu != 3) {
-        const int per_row = g.L[3] >> 2;
-        int row = i / per_row;
-        const int j = i - row * per_row;
-        c[2] = row % g.L[2];
-        row /= g.L[2];
-        c[1] = row % g.L[1];
-        c[0] = row / g.L[1];
-        c[3] = ((k - c[0] - c[1] - c[2] - c[mu]) & 3) + 4 * j;
+        int row = div_by(4 * i, g.dz);
+        const int j = i - row * (g.L[3] >> 2);
+        c[2] = mod_div(row, g.dy);
+        c[1] = mod_div(row, g.dx);
+        c[0] = row;
+        c[3] = ((k - c[0] - c[1] - c[2] - pick4(c, mu)) & 3) + 4 * j;
     } else {
-        const int per_row = g.L[3] >> 1;
-        int row = i / per_row;
-        const int j = i - row * per_row;
-        const int ny2 = g.L[2] >> 1;
-        const int yh = row % ny2;
-        row /= ny2;
-        c[1] = row % g.L[1];
-        c[0] = row / g.L[1];
+        const int row = div_by(2 * i, g.dz);
+        const int j = i - row * (g.L[3] >> 1);
+        int plane = div_by(2 * row, g.dy);
+        const int yh = row - plane * (g.L[2] >> 1);
+        c[1] = mod_div(plane, g.dx);
+        c[0] = plane;
         c[2] = 2 * yh + ((k - c[0] - c[1]) & 1);
         c[3] = (((k - c[0] - c[1] - c[2]) & 3) >> 1) + 2 * j;
     }
@@ -301,7 +297,7 @@ __device__ __forceinline__ M3 staple_action(const double2* __restrict__ U, const
 // The action enters through the staple only (heatbath.hpp:110-129, overrelaxation.hpp:91-116):
 // SPLIT_WILSON, SPLIT_SCALED (c_plaq times the plaquette staple), SPLIT_RECT.
 enum SplitKind { SPLIT_WILSON = 0, SPLIT_SCALED = 1, SPLIT_RECT = 2 };
-constexpr int SPLIT_WAVES = 6, SPLIT_LINKS = 64, SPLIT_BS = SPLIT_WAVES * SPLIT_LINKS;
+constexpr int SPLIT_WAVES = 6, SPLIT_BS = SPLIT_WAVES * SPLIT_LINKS;
 template <bool HEATBATH>
 struct SplitShared {
     double2 part[27 * SPLIT_LINKS];
@@ -414,17 +410,15 @@ __device__ __forceinline__ void update_links_split(double2* __restrict__ U, cons
 }
 
 // Index (in the class's order, t slowest) of the link of this lane in block b of a split
-// launch with nt links per timeslice; -1 for none.  Every timeslice is covered by its own
-// blocks of 64 links (the last one partly); the tc timeslices of a chunk are walked fastest,
-// so that the t-neighbours of a block run in the same XCD at about the same time (24^4,
-// Luescher-Weisz staple: 97 -> 85 us per overrelaxation launch with tc = 3; 20^4, four
-// colours, Wilson staple: 25 -> 20 us with tc = 2).
-__device__ __forceinline__ int split_index(int nt, int b, int tc)
+// launch; -1 for none.
+__device__ __forceinline__ int split_index(const SplitMap& m, int b)
 {
-    const int nbt = (nt + SPLIT_LINKS - 1) / SPLIT_LINKS, per = tc * nbt;
-    const int ch = b / per, q = b - ch * per;
-    const int r = (q / tc) * SPLIT_LINKS + (threadIdx.x & (SPLIT_LINKS - 1));
-    return r < nt ? (ch * tc + q % tc) * nt + r : -1;
+    int q = b;
+    const int ch = div_by(b, m.dper);
+    q -= ch * m.dper.d;
+    const int t = mod_div(q, m.dtc);
+    const int r = q * SPLIT_LINKS + (threadIdx.x & (SPLIT_LINKS - 1));
+    return r < m.nt ? (ch * m.dtc.d + t) * m.nt + r : -1;
 }
 
 }  // namespace lt

@@ -90,6 +90,7 @@ std::vector<LinkMap> order_candidates(const LinkMap& base, bool sweeps)
                 m.xr = xr;
                 m.tc = tc;
                 (sweeps ? m.ycs : m.yc) = yc;
+                finish_map(m);
                 out.push_back(m);
             }
     return out;
@@ -170,6 +171,7 @@ bool cached_tile(const char* path, const std::string& key, const Geom& g, LinkMa
         o.ycs = (int)v[7];
         o.xr = (int)v[8];
         if (o.tc < 1 || o.N[0] % o.tc || o.yc < 1 || o.N[2] % o.yc || o.ycs < 1 || o.N[2] % o.ycs) return false;
+        finish_map(o);
         m = o;
     }
     ms = v[4];

@@ -63,12 +63,12 @@ constexpr int SMALL_VH = LT_SMALL_VH;
 template <bool HEATBATH>
 __global__ void __launch_bounds__(SPLIT_BS) __attribute__((amdgpu_waves_per_eu(3)))
 split_cb2_kernel(double2* __restrict__ U, Geom g, int mu, int par, double prefactor, uint64_t seed, uint64_t counter,
-                 const uint64_t* __restrict__ state, int k, int tc)
+                 const uint64_t* __restrict__ state, int k, SplitMap map)
 {
     __shared__ SplitShared<HEATBATH> sh;
     if (HEATBATH && state) counter = state[0] + (uint64_t)k;
     int c[4] = {0, 0, 0, 0}, s = 0;
-    const int i = split_index((g.V / g.L[0]) >> 1, xcd_block_dir(blockIdx.x, gridDim.x, par), tc);
+    const int i = split_index(map, xcd_block_dir(blockIdx.x, gridDim.x, par));
     if (i >= 0) s = site_of_cb(g, i, par, c);
     update_links_split<HEATBATH, SPLIT_WILSON>(U, g, mu, i >= 0, s, c, prefactor, seed, counter, 1.0, 0.0, sh);
 }
@@ -148,6 +148,7 @@ LinkMap sweep_map(const LinkMap& m)
 {
     LinkMap r = m;
     r.yc = r.ycs;
+    finish_map(r);
     return r;
 }
 
@@ -155,9 +156,9 @@ template <bool HEATBATH>
 void split_cb2(lt_field u, const char* name, int mu, int par, double prefactor, uint64_t counter, const uint64_t* state,
                int k)
 {
-    const Geom& g = u->g;
-    launch(u->ctx, name, split_cb2_kernel<HEATBATH>, dim3((unsigned)g.L[0] * nblocks(g.Vh / g.L[0], SPLIT_LINKS)),
-           dim3(SPLIT_BS), 0, u->d, g, mu, par, prefactor, u->seed, counter, state, k, split_tc(g));
+    const SplitMap m = split_map(u->g, 2);
+    launch(u->ctx, name, split_cb2_kernel<HEATBATH>, dim3(split_blocks(u->g, m)), dim3(SPLIT_BS), 0, u->d, u->g, mu, par,
+           prefactor, u->seed, counter, state, k, m);
 }
 
 // n sweeps; the four-colour ones (split) expect the field in the split order
