@@ -799,7 +799,7 @@ int lt_action_rectangular(lt_field u, double c_plaq, double c_rect, double* acti
     if (!u->su3) return fail(LT_ESTATE, "lt_action_rectangular: the field must hold SU(3) links");
     return guarded([&] {
         use_device(u->ctx);
-        double r[3];
+        double r[2];
         lt::k_rect_sums(u, r);
         const double V = (double)u->g.V;
         *action_normalized = (c_plaq * (6.0 * V - r[0] / 3.0) + c_rect * (12.0 * V - r[1] / 3.0)) / (6.0 * V);
@@ -813,9 +813,7 @@ int lt_topcharge_plaquette(lt_field u, double* q)
     if (!u->su3) return fail(LT_ESTATE, "lt_topcharge_plaquette: the field must hold SU(3) links");
     return guarded([&] {
         use_device(u->ctx);
-        double r[3];
-        lt::k_rect_sums(u, r);
-        *q = r[2] / (16.0 * M_PI * M_PI);
+        *q = lt::k_plaq_charge(u) / (16.0 * M_PI * M_PI);
         return LT_OK;
     });
 }

@@ -247,21 +247,25 @@ __device__ __forceinline__ double body_plaq_link(const double2* __restrict__ U, 
     if (mu < 2) v += plaq_plane(U, g, s, c, par, mu, mu + 2);
     return v;
 }
-// block sums of body_plaq_link, part[blockIdx.x]: a butterfly in each wavefront, then the
-// m.nthreads / 64 wavefront sums in wave order
-__device__ __forceinline__ void plaq_link_partials(const double2* __restrict__ U, const Geom& g, const LinkMap& m,
-                                                   double* part)
+// sum of v over the n lanes of a link-map block into *out: a butterfly in each wavefront, then
+// the n / 64 wavefront sums in wave order (sh: LT_LINK_BS / 64 doubles)
+__device__ __forceinline__ void link_block_sum(double v, int n, double* sh, double* out)
 {
-    __shared__ double sh[LT_LINK_BS / 64];
-    double v = body_plaq_link(U, g, m, link_block(m, blockIdx.x, gridDim.x));
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < (m.nthreads >> 6); ++w) v += sh[w];
-        part[blockIdx.x] = v;
+        for (int w = 1; w < (n >> 6); ++w) v += sh[w];
+        *out = v;
     }
+}
+// block sums of body_plaq_link, part[blockIdx.x]
+__device__ __forceinline__ void plaq_link_partials(const double2* __restrict__ U, const Geom& g, const LinkMap& m,
+                                                   double* part)
+{
+    __shared__ double sh[LT_LINK_BS / 64];
+    link_block_sum(body_plaq_link(U, g, m, link_block(m, blockIdx.x, gridDim.x)), m.nthreads, sh, part + blockIdx.x);
 }
 
 // Running sums in LDS (entries e * n of a per-lane slot, e < 9): a sum waits there between the

@@ -650,6 +650,22 @@ __device__ __forceinline__ void block_sum_to(double v, double* out)
     if (threadIdx.x == 0) *out = a[0];
 }
 
+// the sum of part[stride i], i < n, over one block of BS lanes, in a fixed order: lane i keeps
+// eight running sums of the entries i + BS u (u < 8) of each group of 8 BS entries (eight
+// loads in flight instead of one), the rest into the first, then a fixed pairing; the lanes
+// are left to block_reduce
+template <int BS>
+__device__ __forceinline__ double partials_sum(const double* __restrict__ part, int n, int stride = 1)
+{
+    double a[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    int i = threadIdx.x;
+    for (; i + 7 * BS < n; i += 8 * BS)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) a[u] += part[(size_t)stride * (i + u * BS)];
+    for (; i < n; i += BS) a[0] += part[(size_t)stride * i];
+    return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+}
+
 // ---------------------------------------------------------------------------
 // Philox4x32-10 counter RNG (Salmon et al., SC'11).  Counter layout:
 //   key = seed, ctr = {site, stream<<24 | k<<4 | sub<<2 | mu, counter_lo, counter_hi}
@@ -1280,6 +1296,15 @@ __device__ __forceinline__ int site_of_cb(const Geom& g, int cb, int par, int c[
     return s + flip;
 }
 
+// Sites of the site kernels: 64 consecutive indices i are 32 checkerboard positions, first
+// their parity-0 sites, then their parity-1 sites, so that each half wavefront reads 512
+// consecutive bytes per component.  Walking sites in lexicographic order instead alternates
+// the parity arrays from lane to lane, and the L1 then takes twice the accesses per load (32
+// instead of 16; four times where the direction alternates too).  half_cb may pass the last
+// position where their number is not a multiple of 32.
+__device__ __forceinline__ int half_cb(int i) { return ((i >> 6) << 5) | (i & 31); }
+__device__ __forceinline__ int half_par(int i) { return (i >> 5) & 1; }
+
 // Staple of link (s, mu): sum over nu != mu (ascending) of
 //   U_nu(x) U_mu(x+nu) U_nu(x+mu)^+ + U_nu(x-nu)^+ U_mu(x-nu) U_nu(x-nu+mu)
 // Every partial product of links is in SU(3), so only its rows 0 and 1 are
@@ -1477,6 +1502,119 @@ __device__ __forceinline__ M3 clover_plane(const double2* __restrict__ U, const 
     return C;
 }
 
+// r += leaf - leaf^+ for an SU(3) leaf given by rows 0 and 1 (row 2 = conj(row0 x row1))
+__device__ __forceinline__ void acc_leaf(Tri& r, M3& t)
+{
+    third_row(t);
+    const cd* m = t.m;
+    r.d0 += m[0].im + m[0].im;
+    r.d1 += m[4].im + m[4].im;
+    r.d2 += m[8].im + m[8].im;
+    r.r01 += m[1] - conj(m[3]);
+    r.r02 += m[2] - conj(m[6]);
+    r.r12 += m[5] - conj(m[7]);
+}
+// R = C - C^+ (anti-hermitian, 9 reals) of the clover term C of plane (mu, nu) at site s: the
+// four leaves in the orientation of the reference's CalculateClover<1,1>; retr: Re tr of leaf
+// I, the plaquette.  Every leaf is a product of four links, an SU(3) matrix of which rows 0
+// and 1 are multiplied out; only the nine reals of R are summed.  Each link is loaded two
+// products ahead of the one that takes it (U_mu(x) a second time for leaf IV); the scheduling
+// barriers keep the compiler from hoisting all loads (which spills).
+__device__ __forceinline__ Tri clover_ah(const double2* __restrict__ U, const Geom& g, int s, const int c[4], int par,
+                                         int mu, int nu, double& retr)
+{
+    const int q = par ^ 1, cm = pick4(c, mu), cn = pick4(c, nu);
+    const int smu = up(g, s, cm, mu), snu = up(g, s, cn, nu), smd = dn(g, s, cm, mu), snd = dn(g, s, cn, nu);
+    const int smd_nu = smd + (snu - s), smd_nd = smd + (snd - s), smu_nd = smu + (snd - s);
+    Tri r{0.0, 0.0, 0.0, cd{0.0, 0.0}, cd{0.0, 0.0}, cd{0.0, 0.0}};
+    auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+    Raw6 a, b, k;
+    ld_raw(U, g, s, mu, par, k);
+    ld_raw(U, g, smu, nu, q, a);
+    ld_raw(U, g, snu, mu, q, b);
+    fence();
+    // leaf I: U_mu(x) U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+
+    M3 t = mul_r01(rows01(k), su3_of(a));
+    ld_raw(U, g, s, nu, par, k);
+    fence();
+    t = mul_nd_r01(t, su3_of(b));
+    ld_raw(U, g, smd_nu, mu, par, a);
+    fence();
+    t = mul_nd_r01(t, su3_of(k));
+    ld_raw(U, g, smd, nu, q, b);
+    fence();
+    acc_leaf(r, t);
+    retr = t.m[0].re + t.m[4].re + t.m[8].re;
+    // leaf II: U_nu(x) U_mu(x-mu+nu)^+ U_nu(x-mu)^+ U_mu(x-mu)
+    t = mul_nd_r01(rows01(k), su3_of(a));
+    ld_raw(U, g, smd, mu, q, k);
+    fence();
+    t = mul_nd_r01(t, su3_of(b));
+    ld_raw(U, g, smd_nd, nu, par, a);
+    fence();
+    t = mul_r01(t, su3_of(k));
+    ld_raw(U, g, smd_nd, mu, par, b);
+    fence();
+    acc_leaf(r, t);
+    // leaf III: U_mu(x-mu)^+ U_nu(x-mu-nu)^+ U_mu(x-mu-nu) U_nu(x-nu)
+    t = mul_dd_r01(su3_of(k), su3_of(a));
+    ld_raw(U, g, snd, nu, q, k);
+    fence();
+    t = mul_r01(t, su3_of(b));
+    ld_raw(U, g, snd, mu, q, a);
+    fence();
+    t = mul_r01(t, su3_of(k));
+    ld_raw(U, g, smu_nd, nu, par, b);
+    fence();
+    acc_leaf(r, t);
+    // leaf IV: U_nu(x-nu)^+ U_mu(x-nu) U_nu(x+mu-nu) U_mu(x)^+
+    t = mul_dn_r01(su3_of(k), su3_of(a));
+    ld_raw(U, g, s, mu, par, k);
+    fence();
+    t = mul_r01(t, su3_of(b));
+    t = mul_nd_r01(t, su3_of(k));
+    acc_leaf(r, t);
+    return r;
+}
+// Re tr(A B) of two anti-hermitian matrices in 9 reals
+__device__ __forceinline__ double retr_ah(const Tri& a, const Tri& b)
+{
+    double d = a.d0 * b.d0;
+    d = fma(a.d1, b.d1, d);
+    d = fma(a.d2, b.d2, d);
+    double o = a.r01.re * b.r01.re;
+    o = fma(a.r01.im, b.r01.im, o);
+    o = fma(a.r02.re, b.r02.re, o);
+    o = fma(a.r02.im, b.r02.im, o);
+    o = fma(a.r12.re, b.r12.re, o);
+    o = fma(a.r12.im, b.r12.im, o);
+    return -(d + 2.0 * o);
+}
+// directions of plane p in the order 01, 02, 03, 12, 13, 23.  Planes p and 5 - p are pair p
+// (p < 3) of the topological charge tr R01 R23 - tr R02 R13 + tr R03 R12.
+__device__ __forceinline__ int plane_mu(int p) { return p < 3 ? 0 : (p < 5 ? 1 : 2); }
+__device__ __forceinline__ int plane_nu(int p) { return p < 3 ? p + 1 : (p < 5 ? p - 1 : 3); }
+// The two planes of pair p at site s, each handed to take(plane, R, Re tr plaquette); returns
+// the pair's term of the charge.  A loop, so that one plane at a time has the registers.
+template <typename Take>
+__device__ __forceinline__ double clover_pair(const double2* __restrict__ U, const Geom& g, int s, const int c[4], int par,
+                                              int p, Take take)
+{
+    Tri first{};
+    double q = 0.0;
+#pragma unroll 1
+    for (int j = 0; j < 2; ++j) {
+        const int plane = j ? 5 - p : p;
+        double pl;
+        const Tri r = clover_ah(U, g, s, c, par, plane_mu(plane), plane_nu(plane), pl);
+        take(plane, r, pl);
+        if (j)
+            q = retr_ah(first, r);
+        else
+            first = r;
+    }
+    return p == 1 ? -q : q;
+}
 
 // Derivative constants of the Cayley-Hamilton exponential (Morningstar-Peardon r_ij, b_ij
 // with the sign-flip conjugation rules) from the closed form

@@ -334,7 +334,8 @@ void k_topcharge_density(lt_field u, double* host_q);
 void noalloc_setup(int device);
 // lt_observables' sums through the fixed scratch, final values computed on the device
 void k_observables_noalloc(lt_field u, double* host_out);
-void k_rect_sums(lt_field u, double out[3]);
+void k_rect_sums(lt_field u, double out[2]);
+double k_plaq_charge(lt_field u);
 double k_wilson_loop(lt_field u, lt_field chain, int n0, int n1, int reset);
 void k_polyakov_loop(lt_field u, double* re, double* im);
 void k_stout(lt_ctx ctx, const Geom& g, const LinkMap& m, const double2* in, double2* out, double rho);

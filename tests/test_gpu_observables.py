@@ -67,6 +67,23 @@ def test_matches_oracle(la, lto, gpu_ctx, shape):
     assert np.all(np.abs(got - ref) <= 1e-12 * np.maximum(np.abs(ref), 1.0)), (got, ref)
 
 
+# timeslices and lattices whose parity halves are not multiples of 32 sites, or of a block
+@pytest.mark.parametrize("shape", [(2, 2, 2, 4), (2, 2, 4, 4), (4, 2, 6, 10), (6, 10, 6, 14)])
+def test_clover_fields_match_oracle(la, lto, gpu_ctx, shape):
+    """Timeslice sums and the charge per site; 1e-12 as for the other observables."""
+    flush(f"clover fields {shape}")
+    U = lto.stout(lto.haar(shape, 8), shape, 0.1, 1)
+    f = la.GaugeField(gpu_ctx, shape)
+    f.upload(U)
+    for got, ref in ((la.TopChargeCloverDensity(f), lto.topcharge_density(U, shape)),
+                     (la.TopChargeCloverTimeslice(f), lto.topcharge_timeslice(U, shape)),
+                     (la.EnergyDensity.CloverTimeslice(f), lto.energy_clover_timeslice(U, shape))):
+        got, ref = np.asarray(got).ravel(), np.asarray(ref).ravel()
+        assert got.shape == ref.shape
+        assert np.max(np.abs(got - ref)) <= 1e-12 * max(1.0, np.max(np.abs(ref)))
+    f.close()
+
+
 def test_unit_field(la, lto, gpu_ctx):
     flush("observables unit field")
     shape = (4, 4, 6, 8)
