@@ -28,21 +28,15 @@ __global__ void LT_LINK_KERNEL stout_tape_kernel(const double2* __restrict__ Uin
     body_stout_tape<KEEP>(Uin, Uout, T, g, m, link_block(m, blockIdx.x, gridDim.x), rho, keep);
 }
 
-// one thread per (site, plane): the clover term of that plane.  Block b (XCD-remapped)
-// takes plane b % 6 of site chunk b / 6, so the six planes of a chunk run in neighbouring
-// blocks of one XCD and share its L2 instead of streaming the field once per plane.
-__global__ void __launch_bounds__(CBS) clover_store_kernel(const double2* __restrict__ U, double2* __restrict__ C, Geom g)
+// clover planes and charge: block b (XCD-remapped) takes pair b % 3 of site chunk b / 3, so
+// the three pairs of a chunk run in neighbouring blocks of one XCD and share its L2.  Two waves
+// per SIMD hold a plane's registers (200) without spills: 16^4 39 us, at three waves 42; one
+// lane per (site, plane) and a second pass over the planes for the charge took 47 + 10.
+__global__ void __launch_bounds__(CBS) __attribute__((amdgpu_waves_per_eu(2)))
+clover_charge_kernel(const double2* __restrict__ U, double2* __restrict__ C, Geom g, double* part)
 {
     const int b = xcd_block(blockIdx.x, gridDim.x);
-    const int s = (b / 6) * CBS + threadIdx.x;
-    if (s < g.V) body_clover_store(U, C, g, s, b % 6);
-}
-
-// per site charge density, block partial sums
-__global__ void __launch_bounds__(CBS) qdensity_kernel(const double2* __restrict__ C, Geom g, double* part)
-{
-    const int s = blockIdx.x * CBS + threadIdx.x;
-    block_sum_to<CBS>(s < g.V ? body_qdensity_site(C, g, s) : 0.0, part + blockIdx.x);
+    block_sum_to<CBS>(body_clover_pair(U, C, g, (b / 3) * CBS + threadIdx.x, b % 3), part + b);
 }
 
 __global__ void __launch_bounds__(CBS) sum_kernel(const double* part, int n, double* out)
@@ -89,10 +83,9 @@ void k_stout_tape(lt_ctx ctx, const Geom& g, const LinkMap& m, const double2* in
 
 double k_clover_charge(lt_ctx ctx, const Geom& g, const double2* U, double2* C)
 {
-    launch(ctx, "clover_store", clover_store_kernel, dim3(6 * nblocks(g.V, CBS)), dim3(CBS), 0, U, C, g);
-    unsigned nb = nblocks(g.V, CBS);
+    const unsigned nb = 3 * nblocks(g.V, CBS);
     double* part = ctx->scratch_for(nb + 1);
-    launch(ctx, "qdensity", qdensity_kernel, dim3(nb), dim3(CBS), 0, (const double2*)C, g, part);
+    launch(ctx, "clover_store", clover_charge_kernel, dim3(nb), dim3(CBS), 0, U, C, g, part);
     launch(ctx, "qsum", sum_kernel, dim3(1), dim3(CBS), 0, (const double*)part, (int)nb, part + nb);
     double* h = ctx->host_for(1);
     LT_HIP_CHECK(hipMemcpyAsync(h, part + nb, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));

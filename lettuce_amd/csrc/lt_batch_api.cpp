@@ -276,7 +276,8 @@ int lt_batch_create(lt_ctx ctx, int n_rep, const int* shapes, int n_levels, doub
                 b->levels.push_back(dev_alloc<double2>(b->ctx, nl));
                 b->tapes.push_back(dev_alloc<double2>(b->ctx, (size_t)lt::alg_offset(b->total)));
             }
-            b->part = dev_alloc<double>(b->ctx, (size_t)std::max(b->total_sb, b->total_kb));
+            // three partials per site block (charge) or one per block of the link reductions
+            b->part = dev_alloc<double>(b->ctx, std::max((size_t)3 * b->total_sb, (size_t)b->total_kb));
 
             // per-replica scalar state, one allocation
             const size_t n = (size_t)n_rep;

@@ -120,23 +120,6 @@ __device__ __forceinline__ int plane_of(int a, int b)
 //   R[((plane*2 + parity)*5 + k)*Vh + cb],
 //   k: 0 r01, 1 r02, 2 r12, 3 (Im r00, Im r11), 4 (Im r22, 0);
 // Re r_ii = 0 and r_ji = -conj(r_ij) hold exactly for C - C^+ in floating point.
-__device__ __forceinline__ M3 ld_plane(const double2* __restrict__ R, const Geom& g, int s, int plane, int par)
-{
-    const double2* p = R + slot_base(g, plane * 2 + par, R_SLOTS, cbi(g, s));
-    const double2 a01 = p[0], a02 = p[slot_stride(g)], a12 = p[(size_t)2 * slot_stride(g)];
-    const double2 d01 = p[(size_t)3 * slot_stride(g)], d2 = p[(size_t)4 * slot_stride(g)];
-    M3 r;
-    r.m[0] = cd{0.0, d01.x};
-    r.m[4] = cd{0.0, d01.y};
-    r.m[8] = cd{0.0, d2.x};
-    r.m[1] = cd{a01.x, a01.y};
-    r.m[2] = cd{a02.x, a02.y};
-    r.m[5] = cd{a12.x, a12.y};
-    r.m[3] = cd{-a01.x, a01.y};
-    r.m[6] = cd{-a02.x, a02.y};
-    r.m[7] = cd{-a12.x, a12.y};
-    return r;
-}
 __device__ __forceinline__ Tri ld_plane_tri(const double2* __restrict__ R, const Geom& g, int s, int plane, int par)
 {
     const double2* p = R + slot_base(g, plane * 2 + par, R_SLOTS, cbi(g, s));
@@ -144,24 +127,14 @@ __device__ __forceinline__ Tri ld_plane_tri(const double2* __restrict__ R, const
     const double2 d01 = p[(size_t)3 * slot_stride(g)], d2 = p[(size_t)4 * slot_stride(g)];
     return Tri{d01.x, d01.y, d2.x, cd{a01.x, a01.y}, cd{a02.x, a02.y}, cd{a12.x, a12.y}};
 }
-// stores R = C - C^+ of the clover term C
-__device__ __forceinline__ void st_plane(double2* __restrict__ R, const Geom& g, int s, int plane, int par, const M3& c)
+__device__ __forceinline__ void st_plane(double2* __restrict__ R, const Geom& g, int s, int plane, int par, const Tri& r)
 {
     double2* p = R + slot_base(g, plane * 2 + par, R_SLOTS, cbi(g, s));
-    const cd r01 = c.m[1] - conj(c.m[3]), r02 = c.m[2] - conj(c.m[6]), r12 = c.m[5] - conj(c.m[7]);
-    p[0] = make_double2(r01.re, r01.im);
-    p[slot_stride(g)] = make_double2(r02.re, r02.im);
-    p[(size_t)2 * slot_stride(g)] = make_double2(r12.re, r12.im);
-    p[(size_t)3 * slot_stride(g)] = make_double2(c.m[0].im + c.m[0].im, c.m[4].im + c.m[4].im);
-    p[(size_t)4 * slot_stride(g)] = make_double2(c.m[8].im + c.m[8].im, 0.0);
-}
-
-// R_rhosigma(y) = C_rhosigma - C_sigmarho with C_sigmarho = C_rhosigma^+
-__device__ __forceinline__ M3 R_at(const double2* __restrict__ C, const Geom& g, int y, int ypar, int rho, int sigma)
-{
-    const int lo = rho < sigma ? rho : sigma, hi = rho < sigma ? sigma : rho;
-    M3 r = ld_plane(C, g, y, plane_of(lo, hi), ypar);
-    return rho < sigma ? r : scale(-1.0, r);
+    p[0] = make_double2(r.r01.re, r.r01.im);
+    p[slot_stride(g)] = make_double2(r.r02.re, r.r02.im);
+    p[(size_t)2 * slot_stride(g)] = make_double2(r.r12.re, r.r12.im);
+    p[(size_t)3 * slot_stride(g)] = make_double2(r.d0, r.d1);
+    p[(size_t)4 * slot_stride(g)] = make_double2(r.d2, 0.0);
 }
 
 // stout level with tape: Q = -i rho Algebra(st U^+), U' = exp(iQ) U, Gram-Schmidt.
@@ -193,35 +166,16 @@ __device__ __forceinline__ void body_stout_tape(const double2* __restrict__ Uin,
     stu(Uout, g, s, mu, par, W);
 }
 
-// the clover term of one plane at site s
-__device__ __forceinline__ void body_clover_store(const double2* __restrict__ U, double2* __restrict__ C, const Geom& g,
-                                                  int s, int plane)
+// Planes p and 5 - p of the site of index i (half_cb order), stored, and their term of the
+// charge density Re tr(R01 R23 - R02 R13 + R03 R12)
+__device__ __forceinline__ double body_clover_pair(const double2* __restrict__ U, double2* __restrict__ C, const Geom& g,
+                                                   int i, int p)
 {
+    const int cb = half_cb(i), par = half_par(i);
+    if (cb >= g.Vh) return 0.0;
     int c[4];
-    coords_of(g, s, c);
-    const int par = parity_of(c);
-    double pl;
-    M3 cl;
-    switch (plane) {
-        case 0: cl = clover_plane(U, g, s, c, par, 0, 1, pl); break;
-        case 1: cl = clover_plane(U, g, s, c, par, 0, 2, pl); break;
-        case 2: cl = clover_plane(U, g, s, c, par, 0, 3, pl); break;
-        case 3: cl = clover_plane(U, g, s, c, par, 1, 2, pl); break;
-        case 4: cl = clover_plane(U, g, s, c, par, 1, 3, pl); break;
-        default: cl = clover_plane(U, g, s, c, par, 2, 3, pl); break;
-    }
-    st_plane(C, g, s, plane, par, cl);
-}
-
-// Re tr(F01 F23 - F02 F13 + F03 F12) at site s, F = C - C^+
-__device__ __forceinline__ double body_qdensity_site(const double2* __restrict__ C, const Geom& g, int s)
-{
-    int c[4];
-    coords_of(g, s, c);
-    const int par = parity_of(c);
-    return retr_mul(R_at(C, g, s, par, 0, 1), R_at(C, g, s, par, 2, 3))
-         - retr_mul(R_at(C, g, s, par, 0, 2), R_at(C, g, s, par, 1, 3))
-         + retr_mul(R_at(C, g, s, par, 0, 3), R_at(C, g, s, par, 1, 2));
+    const int s = site_of_cb(g, cb, par, c);
+    return clover_pair(U, g, s, c, par, p, [&](int plane, const Tri& r, double) { st_plane(C, g, s, plane, par, r); });
 }
 
 // Re tr of the plaquette U_mu(x) U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+ (plaquette.hpp:20-24)

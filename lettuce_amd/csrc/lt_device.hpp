@@ -1460,48 +1460,6 @@ __device__ __forceinline__ M3 park_load(const double2* park, int n)
     return a;
 }
 
-// Sum of the four clover leaves of plane (mu, nu) at site s (leaf orientation of
-// the reference's CalculateClover<1,1>); leaf I (the plaquette) is returned too.
-
-// park (optional, see park_store): the running sum of the leaves waits in LDS while the
-// next leaf is formed, and the leaves read their links afresh, so that one leaf at a
-// time holds registers (the tests of park are branches the compiler does not hoist the
-// next leaf's loads above); the same operations in the same order either way.
-__device__ __forceinline__ M3 clover_plane(const double2* __restrict__ U, const Geom& g, int s, const int c[4], int par,
-                                           int mu, int nu, double& retr_plaq, double2* park = nullptr, int n = 0)
-{
-    // every leaf is a product of four links, an SU(3) matrix: rows 0 and 1 are
-    // multiplied out along the chain, row 2 is conj(row0 x row1)
-    const int q = par ^ 1;
-    const int smu = up(g, s, c[mu], mu), snu = up(g, s, c[nu], nu);
-    const int smd = dn(g, s, c[mu], mu), snd = dn(g, s, c[nu], nu);
-    const int smd_nu = up(g, smd, c[nu], nu), smd_nd = dn(g, smd, c[nu], nu), smu_nd = up(g, snd, c[mu], mu);
-    // leaf I: U_mu(x) U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+
-    M3 C = mul_nd_r01(mul_nd_r01(mul_r01(ldu(U, g, s, mu, par), ldu(U, g, smu, nu, q)), ldu(U, g, snu, mu, q)),
-                      ldu(U, g, s, nu, par));
-    third_row(C);
-    retr_plaq = C.m[0].re + C.m[4].re + C.m[8].re;
-    if (park) park_store(park, n, C);
-    // leaf II: U_nu(x) U_mu(x-mu+nu)^+ U_nu(x-mu)^+ U_mu(x-mu)
-    M3 t = mul_r01(mul_nd_r01(mul_nd_r01(ldu(U, g, s, nu, par), ldu(U, g, smd_nu, mu, par)), ldu(U, g, smd, nu, q)),
-                   ldu(U, g, smd, mu, q));
-    if (park) C = park_load(park, n);
-    acc_su3_r01(C, t);
-    if (park) park_store(park, n, C);
-    // leaf III: U_mu(x-mu)^+ U_nu(x-mu-nu)^+ U_mu(x-mu-nu) U_nu(x-nu)
-    t = mul_r01(mul_r01(mul_dd_r01(ldu(U, g, smd, mu, q), ldu(U, g, smd_nd, nu, par)), ldu(U, g, smd_nd, mu, par)),
-                ldu(U, g, snd, nu, q));
-    if (park) C = park_load(park, n);
-    acc_su3_r01(C, t);
-    if (park) park_store(park, n, C);
-    // leaf IV: U_nu(x-nu)^+ U_mu(x-nu) U_nu(x+mu-nu) U_mu(x)^+
-    t = mul_nd_r01(mul_r01(mul_dn_r01(ldu(U, g, snd, nu, q), ldu(U, g, snd, mu, q)), ldu(U, g, smu_nd, nu, par)),
-                   ldu(U, g, s, mu, par));
-    if (park) C = park_load(park, n);
-    acc_su3_r01(C, t);
-    return C;
-}
-
 // r += leaf - leaf^+ for an SU(3) leaf given by rows 0 and 1 (row 2 = conj(row0 x row1))
 __device__ __forceinline__ void acc_leaf(Tri& r, M3& t)
 {
