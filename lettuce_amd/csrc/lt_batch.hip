@@ -140,20 +140,19 @@ bk_clover_charge(const double2* __restrict__ U, double2* __restrict__ C, BatchGr
 
 __global__ void __launch_bounds__(RBS) bk_plaq(const double2* __restrict__ U, BatchGrid bg, double* part)
 {
-    const int r = rep_of(bg.sb, bg.n, blockIdx.x);
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    const int sbk = b / 3;
+    const int r = rep_of(bg.sb, bg.n, sbk);
     const Geom g = bg.reps[r].g;
-    const long long off = bg.reps[r].off;
-    const int s = (blockIdx.x - bg.sb[r]) * RBS + threadIdx.x;
-    block_sum(s < g.V ? body_plaq_site(U + off, g, s) : 0.0, part + blockIdx.x);
+    block_sum(body_plaq_pair(U + bg.reps[r].off, g, (sbk - bg.sb[r]) * RBS + threadIdx.x, b % 3), part + b);
 }
 
 __global__ void __launch_bounds__(RBS) bk_kinetic(const double2* __restrict__ P, BatchGrid bg, double* part)
 {
     const int r = rep_of(bg.kb, bg.n, blockIdx.x);
     const Geom g = bg.reps[r].g;
-    const long long off = bg.reps[r].off;
-    const long long id = (long long)(blockIdx.x - bg.kb[r]) * RBS + threadIdx.x;
-    block_sum(id < 4LL * g.V ? body_kinetic_link(P + off, g, id) : 0.0, part + blockIdx.x);
+    const int i = (blockIdx.x - bg.kb[r]) * RBS + threadIdx.x;
+    block_sum(i < 8 * g.Vh ? body_kinetic_link(P + bg.reps[r].off, g, i) : 0.0, part + blockIdx.x);
 }
 
 // block r: ordered sum of replica r's partials (same order as the single-lattice finish)
@@ -427,8 +426,8 @@ void kb_stout_recursion_run(lt_ctx ctx, const BatchGrid& bg, int total_lb, const
 
 void kb_plaquette(lt_ctx ctx, const BatchGrid& bg, int total_sb, const double2* U, double* part, double* out)
 {
-    launch(ctx, "batch_plaquette", bk_plaq, dim3(total_sb), dim3(RBS), 0, U, bg, part);
-    launch(ctx, "batch_finish", bk_finish, dim3(bg.n), dim3(RBS), 0, (const double*)part, bg.sb, 1, out);
+    launch(ctx, "batch_plaquette", bk_plaq, dim3(3 * total_sb), dim3(RBS), 0, U, bg, part);
+    launch(ctx, "batch_finish", bk_finish, dim3(bg.n), dim3(RBS), 0, (const double*)part, bg.sb, 3, out);
 }
 
 void kb_kinetic(lt_ctx ctx, const BatchGrid& bg, int total_kb, const double2* P, double* part, double* out)
