@@ -484,109 +484,104 @@ __device__ __forceinline__ void exp_constants_c(double c0s, double c1, ExpC& e)
 constexpr double EXP_SERIES_SMALL = 0.02, EXP_SERIES_C1 = 1.0;
 constexpr int EXP_TERMS_SMALL = 12, EXP_TERMS = 20;
 
-// z += i^k x
-template <int K4>
+// z += i^k t x.  k is a template argument all the way: with a run-time k in an unrolled loop
+// the choice of re or im became a selected address, which kept z in scratch memory.
+template <int K>
 __device__ __forceinline__ void acc_ik(cd& z, double t, double x)
 {
-    if (K4 == 0) z.re = fma(t, x, z.re);
-    if (K4 == 1) z.im = fma(t, x, z.im);
-    if (K4 == 2) z.re = fma(-t, x, z.re);
-    if (K4 == 3) z.im = fma(-t, x, z.im);
+    constexpr int q = K & 3;
+    if constexpr (q == 0) z.re = fma(t, x, z.re);
+    if constexpr (q == 1) z.im = fma(t, x, z.im);
+    if constexpr (q == 2) z.re = fma(-t, x, z.re);
+    if constexpr (q == 3) z.im = fma(-t, x, z.im);
 }
-__device__ __forceinline__ void acc_ik(cd& z, int k, double t, double x)
+constexpr double inv_factorial(int k)
 {
-    switch (k & 3) {
-        case 0: acc_ik<0>(z, t, x); break;
-        case 1: acc_ik<1>(z, t, x); break;
-        case 2: acc_ik<2>(z, t, x); break;
-        default: acc_ik<3>(z, t, x); break;
-    }
+    double t = 1.0;
+    for (int i = 2; i <= k; ++i) t /= (double)i;
+    return t;
 }
+// the terms k .. K; gm, g, gp: G_{k-2}, G_{k-1}, G_k
+template <int k, int K>
+__device__ __forceinline__ void exp_terms(double c0, double c1, double gm, double g, double gp, cd& s0, cd& f1, cd& f2)
+{
+    constexpr double t = inv_factorial(k);
+    const double next = k == 2 ? 0.0 : fma(c1, g, c0 * gm);
+    if constexpr (k >= 3) acc_ik<k>(s0, t, g);
+    acc_ik<k>(f2, t, gp);
+    if constexpr (k >= 3) acc_ik<k>(f1, t, next);
+    if constexpr (k < K) exp_terms<k + 1, K>(c0, c1, g, gp, next, s0, f1, f2);
+}
+struct ExpCoeffs {
+    cd f0, f1, f2;
+};
 template <int K>
-__device__ __forceinline__ void exp_series(double c0, double c1, cd& f0, cd& f1, cd& f2)
+__device__ __forceinline__ ExpCoeffs exp_series(double c0, double c1)
 {
-    cd s0 = cd{0.0, 0.0};
-    f1 = cd{0.0, 1.0};        // k = 1: G_2 = 1
-    f2 = cd{0.0, 0.0};
-    double gm = 0.0, g = 0.0, gp = 1.0;   // G_{k-1}, G_k, G_{k+1} at k = 1
-    double t = 1.0;                       // 1/k!
-#pragma unroll
-    for (int k = 2; k <= K; ++k) {
-        const double next = k == 2 ? 0.0 : fma(c1, g, c0 * gm);   // G_{k+1}
-        gm = g;
-        g = gp;
-        gp = next;
-        t /= (double)k;
-        if (k >= 3) acc_ik(s0, k, t, gm);
-        acc_ik(f2, k, t, g);
-        if (k >= 3) acc_ik(f1, k, t, gp);
-    }
-    f0 = cd{fma(c0, s0.re, 1.0), c0 * s0.im};
+    cd s0 = cd{0.0, 0.0}, f1 = cd{0.0, 1.0}, f2 = cd{0.0, 0.0};   // k = 1: G_2 = 1
+    exp_terms<2, K>(c0, c1, 0.0, 0.0, 1.0, s0, f1, f2);
+    return ExpCoeffs{cd{fma(c0, s0.re, 1.0), c0 * s0.im}, f1, f2};
 }
 // f1, f2 and the derivatives b1j = df_j/dc1, b2j = df_j/dc0 (the b_ij of Morningstar-Peardon)
 struct ExpDeriv {
     cd f1, f2, b10, b11, b12, b20, b21, b22;
 };
+// sequences at term k: G_{k-2}, G_{k-1}, G_k and H_{k-3} .. H_k
+struct ExpSeq {
+    double gm, g, gp, hmm, hk1, hk, hp;
+};
+struct ExpSums {
+    cd s0, f1, f2, h2, h1, h0, hm;
+};
+template <int k, int K>
+__device__ __forceinline__ void exp_terms_deriv(double c0, double c1, const ExpSeq& q, ExpSums& s)
+{
+    constexpr double t = inv_factorial(k);
+    const double gnext = k == 2 ? 0.0 : fma(c1, q.g, c0 * q.gm);
+    const double hnext = k <= 2 ? 0.0 : (k == 3 ? 1.0 : fma(c1, q.hk, fma(c0, q.hk1, q.g)));   // H_{k+1}
+    acc_ik<k>(s.f2, t, q.gp);
+    if constexpr (k >= 3) {
+        acc_ik<k>(s.s0, t, q.g);
+        acc_ik<k>(s.f1, t, gnext);
+        acc_ik<k>(s.h2, t, hnext);    // sum i^k/k! H_{k+1}
+    }
+    if constexpr (k >= 4) acc_ik<k>(s.h1, t, q.hp);
+    if constexpr (k >= 5) acc_ik<k>(s.h0, t, q.hk);
+    if constexpr (k >= 6) acc_ik<k>(s.hm, t, q.hk1);
+    if constexpr (k < K)
+        exp_terms_deriv<k + 1, K>(c0, c1, ExpSeq{q.g, q.gp, gnext, q.hk1, q.hk, q.hp, hnext}, s);
+}
 template <int K>
 __device__ __forceinline__ void exp_series_deriv(double c0, double c1, ExpDeriv& d)
 {
-    cd s0 = cd{0.0, 0.0}, h2 = cd{0.0, 0.0}, h1 = cd{0.0, 0.0}, h0 = cd{0.0, 0.0}, hm = cd{0.0, 0.0};
-    cd f1 = cd{0.0, 1.0}, f2 = cd{0.0, 0.0};
-    double gm = 0.0, g = 0.0, gp = 1.0;
-    double hmm = 0.0, hk1 = 0.0, hk = 0.0, hp = 0.0;   // H_{k-2}, H_{k-1}, H_k, H_{k+1}
-    double t = 1.0;
-#pragma unroll
-    for (int k = 2; k <= K; ++k) {
-        const double gnext = k == 2 ? 0.0 : fma(c1, g, c0 * gm);
-        const double hnext = k <= 2 ? 0.0 : (k == 3 ? 1.0 : fma(c1, hk, fma(c0, hk1, g)));   // H_{k+1}
-        gm = g;
-        g = gp;
-        gp = gnext;
-        hmm = hk1;
-        hk1 = hk;
-        hk = hp;
-        hp = hnext;
-        t /= (double)k;
-        acc_ik(f2, k, t, g);
-        if (k >= 3) {
-            acc_ik(s0, k, t, gm);
-            acc_ik(f1, k, t, gp);
-            acc_ik(h2, k, t, hp);    // sum i^k/k! H_{k+1}
-        }
-        if (k >= 4) acc_ik(h1, k, t, hk);
-        if (k >= 5) acc_ik(h0, k, t, hk1);
-        if (k >= 6) acc_ik(hm, k, t, hmm);
-    }
-    d.f1 = f1;
-    d.f2 = f2;
-    d.b10 = c0 * h0;
-    d.b11 = h2;
-    d.b12 = h1;
-    d.b20 = cd{fma(c0, hm.re, s0.re), fma(c0, hm.im, s0.im)};
-    d.b21 = h1;
-    d.b22 = h0;
+    ExpSums s{};
+    s.f1 = cd{0.0, 1.0};
+    exp_terms_deriv<2, K>(c0, c1, ExpSeq{0.0, 0.0, 1.0, 0.0, 0.0, 0.0, 0.0}, s);
+    d.f1 = s.f1;
+    d.f2 = s.f2;
+    d.b10 = c0 * s.h0;
+    d.b11 = s.h2;
+    d.b12 = s.h1;
+    d.b20 = cd{fma(c0, s.hm.re, s.s0.re), fma(c0, s.hm.im, s.s0.im)};
+    d.b21 = s.h1;
+    d.b22 = s.h0;
 }
-__device__ __forceinline__ void exp_coeffs(double c0, double c1, cd& f0, cd& f1, cd& f2)
+// By value: stores through references at the end of the three branches are merged into one
+// store to a selected address, which put the coefficients in scratch memory.
+__device__ __forceinline__ ExpCoeffs exp_coeffs(double c0, double c1)
 {
-    if (c1 <= EXP_SERIES_SMALL) {
-        exp_series<EXP_TERMS_SMALL>(c0, c1, f0, f1, f2);
-    } else if (c1 <= EXP_SERIES_C1) {
-        exp_series<EXP_TERMS>(c0, c1, f0, f1, f2);
-    } else {
-        ExpC e;
-        exp_constants_c(c0, c1, e);
-        f0 = e.denom * e.h0;
-        f1 = e.denom * e.h1;
-        f2 = e.denom * e.h2;
-    }
+    if (c1 <= EXP_SERIES_SMALL) return exp_series<EXP_TERMS_SMALL>(c0, c1);
+    if (c1 <= EXP_SERIES_C1) return exp_series<EXP_TERMS>(c0, c1);
+    ExpC e;
+    exp_constants_c(c0, c1, e);
+    return ExpCoeffs{e.denom * e.h0, e.denom * e.h1, e.denom * e.h2};
 }
 
 // exp(iQ)
 __device__ __forceinline__ M3 su3_exp(const M3& Q)
 {
     M3 Q2 = mul(Q, Q);
-    cd f0, f1, f2;
-    exp_coeffs((1.0 / 3.0) * retr_mul(Q, Q2), 0.5 * (Q2.m[0].re + Q2.m[4].re + Q2.m[8].re), f0, f1, f2);
+    const auto [f0, f1, f2] = exp_coeffs((1.0 / 3.0) * retr_mul(Q, Q2), 0.5 * (Q2.m[0].re + Q2.m[4].re + Q2.m[8].re));
     M3 r;
 #pragma unroll
     for (int i = 0; i < 9; ++i) r.m[i] = f1 * Q.m[i] + f2 * Q2.m[i];
@@ -996,8 +991,7 @@ __device__ __forceinline__ double her_det(const Tri& q)
 __device__ __forceinline__ M3 exp_her(const Tri& q)
 {
     const Tri s = her_square(q);
-    cd f0, f1, f2;
-    exp_coeffs(her_det(q), 0.5 * (s.d0 + s.d1 + s.d2), f0, f1, f2);
+    const auto [f0, f1, f2] = exp_coeffs(her_det(q), 0.5 * (s.d0 + s.d1 + s.d2));
     M3 r;
     r.m[0] = f0 + q.d0 * f1 + s.d0 * f2;
     r.m[4] = f0 + q.d1 * f1 + s.d1 * f2;

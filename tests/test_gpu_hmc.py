@@ -143,6 +143,53 @@ def test_cv_forward_backward_vs_oracle(la, lto, gpu_ctx, n_levels):
     cv.close()
 
 
+# c1 = tr Q^2 / 2 on both sides of the two lines where the exponential changes its evaluation
+# (0.02, 1), far from them, and zero
+@pytest.mark.parametrize("c1", [0.0, 1e-9, 0.0199999, 0.0200001, 0.3, 0.9999999, 1.0000001, 4.0])
+def test_exponential_against_expm(la, gpu_ctx, c1):
+    """The field update of unit links is exp(eps P).  Bar 3e-14: about a hundred roundings of
+    1.1e-16 on numbers of at most 3 (the exponential's polynomial and the Gram-Schmidt step)."""
+    from scipy.linalg import expm
+    flush(f"exponential c1 = {c1}")
+    rng = np.random.default_rng(int(1e7 * c1) + 1)
+    n = 4 * 4**4
+    H = rng.normal(size=(n, 3, 3)) + 1j * rng.normal(size=(n, 3, 3))
+    H[0] = np.diag([1.0, 1.0, -2.0])      # a double eigenvalue, either sign of det Q
+    H[1] = np.diag([-1.0, -1.0, 2.0])
+    H[2] = np.diag([1.0, -1.0, 0.0])
+    H = H + H.conj().transpose(0, 2, 1)
+    H -= np.trace(H, axis1=1, axis2=2)[:, None, None] / 3.0 * np.eye(3)
+    H *= np.sqrt(c1 / (0.5 * np.einsum("nij,nji->n", H, H).real))[:, None, None]
+    ref = np.array([expm(1j * h) for h in H])
+    U, P = gauge(la, gpu_ctx, TINY), matrix(la, gpu_ctx, TINY)
+    U.SetToIdentity()
+    shape = U.download().shape
+    P.upload(np.ascontiguousarray(2j * H).view(np.float64).reshape(shape))
+    la.UpdateFields(U, P, 0.5)
+    got = U.download().view(np.complex128).reshape(n, 3, 3)
+    assert np.max(np.abs(got - ref)) <= 3e-14, np.max(np.abs(got - ref))
+    U.close()
+    P.close()
+
+
+@pytest.mark.parametrize("rho", [0.02, 0.12, 0.4, 0.7])
+def test_cv_force_stout_weights(la, lto, gpu_ctx, rho):
+    """Exponential and derivative of one stout level on rough links: rho runs the arguments
+    through all three evaluations (c1 about 5 rho^2, spread over the links)."""
+    flush(f"cv rho {rho}")
+    shape = (4, 4, 4, 6)
+    U0 = lto.haar(shape, 3)
+    U = gauge(la, gpu_ctx, shape, U0)
+    F = matrix(la, gpu_ctx, shape)
+    cv = la.CollectiveVariable(gpu_ctx, shape, 1, rho)
+    Q = cv.forward(U)
+    cv.backward(0.7, F)
+    Qr, Fr = lto.cv_force(U0, shape, rho, 1, 0.7)
+    assert abs(Q - Qr) <= 1e-12 * max(1.0, abs(Qr))
+    assert rel_err(F.download(), Fr) <= 1e-11
+    cv.close()
+
+
 def test_cv_force_golden16(la, lto, golden, gpu_ctx):
     flush("cv golden 16^4")
     U0 = lto.stout(lto.haar(G16, 0), G16, 0.1, 3)
