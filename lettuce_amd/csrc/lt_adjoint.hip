@@ -5,10 +5,11 @@
 //
 // Buffers (general 3x3 layout unless noted):
 //   levels    n+1 link fields (two-row SU(3))
-//   tape      per level, per link: the hermitian exponent Q = -i rho Algebra(st U^+), 8 reals (ld_her8)
+//   tape      per level, per link: the hermitian exponent Q = -i rho Algebra(st U^+), 8 reals (ld_her8_tri)
 //   clover    6 planes per site, R = C - C^+ in 9 reals: C[((plane*2 + parity)*5 + k)*Vh + cb]
-//   sigma     force being propagated (in place, level by level)
-//   lambda    per-link Lambda of the current level, 8 reals (ld_her8)
+//   sigma     force being propagated (in place, level by level): Y of lambda_link in 8 reals
+//             between the levels, the whole matrix at the ends
+//   lambda    per-link Lambda of the current level, 8 reals (ld_her8_tri)
 // The per-thread bodies live in lt_bodies.hpp and are shared with the
 // replica-batched kernels.
 #include "lt_internal.hpp"
@@ -55,20 +56,19 @@ __global__ void LT_LINK_KERNEL clover_deriv_all_kernel(const double2* __restrict
     body_clover_deriv_all<LAMBDA>(U, C, F, g, m, link_block(m, blockIdx.x, gridDim.x), scale_factor, acc, next);
 }
 
-__global__ void LT_LINK_KERNEL lambda_kernel(const double2* __restrict__ U, const double2* __restrict__ Uprev,
-                                             double2* __restrict__ Sig, const double2* __restrict__ T,
+__global__ void LT_LINK_KERNEL lambda_kernel(double2* __restrict__ Sig, const double2* __restrict__ T,
                                              double2* __restrict__ Lam, Geom g, LinkMap m)
 {
-    body_lambda(U, Uprev, Sig, T, Lam, g, m, link_block(m, blockIdx.x, gridDim.x));
+    body_lambda(Sig, T, Lam, g, m, link_block(m, blockIdx.x, gridDim.x));
 }
 
 template <int MODE>
 __global__ void LT_LINK_KERNEL sigma_all_kernel(const double2* __restrict__ U, double2* __restrict__ Sig,
-                                                const double2* __restrict__ T, const double2* __restrict__ Lam, Geom g,
-                                                LinkMap m, double rho, MomentumKick kick, SigmaNext next)
+                                                const double2* __restrict__ Lam, Geom g, LinkMap m, double rho,
+                                                MomentumKick kick, SigmaNext next)
 {
     extern __shared__ double2 lds[];
-    body_sigma_all<MODE>(U, Sig, T, Lam, g, m, link_block(m, blockIdx.x, gridDim.x), rho, lds, kick, next);
+    body_sigma_all<MODE>(U, Sig, Lam, g, m, link_block(m, blockIdx.x, gridDim.x), rho, lds, kick, next);
 }
 
 }  // namespace
@@ -113,22 +113,20 @@ void k_stout_recursion_run(lt_ctx ctx, const Geom& g, const LinkMap& m, const Le
     const size_t lds = 18 * m.nthreads * sizeof(double2);
     int cur = 0;
     if (!top_lambda_done)
-        launch(ctx, "stout_lambda", lambda_kernel, grid, block, 0, level(hi - 1), level(hi), Sig, tape(hi - 1), lam[cur],
-               g, m);
+        launch(ctx, "stout_lambda", lambda_kernel, grid, block, 0, Sig, tape(hi - 1), lam[cur], g, m);
     for (int k = hi; k > lo; --k) {
         const double2* U = level(k - 1);
-        const double2* T = tape(k - 1);
         const double2* L = lam[cur];
         if (k - 1 > lo) {
-            const SigmaNext next{level(k - 2), tape(k - 2), lam[cur ^ 1]};
-            launch(ctx, "stout_sigma", sigma_all_kernel<SIGMA_LAMBDA>, grid, block, lds, U, Sig, T, L, g, m, rho,
+            const SigmaNext next{tape(k - 2), lam[cur ^ 1]};
+            launch(ctx, "stout_sigma", sigma_all_kernel<SIGMA_LAMBDA>, grid, block, lds, U, Sig, L, g, m, rho,
                    MomentumKick{}, next);
             cur ^= 1;
         } else if (kick && k == 1) {
-            launch(ctx, "stout_sigma", sigma_all_kernel<SIGMA_KICK>, grid, block, lds, U, Sig, T, L, g, m, rho, *kick,
+            launch(ctx, "stout_sigma", sigma_all_kernel<SIGMA_KICK>, grid, block, lds, U, Sig, L, g, m, rho, *kick,
                    SigmaNext{});
         } else {
-            launch(ctx, "stout_sigma", sigma_all_kernel<SIGMA_STORE>, grid, block, lds, U, Sig, T, L, g, m, rho,
+            launch(ctx, "stout_sigma", sigma_all_kernel<SIGMA_STORE>, grid, block, lds, U, Sig, L, g, m, rho,
                    MomentumKick{}, SigmaNext{});
         }
     }

@@ -79,28 +79,27 @@ __global__ void LT_LINK_KERNEL bk_clover_deriv_all(const double2* __restrict__ U
 {
     extern __shared__ double2 acc[];
     LT_BATCH_LINK_PROLOGUE
-    if (LAMBDA) next = SigmaNext{next.U + off, next.T + alg_offset(off), next.Lam + alg_offset(off)};
+    if (LAMBDA) next = SigmaNext{next.T + alg_offset(off), next.Lam + alg_offset(off)};
     body_clover_deriv_all<LAMBDA>(U + off, C + clover_offset(off), F + off, g, m, lb, scale[r], acc, next);
 }
 
-__global__ void LT_LINK_KERNEL bk_lambda(const double2* __restrict__ U, const double2* __restrict__ Uprev,
-                                         double2* __restrict__ Sig, const double2* __restrict__ T,
+__global__ void LT_LINK_KERNEL bk_lambda(double2* __restrict__ Sig, const double2* __restrict__ T,
                                          double2* __restrict__ Lam, BatchGrid bg)
 {
     LT_BATCH_LINK_PROLOGUE
-    body_lambda(U + off, Uprev + off, Sig + off, T + alg_offset(off), Lam + alg_offset(off), g, m, lb);
+    body_lambda(Sig + off, T + alg_offset(off), Lam + alg_offset(off), g, m, lb);
 }
 
 template <int MODE>
 __global__ void LT_LINK_KERNEL bk_sigma_all(const double2* __restrict__ U, double2* __restrict__ Sig,
-                                            const double2* __restrict__ T, const double2* __restrict__ Lam, BatchGrid bg,
-                                            double rho, MomentumKick kick, SigmaNext next)
+                                            const double2* __restrict__ Lam, BatchGrid bg, double rho,
+                                            MomentumKick kick, SigmaNext next)
 {
     extern __shared__ double2 lds[];
     LT_BATCH_LINK_PROLOGUE
     if (MODE == SIGMA_KICK) kick.P += off;
-    if (MODE == SIGMA_LAMBDA) next = SigmaNext{next.U + off, next.T + alg_offset(off), next.Lam + alg_offset(off)};
-    body_sigma_all<MODE>(U + off, Sig + off, T + alg_offset(off), Lam + alg_offset(off), g, m, lb, rho, lds, kick, next);
+    if (MODE == SIGMA_LAMBDA) next = SigmaNext{next.T + alg_offset(off), next.Lam + alg_offset(off)};
+    body_sigma_all<MODE>(U + off, Sig + off, Lam + alg_offset(off), g, m, lb, rho, lds, kick, next);
 }
 
 #undef LT_BATCH_LINK_PROLOGUE
@@ -403,22 +402,20 @@ void kb_stout_recursion_run(lt_ctx ctx, const BatchGrid& bg, int total_lb, const
     const size_t lds = 18 * block.x * sizeof(double2);
     int cur = 0;
     if (!top_lambda_done)
-        launch(ctx, "batch_stout_lambda", bk_lambda, grid, block, 0, level(hi - 1), level(hi), Sig, tape(hi - 1),
-               lam[cur], bg);
+        launch(ctx, "batch_stout_lambda", bk_lambda, grid, block, 0, Sig, tape(hi - 1), lam[cur], bg);
     for (int k = hi; k > lo; --k) {
         const double2* U = level(k - 1);
-        const double2* T = tape(k - 1);
         const double2* L = lam[cur];
         if (k - 1 > lo) {
-            const SigmaNext next{level(k - 2), tape(k - 2), lam[cur ^ 1]};
-            launch(ctx, "batch_stout_sigma", bk_sigma_all<SIGMA_LAMBDA>, grid, block, lds, U, Sig, T, L, bg, rho,
+            const SigmaNext next{tape(k - 2), lam[cur ^ 1]};
+            launch(ctx, "batch_stout_sigma", bk_sigma_all<SIGMA_LAMBDA>, grid, block, lds, U, Sig, L, bg, rho,
                    MomentumKick{}, next);
             cur ^= 1;
         } else if (kick && k == 1) {
-            launch(ctx, "batch_stout_sigma", bk_sigma_all<SIGMA_KICK>, grid, block, lds, U, Sig, T, L, bg, rho, *kick,
+            launch(ctx, "batch_stout_sigma", bk_sigma_all<SIGMA_KICK>, grid, block, lds, U, Sig, L, bg, rho, *kick,
                    SigmaNext{});
         } else {
-            launch(ctx, "batch_stout_sigma", bk_sigma_all<SIGMA_STORE>, grid, block, lds, U, Sig, T, L, bg, rho,
+            launch(ctx, "batch_stout_sigma", bk_sigma_all<SIGMA_STORE>, grid, block, lds, U, Sig, L, bg, rho,
                    MomentumKick{}, SigmaNext{});
         }
     }

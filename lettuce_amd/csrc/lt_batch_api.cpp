@@ -169,8 +169,7 @@ void enqueue_step(lt_batch b, const StepKey& p, int n_sub)
                 lt::kb_dvdq(ctx, bg, st, bias, sub ? isub++ : -1);
                 const int n = b->n_levels;
                 // the clover derivative goes on with the Lambda of the top level
-                const lt::SigmaNext top{n > 0 ? b->levels[n - 1] : nullptr, n > 0 ? b->tapes[n - 1] : nullptr,
-                                        b->lambda[0]};
+                const lt::SigmaNext top{n > 0 ? b->tapes[n - 1] : nullptr, b->lambda[0]};
                 lt::kb_clover_deriv(ctx, bg, b->total_lb, b->levels[n], b->clover, b->F, st.dvdq, n > 0 ? &top : nullptr);
                 // KICK_BOTH: UpdateMomenta applied by the last kernel of the force (level 0 = U)
                 const lt::MomentumKick mk{b->P, e * p.beta / 6.0, e};

@@ -248,12 +248,11 @@ __device__ __forceinline__ void park_acc(double2* slot, int n, const M3& a)
 // 1500 FP64 instructions per nu instead of 1900.
 // LDS: 15 x 16 bytes per lane of the block.
 constexpr int CDERIV_SLOTS = 15;
-__device__ __forceinline__ void lambda_link(const double2* __restrict__ U, const M3& Lprev, const M3& sig,
-                                            double2* __restrict__ Sig, const double2* __restrict__ T,
+__device__ __forceinline__ void lambda_link(const M3& sig, const Tri& Q, double2* __restrict__ Sig,
                                             double2* __restrict__ Lam, const Geom& g, int s, int mu, int par);
 // LAMBDA: the force is the Sigma of the top stout level; instead of storing it the kernel
-// goes on with that level's Lambda (lambda_link, next: the level below, its tape and the
-// Lambda buffer), as the first launch of the stout-force recursion would.
+// goes on with that level's Lambda (lambda_link, next: its tape and the Lambda buffer), as the
+// first launch of the stout-force recursion would.
 template <bool LAMBDA>
 __device__ __forceinline__ void body_clover_deriv_all(const double2* __restrict__ U, const double2* __restrict__ C,
                                                       double2* __restrict__ F, const Geom& g, const LinkMap& m, int b,
@@ -317,28 +316,31 @@ __device__ __forceinline__ void body_clover_deriv_all(const double2* __restrict_
     const M3 L = ldu(U, g, s, mu, par);
     a = scale(scale_factor * pref, algebra(mul(L, a)));
     if (LAMBDA)
-        lambda_link(next.U, L, a, F, next.T, next.Lam, g, s, mu, par);
+        lambda_link(a, ld_her8_tri(next.T, g, s, mu, par), F, next.Lam, g, s, mu, par);
     else
         st_link(F, g, s, mu, par, a);
 }
 
-// Sigma' = Uprev^+ Sigma (stored in place) and
-// Lambda = TracelessHermitian(tr(B1 G) Q + tr(B2 G) Q^2 + f1 G + f2 (Q G + G Q)), G = U Sigma'
-// one link, with Uprev's link and Sigma given
-__device__ __forceinline__ void lambda_link(const double2* __restrict__ U, const M3& Lprev, const M3& sig,
-                                            double2* __restrict__ Sig, const double2* __restrict__ T,
+// Lambda = TracelessHermitian(tr(B1 G) Q + tr(B2 G) Q^2 + f1 G + f2 (Q G + G Q)), G = U Sigma',
+// Sigma' = Uprev^+ Sigma, of one link.  Uprev = exp(iQ) U and Sigma is anti-hermitian and
+// traceless, so G = exp(-iQ) Sigma needs neither field, and what the level below adds to its
+// own terms is U (Sigma' exp(iQ)) = exp(-iQ) Sigma exp(iQ) = Y, again anti-hermitian and
+// traceless: Y goes to Sig in 8 reals.  Storing Sigma' (9 complex entries), reading it, the
+// tape and the next level's links again and evaluating the exponential once more took 736
+// bytes a link and level instead of 416, and about 10 % more FP64 instructions.
+__device__ __forceinline__ void lambda_link(const M3& sig, const Tri& Q, double2* __restrict__ Sig,
                                             double2* __restrict__ Lam, const Geom& g, int s, int mu, int par)
 {
-    M3 sp = mul_dn(Lprev, sig);
-    st_link(Sig, g, s, mu, par, sp);
-    const Tri Q = ld_her8_tri(T, g, s, mu, par);
-    const M3 G = mul(ldu(U, g, s, mu, par), sp);
-    M3 QG = m3_zero();   // Q G + G Q, of trace 2 tr(Q G)
-    mul_tri_acc<false, 1>(QG, G, Q);
-    tri_mul_acc<false, 1>(QG, Q, G);
     const Tri Q2 = her_square(Q);
     ExpDeriv d;
     exp_deriv(her_det(Q), 0.5 * (Q2.d0 + Q2.d1 + Q2.d2), d);
+    const M3 E = her_poly(d.f0, d.f1, d.f2, Q, Q2);
+    M3 G = m3_zero();
+    mul_tri_acc<true, 1>(G, dag(E), ah_tri(sig));
+    st_ah8(Sig, g, s, mu, par, mul_ah(G, E));
+    M3 QG = m3_zero();   // Q G + G Q, of trace 2 tr(Q G)
+    mul_tri_acc<false, 1>(QG, G, Q);
+    tri_mul_acc<false, 1>(QG, Q, G);
     // tr(B_i G) = b_i0 tr G + b_i1 tr(Q G) + b_i2 tr(Q^2 G)
     const cd tg = trace(G), tqg = 0.5 * trace(QG);
     cd tq2g = Q2.d0 * G.m[0] + Q2.d1 * G.m[4] + Q2.d2 * G.m[8];
@@ -364,13 +366,13 @@ __device__ __forceinline__ void lambda_link(const double2* __restrict__ U, const
     Gam.m[5] += t1.re * Q.r12 + t2.re * Q2.r12;
     st_her8(Lam, g, s, mu, par, Gam);
 }
-__device__ __forceinline__ void body_lambda(const double2* __restrict__ U, const double2* __restrict__ Uprev,
-                                            double2* __restrict__ Sig, const double2* __restrict__ T,
+// Sigma as a whole matrix in Sig
+__device__ __forceinline__ void body_lambda(double2* __restrict__ Sig, const double2* __restrict__ T,
                                             double2* __restrict__ Lam, const Geom& g, const LinkMap& m, int b)
 {
     int mu, par, c[4], s;
     if (!map_link_b(g, m, b, mu, par, c, s)) return;
-    lambda_link(U, ldu(Uprev, g, s, mu, par), ld(Sig, g, s, mu, par), Sig, T, Lam, g, s, mu, par);
+    lambda_link(ld(Sig, g, s, mu, par), ld_her8_tri(T, g, s, mu, par), Sig, Lam, g, s, mu, par);
 }
 
 // The six-term sum and the staple st are formed in one loop over nu != mu from the same
@@ -383,12 +385,16 @@ __device__ __forceinline__ void body_lambda(const double2* __restrict__ U, const
 // The products with a Lambda use that it is hermitian (mul_tri_acc).  About 1250 FP64
 // instructions per nu instead of 1450.
 // LDS: 18 x 16 bytes per lane of the block.
+// The level's Sigma is Y + i rho Algebra(U (st^+ Lambda - sum)), Y from lambda_link.
+// Bound by load latency and VALU issue together at the two waves per SIMD that 246 registers
+// and 288 bytes of LDS a lane leave: a wave alone needs 10 us of VALU issue and twice that in
+// all, the first direction's halves longest (their lines come from beyond the L2).  b and its
+// Lambda are loaded a half ahead, the link's own after the last half.  Between events, levels
+// with a Lambda and the last one: 16 x 8^4 90 -> 84.7 us, 16^4 106 -> 98 us with Y instead of
+// Sigma' and the early loads; loading every operand two products ahead spills 68 registers.
 // MODE SIGMA_STORE stores the result in Sig.  SIGMA_LAMBDA goes on with the Lambda of the
-// level below for the same link (lambda_link: its Uprev is this level's U, whose link is
-// at hand, and Sigma the result in registers), with that level's field, tape and Lambda
-// buffer in next (not the Lambda buffer this launch reads: other lanes still read their
-// neighbours' entries there); the same operations as the two launches, without the store
-// and load of Sigma between them.
+// level below for the same link, with that level's tape and Lambda buffer in next (not the
+// Lambda buffer this launch reads: other lanes still read their neighbours' entries there).
 // SIGMA_KICK (the last level of the recursion inside a metadynamics momentum update): the
 // result is the bias force at level 0, and instead of storing it the kernel applies
 // UpdateMomenta to the link, P += a Algebra(st U^+) + bf * force, with the staple it
@@ -399,7 +405,7 @@ __device__ __forceinline__ void body_lambda(const double2* __restrict__ U, const
 enum SigmaMode { SIGMA_STORE = 0, SIGMA_KICK = 1, SIGMA_LAMBDA = 2 };
 template <int MODE>
 __device__ __forceinline__ void body_sigma_all(const double2* __restrict__ U, double2* __restrict__ Sig,
-                                               const double2* __restrict__ T, const double2* __restrict__ Lam,
+                                               const double2* __restrict__ Lam,
                                                const Geom& g, const LinkMap& m, int b, double rho, double2* lds,
                                                const MomentumKick& kick, const SigmaNext& next)
 {
@@ -412,31 +418,39 @@ __device__ __forceinline__ void body_sigma_all(const double2* __restrict__ U, do
     park_store(st_slot, n, m3_zero());
     const int q = par ^ 1;
     const int smu = up(g, s, pick4(c, mu), mu);
+    auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+    Raw6 rb;
+    Raw4 rl;
+    int nu = mu == 0 ? 1 : 0, cnu = pick4(c, nu), snu = up(g, s, cnu, nu);
+    ld_raw(U, g, snu, mu, q, rb);
+    ld_raw4(Lam, g, snu, mu, q, rl);
 #pragma unroll 1
     for (int k = 0; k < 3; ++k) {
-        const int nu = k < mu ? k : k + 1;
-        const int cnu = pick4(c, nu);
-        const int snu = up(g, s, cnu, nu), snd = dn(g, s, cnu, nu);
+        const int snd = dn(g, s, cnu, nu);
         const int smu_nd = dn(g, smu, cnu, nu);
         {
             const M3 a = ldu(U, g, s, nu, par);
-            const M3 b = ldu(U, g, snu, mu, q);
             const M3 cc = ldu(U, g, smu, nu, q);
+            const M3 b = su3_of(rb);
+            M3 K = m3_zero();
+            mul_tri_acc<false, 1>(K, dag(b), her_of(rl));
             M3 t = mul_nd_r01(mul_r01(a, b), cc);   // staple, upper term
             third_row(t);
             park_acc<1>(st_slot, n, t);
-            M3 K = m3_zero();
-            mul_tri_acc<false, 1>(K, dag(b), ld_her8_tri(Lam, g, snu, mu, q));
             M3 X = mul_nd(mul(cc, K), a);
+            fence();
+            ld_raw(U, g, snd, mu, q, rb);            // e and its Lambda for the lower half
+            ld_raw4(Lam, g, snd, mu, q, rl);
+            fence();
             t = dag(t);
             mul_tri_acc<false, 1>(X, t, ld_her8_tri(Lam, g, s, nu, par));
             tri_mul_acc<false, -1>(X, ld_her8_tri(Lam, g, smu, nu, q), t);
             park_acc<1>(fs_slot, n, X);
         }
         {
-            const M3 e = ldu(U, g, snd, mu, q);
             const M3 f = ldu(U, g, smu_nd, nu, par);
             const M3 d = ldu(U, g, snd, nu, q);
+            const M3 e = su3_of(rb);
             M3 t = mul_r01(e, f);
             third_row(t);
             t = mul_dn_r01(d, t);                   // staple, lower term
@@ -444,29 +458,42 @@ __device__ __forceinline__ void body_sigma_all(const double2* __restrict__ U, do
             park_acc<1>(st_slot, n, t);
             const M3 ed = dag(e);
             M3 K = m3_zero();
-            mul_tri_acc<false, 1>(K, ed, ld_her8_tri(Lam, g, snd, mu, q) - ld_her8_tri(Lam, g, snd, nu, q));
+            mul_tri_acc<false, 1>(K, ed, her_of(rl) - ld_her8_tri(Lam, g, snd, nu, q));
             tri_mul_acc<false, 1>(K, ld_her8_tri(Lam, g, smu_nd, nu, par), ed);
+            fence();
+            // the next direction's b and its Lambda; after the last one the link's own
+            if (k < 2) {
+                nu = k + 1 < mu ? k + 1 : k + 2;
+                cnu = pick4(c, nu);
+                snu = up(g, s, cnu, nu);
+            }
+            const int sn = k < 2 ? snu : s, pn = k < 2 ? q : par;
+            ld_raw(U, g, sn, mu, pn, rb);
+            ld_raw4(Lam, g, sn, mu, pn, rl);
+            fence();
             park_acc<1>(fs_slot, n, mul(mul_dn(f, K), d));
         }
     }
-    M3 cl = m3_zero();   // st^+ Lambda
-    mul_tri_acc<false, 1>(cl, dag(park_load(st_slot, n)), ld_her8_tri(Lam, g, s, mu, par));
-    const M3 fs = park_load(fs_slot, n);
-    M3 inner = mul(ld(Sig, g, s, mu, par), exp_her(ld_her8_tri(T, g, s, mu, par)));
+    Raw4 y;
+    ld_ah8(Sig, g, s, mu, par, y);
+    M3 p;
+    Raw4 tape;
+    if (MODE == SIGMA_LAMBDA) ld_raw4(next.T, g, s, mu, par, tape);
+    if (MODE == SIGMA_KICK) p = ld(kick.P, g, s, mu, par);
+    fence();
+    M3 cl = m3_zero();   // st^+ Lambda - the six-term sum
+    mul_tri_acc<false, 1>(cl, dag(park_load(st_slot, n)), her_of(rl));
+    cl = sub(cl, park_load(fs_slot, n));
+    const M3 L = su3_of(rb);
 #pragma unroll
-    for (int e = 0; e < 9; ++e) {
-        cd d = cl.m[e] - fs.m[e];
-        inner.m[e] += cd{-rho * d.im, rho * d.re};
-    }
-    const M3 L = ldu(U, g, s, mu, par);
-    const M3 sig = algebra(mul(L, inner));
+    for (int e = 0; e < 9; ++e) cl.m[e] = cd{-rho * cl.m[e].im, rho * cl.m[e].re};
+    const M3 sig = add_ah(algebra(mul(L, cl)), her_of(y));
     if (MODE == SIGMA_STORE) {
         st_link(Sig, g, s, mu, par, sig);
     } else if (MODE == SIGMA_LAMBDA) {
-        lambda_link(next.U, L, sig, Sig, next.T, next.Lam, g, s, mu, par);
+        lambda_link(sig, her_of(tape), Sig, next.Lam, g, s, mu, par);
     } else {
         const M3 A = algebra(mul_nd(park_load(st_slot, n), L));
-        M3 p = ld(kick.P, g, s, mu, par);
 #pragma unroll
         for (int e = 0; e < 9; ++e) p.m[e] += kick.a * A.m[e] + kick.bf * sig.m[e];
         st_link(kick.P, g, s, mu, par, p);

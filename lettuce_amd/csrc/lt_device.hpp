@@ -522,9 +522,9 @@ __device__ __forceinline__ ExpCoeffs exp_series(double c0, double c1)
     exp_terms<2, K>(c0, c1, 0.0, 0.0, 1.0, s0, f1, f2);
     return ExpCoeffs{cd{fma(c0, s0.re, 1.0), c0 * s0.im}, f1, f2};
 }
-// f1, f2 and the derivatives b1j = df_j/dc1, b2j = df_j/dc0 (the b_ij of Morningstar-Peardon)
+// f0, f1, f2 and the derivatives b1j = df_j/dc1, b2j = df_j/dc0 (the b_ij of Morningstar-Peardon)
 struct ExpDeriv {
-    cd f1, f2, b10, b11, b12, b20, b21, b22;
+    cd f0, f1, f2, b10, b11, b12, b20, b21, b22;
 };
 // sequences at term k: G_{k-2}, G_{k-1}, G_k and H_{k-3} .. H_k
 struct ExpSeq {
@@ -557,6 +557,7 @@ __device__ __forceinline__ void exp_series_deriv(double c0, double c1, ExpDeriv&
     ExpSums s{};
     s.f1 = cd{0.0, 1.0};
     exp_terms_deriv<2, K>(c0, c1, ExpSeq{0.0, 0.0, 1.0, 0.0, 0.0, 0.0, 0.0}, s);
+    d.f0 = cd{fma(c0, s.s0.re, 1.0), c0 * s.s0.im};
     d.f1 = s.f1;
     d.f2 = s.f2;
     d.b10 = c0 * s.h0;
@@ -986,12 +987,9 @@ __device__ __forceinline__ double her_det(const Tri& q)
                  n12 = q.r12.re * q.r12.re + q.r12.im * q.r12.im;
     return q.d0 * q.d1 * q.d2 - q.d0 * n12 - q.d1 * n02 - q.d2 * n01 + 2.0 * (t.re * q.r02.re + t.im * q.r02.im);
 }
-// exp(iQ) for Q hermitian traceless: Q^2 from its six independent entries, c0 = det Q and
-// c1 = tr(Q^2)/2 from Q's entries
-__device__ __forceinline__ M3 exp_her(const Tri& q)
+// f0 + f1 Q + f2 Q^2, s = Q^2
+__device__ __forceinline__ M3 her_poly(cd f0, cd f1, cd f2, const Tri& q, const Tri& s)
 {
-    const Tri s = her_square(q);
-    const auto [f0, f1, f2] = exp_coeffs(her_det(q), 0.5 * (s.d0 + s.d1 + s.d2));
     M3 r;
     r.m[0] = f0 + q.d0 * f1 + s.d0 * f2;
     r.m[4] = f0 + q.d1 * f1 + s.d1 * f2;
@@ -1003,6 +1001,14 @@ __device__ __forceinline__ M3 exp_her(const Tri& q)
     r.m[6] = f1 * conj(q.r02) + f2 * conj(s.r02);
     r.m[7] = f1 * conj(q.r12) + f2 * conj(s.r12);
     return r;
+}
+// exp(iQ) for Q hermitian traceless: Q^2 from its six independent entries, c0 = det Q and
+// c1 = tr(Q^2)/2 from Q's entries
+__device__ __forceinline__ M3 exp_her(const Tri& q)
+{
+    const Tri s = her_square(q);
+    const auto [f0, f1, f2] = exp_coeffs(her_det(q), 0.5 * (s.d0 + s.d1 + s.d2));
+    return her_poly(f0, f1, f2, q, s);
 }
 // exp(c Z) for Z anti-hermitian traceless in the 8-real form (the flow's Z): exp(iQ) with
 // Q = -i c Z hermitian traceless
@@ -1081,6 +1087,71 @@ __device__ __forceinline__ void tri_mul_acc(M3& C, const Tri& R, const M3& A)
         cmul_acc<LO>(C.m[6 + j], conj(R.r12), y);
         diag_acc<AH, SG>(C.m[6 + j], z, R.d2);
     }
+}
+
+// One 8-real algebra or hermitian entry as loaded
+struct Raw4 {
+    double2 v[4];
+};
+__device__ __forceinline__ void ld_raw4(const double2* __restrict__ Z, const Geom& g, int s, int mu, int par, Raw4& r)
+{
+    const double2* p = Z + slot_base(g, mu * 2 + par, 4, cbi(g, s));
+#pragma unroll
+    for (int c = 0; c < 4; ++c) r.v[c] = p[(size_t)c * slot_stride(g)];
+}
+__device__ __forceinline__ Tri her_of(const Raw4& r)
+{
+    return Tri{r.v[0].x, r.v[0].y, -(r.v[0].x + r.v[0].y), cd{r.v[1].x, r.v[1].y}, cd{r.v[2].x, r.v[2].y},
+               cd{r.v[3].x, r.v[3].y}};
+}
+__device__ __forceinline__ Tri ah_tri(const M3& a) { return Tri{a.m[0].im, a.m[4].im, a.m[8].im, a.m[1], a.m[2], a.m[5]}; }
+// A + R, R anti-hermitian
+__device__ __forceinline__ M3 add_ah(M3 a, const Tri& r)
+{
+    a.m[0].im += r.d0;
+    a.m[4].im += r.d1;
+    a.m[8].im += r.d2;
+    a.m[1] += r.r01;
+    a.m[2] += r.r02;
+    a.m[5] += r.r12;
+    a.m[3] += cd{-r.r01.re, r.r01.im};
+    a.m[6] += cd{-r.r02.re, r.r02.im};
+    a.m[7] += cd{-r.r12.re, r.r12.im};
+    return a;
+}
+// A B where the product is known to be anti-hermitian and traceless
+__device__ __forceinline__ Tri mul_ah(const M3& A, const M3& B)
+{
+    auto entry = [&](int i, int j) {
+        cd z = A.m[3 * i] * B.m[j];
+        cmul_acc<1>(z, A.m[3 * i + 1], B.m[3 + j]);
+        cmul_acc<1>(z, A.m[3 * i + 2], B.m[6 + j]);
+        return z;
+    };
+    auto diag = [&](int i) {
+        double d = 0.0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) d = fma(A.m[3 * i + k].re, B.m[3 * k + i].im, fma(A.m[3 * i + k].im, B.m[3 * k + i].re, d));
+        return d;
+    };
+    const double d0 = diag(0), d1 = diag(1);
+    return Tri{d0, d1, -(d0 + d1), entry(0, 1), entry(0, 2), entry(1, 2)};
+}
+// An anti-hermitian traceless field in 8 reals in the first four of the nine slots of a link
+// field's entry
+__device__ __forceinline__ void ld_ah8(const double2* __restrict__ S, const Geom& g, int s, int mu, int par, Raw4& r)
+{
+    const double2* p = S + slot_base(g, mu * 2 + par, 9, cbi(g, s));
+#pragma unroll
+    for (int c = 0; c < 4; ++c) r.v[c] = p[(size_t)c * slot_stride(g)];
+}
+__device__ __forceinline__ void st_ah8(double2* __restrict__ S, const Geom& g, int s, int mu, int par, const Tri& y)
+{
+    double2* p = S + slot_base(g, mu * 2 + par, 9, cbi(g, s));
+    p[0] = make_double2(y.d0, y.d1);
+    p[slot_stride(g)] = make_double2(y.r01.re, y.r01.im);
+    p[(size_t)2 * slot_stride(g)] = make_double2(y.r02.re, y.r02.im);
+    p[(size_t)3 * slot_stride(g)] = make_double2(y.r12.re, y.r12.im);
 }
 
 // complex-double offset of a replica's 8-real field given its link-field offset
@@ -1610,7 +1681,7 @@ __device__ __forceinline__ void exp_deriv_closed(const ExpC& e, ExpDeriv& out)
             b22 = bd * (r12 - (3.0 * u) * r22 - (24.0 * u) * f2);
         }
     }
-    out = ExpDeriv{f1, f2, b10, b11, b12, b20, b21, b22};
+    out = ExpDeriv{f0, f1, f2, b10, b11, b12, b20, b21, b22};
 }
 // f1, f2 and the b_ij of exp(iQ) from c0 = det Q, c1 = tr(Q^2)/2
 __device__ __forceinline__ void exp_deriv(double c0, double c1, ExpDeriv& d)

@@ -322,7 +322,7 @@ double cv_forward(lt_cv cv, lt_field U)
 
 // CV adjoint into F: dvdq * dQ/dU through the clover derivative and n recursions.
 // With kick (n > 0 only) the last recursion step applies the momentum update to
-// kick->P instead of storing the level-0 force, and F is left holding level 1's.
+// kick->P instead of storing the level-0 force, and F is left as scratch.
 void cv_backward(lt_cv cv, double dvdq, double2* F, const lt::MomentumKick* kick = nullptr)
 {
     const int n = cv->n_levels;
@@ -332,7 +332,7 @@ void cv_backward(lt_cv cv, double dvdq, double2* F, const lt::MomentumKick* kick
             return;
         }
         // the clover derivative goes on with the Lambda of the top level
-        const lt::SigmaNext top{cv->levels[n - 1], cv->tapes[n - 1], cv->lambda[0]};
+        const lt::SigmaNext top{cv->tapes[n - 1], cv->lambda[0]};
         lt::k_clover_deriv(cv->ctx, cv->g, cv->map, cv->levels[n], cv->clover, F, dvdq, &top);
         lt::k_stout_recursion_run(
             cv->ctx, cv->g, cv->map, [&](int j) -> const double2* { return cv->levels[j]; },
