@@ -405,7 +405,7 @@ int lt_batch_results(lt_batch b, double *dH, int *accepted, double *cv, int *lab
  * kernels on scratch copies and keeps the fastest; results are bit-identical for
  * every tile.  cache_path (may be NULL) is a JSON file of tuned tiles keyed by GPU
  * architecture, extents and kernel family; a cached entry is applied without timing. */
-#define LT_TUNE_SWEEP 1   /* heatbath / overrelaxation colour kernels */
+#define LT_TUNE_SWEEP 1   /* the plaquette pass of an update (its colour launches have a fixed shape) */
 #define LT_TUNE_FLOW  2   /* stout / Wilson-flow stage kernels */
 int lt_autotune_field(lt_field f, int family, const char *cache_path, int tile_out[4], double *best_ms);
 /* per distinct replica extent: the tile of the batched MetaD force kernels */

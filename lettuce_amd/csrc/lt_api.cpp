@@ -76,7 +76,6 @@ bool make_linkmap(const Geom& g, int tt, int tx, int ty, int tz, LinkMap& m)
 #if LT_YCHUNK > 0
     if (m.N[2] % LT_YCHUNK == 0) m.yc = LT_YCHUNK;
 #endif
-    // the colour sweeps walk all y tiles of an x step in one chunk
     m.ycs = m.N[2];
     m.xr = LT_XCD_REMAP;
     finish_map(m);

@@ -517,7 +517,7 @@ int lt_batch_autotune(lt_batch b, const char* cache_path)
                     if (lt::map_blocks(c) == nb) cands.push_back(c);
                 if (cands.empty()) cands.push_back(cur);
                 best = lt::tune(b->ctx, cands, cur, run, ms, 2);
-                best = lt::tune(b->ctx, lt::order_candidates(best, false), best, run, ms, 2);
+                best = lt::tune(b->ctx, lt::order_candidates(best), best, run, ms, 2);
                 lt::store_tile(cache_path, key, best, ms);
             }
             apply(best);

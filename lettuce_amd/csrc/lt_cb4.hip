@@ -20,47 +20,30 @@ namespace lt {
 
 namespace {
 
-constexpr int BS = LT_LINK_BS;
 constexpr int RBS = 256;
 
-// One thread per link of the class (cb4_site), consecutive threads along z.
-// Colours 1 and 3 walk the blocks backwards (xcd_block_dir): consecutive colour
-// launches then start where the previous one ended.
-template <bool HEATBATH>
-__global__ void LT_LINK_KERNEL sweep_cb4_kernel(double2* __restrict__ U, Geom g, int mu, int colour,
-                                                 double prefactor, uint64_t seed, uint64_t counter)
-{
-    int c[4], s;
-    if (!cb4_site(g, mu, colour, xcd_block_dir(blockIdx.x, gridDim.x, colour & 1) * BS + threadIdx.x, c, s)) return;
-    update_link<HEATBATH>(U, g, s, c, mu, parity_of(c), prefactor, seed, counter);
-}
-
-// heatbath of a captured update: Philox counter state[0] + k from device memory
-__global__ void LT_LINK_KERNEL hb_cb4_graph_kernel(double2* __restrict__ U, Geom g, int mu, int colour, double prefactor,
-                                                   uint64_t seed, const uint64_t* __restrict__ state, int k)
-{
-    int c[4], s;
-    if (!cb4_site(g, mu, colour, xcd_block_dir(blockIdx.x, gridDim.x, colour & 1) * BS + threadIdx.x, c, s)) return;
-    update_link<true>(U, g, s, c, mu, parity_of(c), prefactor, seed, state[0] + (uint64_t)k);
-}
-
-// Six wavefronts per 64 links (update_links_split), three waves per SIMD.  Rectangle staple:
-// one lane per link with the sum parked in LDS ran about 9500 FP64 instructions in a row at
-// two waves per SIMD, and a 24^4 launch was 1296 waves on 1024 SIMDs: 186 us per
-// overrelaxation launch there, 322 us at 32^4; now 85 and 207 us (heatbath 195 -> 94 us at
-// 24^4).  What bounds it now is the latency of the twelve link loads of a part, about half
-// of whose lines miss the L2, at one load in flight ahead of the products.
-template <bool HEATBATH, int KIND>
-__global__ void __launch_bounds__(SPLIT_BS) __attribute__((amdgpu_waves_per_eu(3)))
-split_cb4_kernel(double2* __restrict__ U, Geom g, int mu, int colour, double prefactor, uint64_t seed, uint64_t counter,
+// Colours 1 and 3 walk the blocks backwards (xcd_block_dir): consecutive colour launches then
+// start where the previous one ended.  In a captured update the Philox counter is state[0] + k
+// from device memory.
+// Wilson staple, between events, against one lane per link: overrelaxation 8^4 12.1 -> 8.3 us,
+// 16^4 12.7 -> 9.2, 28^4 76 -> 51.8, 32^4 77.3 -> 75.2; heatbath 8^4 21.7 -> 11.7, 16^4 21.3 ->
+// 13.5, 28^4 89 -> 63.3, 32^4 89 -> 80.  Small ones are bound by the latency of one link, large
+// ones by the memory behind the L2.
+// Rectangle staple: one lane per link with the sum parked in LDS ran about 9500 FP64
+// instructions in a row at two waves per SIMD, 186 us per overrelaxation launch at 24^4 and 322
+// us at 32^4; now 81.6 and 199 us (heatbath 195 -> 92 us at 24^4).  About half of its lines miss
+// the L2: 385 MB a launch at 24^4, 53 us at the rate at which the memory-side cache reads.
+template <bool HEATBATH, int KIND, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(split_eu(HEATBATH, KIND, WAVES))))
+sweep_cb4_kernel(double2* __restrict__ U, Geom g, int mu, int colour, double prefactor, uint64_t seed, uint64_t counter,
                  const uint64_t* __restrict__ state, int k, double c_plaq, double c_rect, SplitMap map)
 {
-    __shared__ SplitShared<HEATBATH> sh;
+    __shared__ SplitShared<HEATBATH, WAVES> sh;
     if (HEATBATH && state) counter = state[0] + (uint64_t)k;
     int c[4], s = 0;
     const int i = split_index(map, xcd_block_dir(blockIdx.x, gridDim.x, colour & 1));
     const bool on = i >= 0 && cb4_site(g, mu, colour, i, c, s);
-    update_links_split<HEATBATH, KIND>(U, g, mu, on, s, c, prefactor, seed, counter, c_plaq, c_rect, sh);
+    update_links_split<HEATBATH, KIND, WAVES>(U, g, mu, on, s, c, prefactor, seed, counter, c_plaq, c_rect, sh);
 }
 
 // PlaquetteSum block partials of a captured four-colour update (the field is in the
@@ -102,55 +85,52 @@ void k_cb_layout(lt_field u, int to_split)
 
 namespace {
 
-// Whether a Wilson colour launch uses the split kernel.  Rows of 32 z (or a multiple) give a
-// class whole 128-byte lines per row, and one lane per link is faster there once the launch
-// fills the GPU (32^4: overrelaxation 77 against 90 us, heatbath 90 against 102 us; 16^2 x
-// 32^2: 22.0 against 23.4 us).  Shorter rows leave half lines, which the six wavefronts of a
-// block share in the L1 (28^4: 76 -> 58 us, heatbath 89 -> 67 us), and launches below two
-// blocks per compute unit are bound by the latency of one link (8^4: 12.1 -> 8.3 us,
-// heatbath 21.7 -> 11.6 us; 16^4: 12.7 -> 9.6 and 21.3 -> 13.7 us).
-bool split_launches(const Geom& g) { return g.L[3] % 32 != 0 || g.V / 4 <= 32768; }
-
-template <bool HEATBATH, int KIND>
-void split_launch(lt_field u, const char* name, int mu, int colour, double prefactor, uint64_t counter,
+template <bool HEATBATH, int KIND, int WAVES>
+void colour_waves(lt_field u, const char* name, int mu, int colour, double prefactor, uint64_t counter,
                   const uint64_t* state, int k, double c_plaq, double c_rect)
 {
     const SplitMap m = split_map(u->g, 4);
-    launch(u->ctx, name, split_cb4_kernel<HEATBATH, KIND>, dim3(split_blocks(u->g, m)), dim3(SPLIT_BS), 0, u->d, u->g, mu,
-           colour, prefactor, u->seed, counter, state, k, c_plaq, c_rect, m);
+    launch(u->ctx, name, sweep_cb4_kernel<HEATBATH, KIND, WAVES>, dim3(split_blocks(u->g, m)), dim3(64 * WAVES), 0, u->d,
+           u->g, mu, colour, prefactor, u->seed, counter, state, k, c_plaq, c_rect, m);
+}
+
+// Wavefronts per block.  Three, of which four blocks fit a compute unit, wherever the parts are
+// of one wavefront's size: the heatbath (20^4 24.8 -> 22.6 us, 24^4 37.8 -> 37.2 against six).
+// Overrelaxation takes three where rows of a multiple of 32 z give a class whole 128-byte lines
+// per row (32^4 75.2 against 79.8 us with six, 16^2 x 32^2 20.8 and 21.6) and six where rows
+// leave half lines, which the six wavefronts of a block then share in the L1 (24^4 30.0 us
+// against 34.0 with three, 28^4 51.8 and 59.7, 48 x 24^3 51 and 62).  The rectangle staple's
+// parts spill with two sides in a wavefront.
+template <bool HEATBATH, int KIND>
+void colour_launch(lt_field u, const char* name, int mu, int colour, double prefactor, uint64_t counter,
+                   const uint64_t* state, int k, double c_plaq, double c_rect)
+{
+    if constexpr (KIND == SPLIT_RECT)
+        colour_waves<HEATBATH, KIND, 6>(u, name, mu, colour, prefactor, counter, state, k, c_plaq, c_rect);
+    else if (HEATBATH || u->g.L[3] % 32 == 0)
+        colour_waves<HEATBATH, KIND, 3>(u, name, mu, colour, prefactor, counter, state, k, c_plaq, c_rect);
+    else
+        colour_waves<false, KIND, 6>(u, name, mu, colour, prefactor, counter, state, k, c_plaq, c_rect);
 }
 
 }  // namespace
 
 void k_cb4_colour(lt_field u, bool heatbath, int mu, int colour, double prefactor, uint64_t counter, const char* name)
 {
-    const dim3 grid(nblocks(u->g.V / 4, BS)), block(BS);
-    const bool split = split_launches(u->g);
-    if (heatbath && split)
-        split_launch<true, SPLIT_WILSON>(u, name, mu, colour, prefactor, counter, nullptr, 0, 1.0, 0.0);
-    else if (split)
-        split_launch<false, SPLIT_WILSON>(u, name, mu, colour, prefactor, counter, nullptr, 0, 1.0, 0.0);
-    else if (heatbath)
-        launch(u->ctx, name, sweep_cb4_kernel<true>, grid, block, 0, u->d, u->g, mu, colour, prefactor, u->seed, counter);
-    else
-        launch(u->ctx, name, sweep_cb4_kernel<false>, grid, block, 0, u->d, u->g, mu, colour, prefactor, u->seed,
-               counter);
+    auto* f = heatbath ? colour_launch<true, SPLIT_WILSON> : colour_launch<false, SPLIT_WILSON>;
+    f(u, name, mu, colour, prefactor, counter, nullptr, 0, 1.0, 0.0);
 }
 
 void k_cb4_colour_graph_hb(lt_field u, int mu, int colour, double prefactor, const uint64_t* state, int k)
 {
-    if (split_launches(u->g))
-        split_launch<true, SPLIT_WILSON>(u, "hb_cb4", mu, colour, prefactor, 0, state, k, 1.0, 0.0);
-    else
-        launch(u->ctx, "hb_cb4", hb_cb4_graph_kernel, dim3(nblocks(u->g.V / 4, BS)), dim3(BS), 0, u->d, u->g, mu, colour,
-               prefactor, u->seed, state, k);
+    colour_launch<true, SPLIT_WILSON>(u, "hb_cb4", mu, colour, prefactor, 0, state, k, 1.0, 0.0);
 }
 
 void k_cb4_colour_action(lt_field u, bool heatbath, int mu, int colour, double prefactor, uint64_t counter,
                          double c_plaq, double c_rect, const char* name)
 {
-    auto* f = heatbath ? (c_rect != 0.0 ? split_launch<true, SPLIT_RECT> : split_launch<true, SPLIT_SCALED>)
-                       : (c_rect != 0.0 ? split_launch<false, SPLIT_RECT> : split_launch<false, SPLIT_SCALED>);
+    auto* f = heatbath ? (c_rect != 0.0 ? colour_launch<true, SPLIT_RECT> : colour_launch<true, SPLIT_SCALED>)
+                       : (c_rect != 0.0 ? colour_launch<false, SPLIT_RECT> : colour_launch<false, SPLIT_SCALED>);
     f(u, name, mu, colour, prefactor, counter, nullptr, 0, c_plaq, c_rect);
 }
 

@@ -1258,7 +1258,7 @@ struct LinkMap {
     int tc;       // t tiles per chunk (divides N[0])
     int yc;       // y tiles per chunk (divides N[2]) of the Jacobi kernels (flow, stout, MetaD)
     int lin;      // linear map: block b covers checkerboard sites [b * nthreads, (b + 1) * nthreads)
-    int ycs;      // y tiles per chunk of the colour sweeps
+    int ycs;      // kept with a tuned map's file entry; orders nothing
     int xr;       // spread the block index over the XCDs (xcd_block)
     // divisions of map_site_b, from the numbers above (finish_map)
     Div dtx, dty, dtz, dtc, dnz, dyc, dnx, dny;
@@ -1287,13 +1287,8 @@ struct SplitMap {
     Div dtc, dper;   // by tc, and by the blocks of a chunk
 };
 
-// Block index of a link kernel in its map's order: spread over the XCDs when m.xr is
-// set, walked backwards when rev is set.
-__device__ __forceinline__ int link_block(const LinkMap& m, int b, int nb, int rev = 0)
-{
-    if (m.xr) return xcd_block_dir(b, nb, rev);
-    return rev ? nb - 1 - b : b;
-}
+// Block index of a link kernel in its map's order: spread over the XCDs when m.xr is set.
+__device__ __forceinline__ int link_block(const LinkMap& m, int b, int nb) { return m.xr ? xcd_block(b, nb) : b; }
 
 // tile order, fastest first: t within its chunk, z, y within its chunk, x, y chunk, t chunk
 __device__ __forceinline__ int site_of_cb(const Geom& g, int cb, int par, int c[4]);
@@ -1330,10 +1325,6 @@ __device__ __forceinline__ bool map_site_b(const Geom& g, const LinkMap& m, int 
 __device__ __forceinline__ bool map_site(const Geom& g, const LinkMap& m, int par, int c[4], int& s)
 {
     return map_site_b(g, m, link_block(m, blockIdx.x, gridDim.x), par, c, s);
-}
-__device__ __forceinline__ bool map_site_dir(const Geom& g, const LinkMap& m, int par, int rev, int c[4], int& s)
-{
-    return map_site_b(g, m, link_block(m, blockIdx.x, gridDim.x, rev), par, c, s);
 }
 
 // Jacobi kernels over all links: the 8 (mu, parity) classes of one tile are

@@ -325,7 +325,7 @@ void k_or_sweep_action(lt_field u, int n, double c_plaq, double c_rect);
 void k_heatbath_sweep_action(lt_field u, double beta, int n, double c_plaq, double c_rect);
 void k_observables(lt_field u, double* host_out);
 // sum over sites and planes of Re tr P, the planes of a site spread over its links (the HMC
-// Hamiltonian keeps k_plaquette_sum, one site per lane, which the replica batch repeats)
+// Hamiltonian keeps k_plaquette_sum, a plane pair per lane, which the replica batch repeats)
 double k_plaquette_planes(lt_field u);
 // per-site clover charge density (V doubles, lexicographic order) into host memory
 void k_topcharge_density(lt_field u, double* host_q);

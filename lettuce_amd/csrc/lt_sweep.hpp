@@ -2,7 +2,7 @@
 // two-colour kernels (lt_update.hip) and the four-colour kernels (lt_cb4.hip):
 // SU(2)-subgroup extraction and embedding, overrelaxation, the Kennedy-Pendleton /
 // Fabricius-Haan heatbath sampler with Philox draws, the Checkerboard4 site map and
-// the link update with the Wilson or the rectangular staple.
+// the link update, several wavefronts per 64 links, with the Wilson or the rectangular staple.
 #pragma once
 
 #include "lt_device.hpp"
@@ -99,31 +99,10 @@ __device__ __forceinline__ SU2 kp_element(SU2 V, double lambda_sq, double cos_th
     SU2 Vd{conj(V.e11), -V.e12};
     return su2_mul(X, Vd);
 }
-__device__ __forceinline__ SU2 kp_finish(SU2 V, double lambda_sq, uint64_t seed, uint32_t site, uint32_t sub,
-                                         uint32_t mu, uint64_t counter)
-{
-    double ct, cp, sp;
-    kp_direction(seed, site, sub, mu, counter, ct, cp, sp);
-    return kp_element(V, lambda_sq, ct, cp, sp);
-}
-
 // Kennedy-Pendleton / Fabricius-Haan SU(2) sampler in the reference's draw order: the
 // first accepted attempt k = 0, 1, ..., max_iter; after max_iter+1 rejected attempts
-// the identity is returned.
+// the identity is taken.
 constexpr int KP_MAX_ITER = 10;
-__device__ __forceinline__ SU2 heatbath_su2(SU2 A, double prefactor, uint64_t seed, uint32_t site, uint32_t sub,
-                                            uint32_t mu, uint64_t counter)
-{
-    const double an = 1.0 / sqrt(su2_det(A));
-    SU2 V{an * A.e11, an * A.e12};
-    const double coef = -0.25 * prefactor * an;
-    double lambda_sq = 0.0;
-    for (int k = 0;; ++k) {
-        if (k > KP_MAX_ITER) return SU2{cd{1.0, 0.0}, cd{0.0, 0.0}};
-        if (kp_attempt(seed, site, sub, mu, counter, k, coef, lambda_sq)) break;
-    }
-    return kp_finish(V, lambda_sq, seed, site, sub, mu, counter);
-}
 
 // Site i in [0, V/4) of colour k of direction mu under Checkerboard4, where the colour
 // is (t + x + y + z + x_mu) mod 4 (iterators.hpp:141-169; extents divisible by 4):
@@ -154,42 +133,6 @@ __device__ __forceinline__ bool cb4_site(const Geom& g, int mu, int k, int i, in
     }
     s = ((c[0] * g.L[1] + c[1]) * g.L[2] + c[2]) * g.L[3] + c[3];
     return true;
-}
-
-// overrelaxation with the software-pipelined staple (the heatbath's sampler
-// leaves no registers for it)
-#ifndef LT_OR_PIPE
-#define LT_OR_PIPE 1
-#endif
-template <bool HEATBATH>
-__device__ __forceinline__ void update_link(double2* __restrict__ U, const Geom& g, int s, const int c[4], int mu,
-                                            int par, double prefactor, uint64_t seed, uint64_t counter)
-{
-    M3 st, L;
-    if (LT_OR_PIPE && !HEATBATH) {
-        Raw6 own;
-        st = staple_pipelined(U, g, s, c, mu, par, own);
-        L = su3_of(own);
-    } else {
-        st = staple(U, g, s, c, mu);
-        L = ldu(U, g, s, mu, par);
-    }
-#pragma unroll
-    for (int sub = 0; sub < 3; ++sub) {
-        const int i = sub == 2 ? 1 : 0;
-        const int j = sub == 0 ? 1 : 2;
-        SU2 A = extract(L, st, i, j);
-        SU2 X;
-        if (HEATBATH)
-            X = heatbath_su2(A, prefactor, seed, (uint32_t)s, (uint32_t)sub, (uint32_t)mu, counter);
-        else
-            X = overrelax(A);
-        embed_mul(L, X, i, j);
-    }
-    gram_schmidt(L);
-    // the updated link is not read again in this launch: a streaming store keeps the
-    // L2 for the neighbour links (-0.3 % overrelaxation, -0.8 % heatbath launch at 32^4)
-    stu_stream(U, g, s, mu, par, L);
 }
 
 // The part of Rectangular<R>::Staple (rectangular_action.hpp:103-242) of link (x, mu) that
@@ -288,19 +231,29 @@ __device__ __forceinline__ M3 staple_action(const double2* __restrict__ U, const
     return st;
 }
 
-// A colour launch with the staple split over wavefronts.  A block of six wavefronts updates
-// 64 links: wavefront w forms the part of the staple on side w & 1 of the (w >> 1)-th
-// direction nu != mu; the parts are added through LDS and the first wavefront applies the
-// SU(2) steps.  The heatbath's random numbers do not depend on the link: wavefront w also
-// draws attempt w / 3 of subgroup w % 3, the first three the directions, while the links of
-// their parts are on the way; only the rare third attempts are drawn in the SU(2) steps.
+// A colour launch with the staple split over wavefronts.  A block of WAVES wavefronts updates
+// 64 links: wavefront w forms the part of the staple of the w-th direction nu != mu (WAVES = 3)
+// or of side w & 1 of the (w >> 1)-th one (6); the parts are added through LDS and the first
+// wavefront applies the SU(2) steps.  The heatbath's random numbers do not depend on the link:
+// the wavefronts also draw the first two attempts and the direction of the three subgroups
+// while the links of their parts are on the way; only the rare third attempts are drawn in the
+// SU(2) steps.  One lane per link holds a whole SIMD's registers at two wavefronts and runs
+// 5000 instructions in a row.
 // The action enters through the staple only (heatbath.hpp:110-129, overrelaxation.hpp:91-116):
 // SPLIT_WILSON, SPLIT_SCALED (c_plaq times the plaquette staple), SPLIT_RECT.
 enum SplitKind { SPLIT_WILSON = 0, SPLIT_SCALED = 1, SPLIT_RECT = 2 };
-constexpr int SPLIT_WAVES = 6, SPLIT_BS = SPLIT_WAVES * SPLIT_LINKS;
-template <bool HEATBATH>
+// Wavefronts per SIMD.  Blocks of six go 2, 2, 1, 1 on the SIMDs of a compute unit, so two of
+// them are resident only where four wavefronts fit a SIMD: overrelaxation with the plaquette
+// staple, 123 registers (four colours at 28^4 55.6 us with 133 registers, 51.8 with 123).  The
+// rectangle staple needs 188 without spills and has one block either way (24^4 84.5 -> 81.6
+// us; its heatbath gains nothing and keeps three).  Blocks of three fill three per SIMD.
+constexpr int split_eu(bool heatbath, int kind, int waves)
+{
+    return heatbath || waves == 3 ? 3 : kind == SPLIT_RECT ? 2 : 4;
+}
+template <bool HEATBATH, int WAVES>
 struct SplitShared {
-    double2 part[27 * SPLIT_LINKS];
+    double2 part[(WAVES == 6 ? 27 : 18) * SPLIT_LINKS];
     double draw[HEATBATH ? 21 * SPLIT_LINKS : 1];   // y, r0 of (subgroup, attempt); cos, cos, sin of the directions
 };
 
@@ -324,24 +277,29 @@ __device__ __forceinline__ M3 staple_wilson_side(const double2* __restrict__ U, 
 }
 
 // on: whether this lane holds a link (s, mu) of the launch
-template <bool HEATBATH, int KIND>
+template <bool HEATBATH, int KIND, int WAVES>
 __device__ __forceinline__ void update_links_split(double2* __restrict__ U, const Geom& g, int mu, bool on, int s,
                                                    const int c[4], double prefactor, uint64_t seed, uint64_t counter,
-                                                   double c_plaq, double c_rect, SplitShared<HEATBATH>& sh)
+                                                   double c_plaq, double c_rect, SplitShared<HEATBATH, WAVES>& sh)
 {
+    static_assert(WAVES == 6 || (WAVES == 3 && KIND != SPLIT_RECT), "no such split");
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
     M3 st = m3_zero();
     int par = 0;
+    auto draw_attempt = [&](int sub, int attempt) {
+        double y, r0;
+        kp_draw(seed, (uint32_t)s, (uint32_t)sub, (uint32_t)mu, counter, attempt, y, r0);
+        const int slot = 2 * (sub + 3 * attempt);
+        sh.draw[slot * SPLIT_LINKS + lane] = y;
+        sh.draw[(slot + 1) * SPLIT_LINKS + lane] = r0;
+    };
     auto draws = [&]() {
         if (HEATBATH) {
-            const uint32_t sub = (uint32_t)(w % 3);
-            double y, r0;
-            kp_draw(seed, (uint32_t)s, sub, (uint32_t)mu, counter, w / 3, y, r0);
-            sh.draw[(2 * w) * SPLIT_LINKS + lane] = y;
-            sh.draw[(2 * w + 1) * SPLIT_LINKS + lane] = r0;
+            draw_attempt(w % 3, w / 3);
+            if (WAVES == 3) draw_attempt(w, 1);
             if (w < 3) {
                 double ct, cp, sp;
-                kp_direction(seed, (uint32_t)s, sub, (uint32_t)mu, counter, ct, cp, sp);
+                kp_direction(seed, (uint32_t)s, (uint32_t)w, (uint32_t)mu, counter, ct, cp, sp);
                 sh.draw[(12 + 3 * w) * SPLIT_LINKS + lane] = ct;
                 sh.draw[(13 + 3 * w) * SPLIT_LINKS + lane] = cp;
                 sh.draw[(14 + 3 * w) * SPLIT_LINKS + lane] = sp;
@@ -350,16 +308,19 @@ __device__ __forceinline__ void update_links_split(double2* __restrict__ U, cons
     };
     if (on) {
         par = parity_of(c);
-        const int nu = (w >> 1) + ((w >> 1) >= mu);
+        const int d = WAVES == 6 ? w >> 1 : w, nu = d + (d >= mu);
         if (KIND == SPLIT_RECT) {
             draws();
             st = (w & 1) ? staple_action_side<false, true>(U, g, s, c, mu, nu, par, c_plaq, c_rect)
                          : staple_action_side<true, true>(U, g, s, c, mu, nu, par, c_plaq, c_rect);
-        } else {
+        } else if (WAVES == 6) {
             st = (w & 1) ? staple_wilson_side<false>(U, g, s, c, mu, nu, par, draws)
                          : staple_wilson_side<true>(U, g, s, c, mu, nu, par, draws);
-            if (KIND == SPLIT_SCALED) st = scale(c_plaq, st);
+        } else {
+            st = staple_wilson_side<true>(U, g, s, c, mu, nu, par, draws);
+            acc(st, staple_wilson_side<false>(U, g, s, c, mu, nu, par, [] {}));
         }
+        if (KIND == SPLIT_SCALED) st = scale(c_plaq, st);
     }
     auto put = [&](int slot) {
 #pragma unroll
@@ -372,19 +333,25 @@ __device__ __forceinline__ void update_links_split(double2* __restrict__ U, cons
             st.m[e] += cd{v.x, v.y};
         }
     };
-    if (w >= 3) put(w - 3);
-    __syncthreads();
-    if (w < 3) add_from(w);
-    if (w == 1 || w == 2) put(w);
+    if (WAVES == 6) {
+        if (w >= 3) put(w - 3);
+        __syncthreads();
+        if (w < 3) add_from(w);
+        if (w == 1 || w == 2) put(w);
+    } else if (w) {
+        put(w - 1);
+    }
     __syncthreads();
     if (w || !on) return;
     M3 L = ldu(U, g, s, mu, par);
-    add_from(1);
-    add_from(2);
+    add_from(WAVES == 6 ? 1 : 0);
+    add_from(WAVES == 6 ? 2 : 1);
 #pragma unroll
     for (int sub = 0; sub < 3; ++sub) {
         const int i = sub == 2 ? 1 : 0;
         const int j = sub == 0 ? 1 : 2;
+        // one subgroup at a time has the registers
+        __builtin_amdgcn_sched_barrier(0);
         const SU2 A = extract(L, st, i, j);
         SU2 X;
         if (HEATBATH) {

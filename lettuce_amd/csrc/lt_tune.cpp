@@ -66,9 +66,8 @@ std::vector<LinkMap> tile_candidates(const Geom& g, int threads)
 }
 
 // Site orders of one block shape: t tiles per chunk (1, or one t-slab per XCD), y tiles
-// per chunk (1, 2 or all) for the family's kernels (Jacobi: yc, colour sweeps: ycs), and
-// the block index spread over the XCDs or not.  Every order gives the same results.
-std::vector<LinkMap> order_candidates(const LinkMap& base, bool sweeps)
+// per chunk (1, 2 or all), and the block index spread over the XCDs or not.  Every order gives the same results.
+std::vector<LinkMap> order_candidates(const LinkMap& base)
 {
     std::vector<LinkMap> out;
     if (base.lin) {   // a linear map only chooses the XCD spread
@@ -89,7 +88,7 @@ std::vector<LinkMap> order_candidates(const LinkMap& base, bool sweeps)
                 LinkMap m = base;
                 m.xr = xr;
                 m.tc = tc;
-                (sweeps ? m.ycs : m.yc) = yc;
+                m.yc = yc;
                 finish_map(m);
                 out.push_back(m);
             }
@@ -111,7 +110,8 @@ std::string tune_key(int device, const Geom& g, const char* family)
 
 // Cache file: one JSON object, "key": [tt, tx, ty, tz, ms, tc, yc, ycs, xr] per entry (tt =
 // tx = ty = 0: a linear map of tz consecutive checkerboard sites per block; tc, yc, ycs, xr:
-// the site order, see order_candidates; entries of five numbers keep the default order).
+// the site order, see order_candidates; ycs belonged to colour kernels on the map and orders
+// nothing now; entries of five numbers keep the default order).
 static std::map<std::string, std::array<double, 9>> read_cache(const char* path)
 {
     std::map<std::string, std::array<double, 9>> m;
@@ -283,12 +283,14 @@ extern "C" int lt_autotune_field(lt_field f, int family, const char* cache_path,
                 // shape; the field's default map is the incumbent
                 const lt::LinkMap d = lt::default_linkmap(f->g);
                 if (family == LT_TUNE_SWEEP) {
+                    // the colour launches have their own block shape and order; the
+                    // plaquette pass of an update runs over the map
                     auto run = [&](const lt::LinkMap& c) {
                         tmp.map = c;
-                        lt::k_or_sweep(&tmp, 1, LT_CB2);
+                        (void)lt::k_plaquette_planes(&tmp);
                     };
                     m = lt::tune(ctx, lt::tile_candidates(f->g, 0), d, run, ms, 3);
-                    m = lt::tune(ctx, lt::order_candidates(m, true), m, run, ms, 3);
+                    m = lt::tune(ctx, lt::order_candidates(m), m, run, ms, 3);
                 } else {
                     b = scratch_links(nl);
                     z = scratch_links((size_t)32 * f->g.Vh);
@@ -296,7 +298,7 @@ extern "C" int lt_autotune_field(lt_field f, int family, const char* cache_path,
                         lt::k_flow_stage(ctx, f->g, c, a, b, z, 0.0, 0.01, 0.25, 0, 1);
                     };
                     m = lt::tune(ctx, lt::tile_candidates(f->g, 0), d, run, ms, 3);
-                    m = lt::tune(ctx, lt::order_candidates(m, false), m, run, ms, 3);
+                    m = lt::tune(ctx, lt::order_candidates(m), m, run, ms, 3);
                 }
             } catch (...) {
                 (void)hipStreamSynchronize(ctx->stream);

@@ -14,7 +14,7 @@ namespace lt {
 std::vector<LinkMap> tile_candidates(const Geom& g, int threads);
 // site orders (t / y chunking, XCD spread) of one block shape, for the colour sweeps
 // (sweeps = true) or the Jacobi kernels
-std::vector<LinkMap> order_candidates(const LinkMap& base, bool sweeps);
+std::vector<LinkMap> order_candidates(const LinkMap& base);
 // "<arch>|<Nt>x<Nx>x<Ny>x<Nz>|<family>"
 std::string tune_key(int device, const Geom& g, const char* family);
 // cache lookup / update (no-op without a path)

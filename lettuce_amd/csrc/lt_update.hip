@@ -2,11 +2,10 @@
 // overrelaxation and Cabibbo-Marinari pseudo-heatbath with Philox draws.
 //
 // One launch updates one colour class of one direction mu.  With the 2-colour
-// schedule a colour class is exactly one parity array, so every thread owns one
-// link and writes it in place; the staple only reads links of other directions or
-// of the opposite parity, so the update is race free.  The 4-colour schedule
-// (colour (sum + x_mu) mod 4) runs in lt_cb4.hip, one thread per site of the class,
-// on the field reordered for the duration of the call.
+// schedule a colour class is exactly one parity array, and every link is written in
+// place by one lane; the staple only reads links of other directions or of the opposite
+// parity, so the update is race free.  The 4-colour schedule (colour (sum + x_mu) mod 4)
+// runs in lt_cb4.hip on the field reordered for the duration of the call.
 #include "lt_internal.hpp"
 #include "lt_bodies.hpp"
 #include "lt_sweep.hpp"
@@ -17,60 +16,33 @@ namespace {
 
 constexpr int BS = LT_LINK_BS;
 
-#ifndef LT_SWEEP_WAVES
-#define LT_SWEEP_WAVES LT_LINK_WAVES
-#endif
-// Every launch of a sweep reads all eight half-fields, so the parity-1 launch of each
-// direction walks the tiles backwards (rev, xcd_block_dir) and starts on the lines the
-// parity-0 launch touched last, which are still in the L2 and the memory-side cache
-// (overrelaxation colour launch -7 % at 32^4).
+// Three wavefronts per 64 links (update_links_split).  Every launch of a sweep reads all eight
+// half-fields, so the parity-1 launch of each direction walks the blocks backwards
+// (xcd_block_dir) and starts on the lines the parity-0 launch touched last, which are still in
+// the L2 and the memory-side cache.  In a captured update the Philox counter is read from
+// device memory (state[0], advanced by the graph itself) instead of a launch argument, so one
+// captured graph serves every replay; sweep k of an update draws with counter state[0] + k, as
+// the eager sweeps draw with the field's counter.
+// Small launches are bound by the latency of one link (8^4: 7.7 us between events, heatbath
+// 11.5, of which about 6 us are the launch itself), large ones by the memory behind the L2
+// (32^4: 94 us for 453 MB).  Overrelaxation and heatbath with one lane per link: 16^4 10.9 and
+// 21 us, now 10.0 and 16; 24^4 36 and 57, now 32 and 45; 28^4 82 and 98, now 54 and 71; 32^4
+// 96.7 and 126, now 94 and 114.  Only where the blocks of three just pass one round of the
+// GPU's 1024 or two is one lane as good (20^4: 25.0 against 26.1 us; the heatbath there 37.4
+// and 29.8).
+constexpr int CB2_WAVES = 3;
 template <bool HEATBATH>
-__global__ void __launch_bounds__(LT_LINK_BS) __attribute__((amdgpu_waves_per_eu(LT_SWEEP_WAVES)))
-sweep_cb2_kernel(double2* __restrict__ U, Geom g, LinkMap m, int mu, int par, double prefactor, uint64_t seed,
-                 uint64_t counter, int rev)
-{
-    int c[4], s;
-    if (!map_site_dir(g, m, par, rev, c, s)) return;
-    update_link<HEATBATH>(U, g, s, c, mu, par, prefactor, seed, counter);
-}
-
-// Heatbath colour kernels of a captured update: the Philox counter is read from
-// device memory (state[0], advanced by the graph itself) instead of a launch argument,
-// so one captured graph serves every replay; sweep k of an update draws with
-// counter state[0] + k, as the eager sweeps draw with the field's counter.
-__global__ void __launch_bounds__(LT_LINK_BS) __attribute__((amdgpu_waves_per_eu(LT_SWEEP_WAVES)))
-hb_cb2_graph_kernel(double2* __restrict__ U, Geom g, LinkMap m, int mu, int par, double prefactor, uint64_t seed,
-                    const uint64_t* __restrict__ state, int k, int rev)
-{
-    int c[4], s;
-    if (!map_site_dir(g, m, par, rev, c, s)) return;
-    update_link<true>(U, g, s, c, mu, par, prefactor, seed, state[0] + (uint64_t)k);
-}
-
-// ---- small lattices ---------------------------------------------------------------
-// A colour launch of a few thousand links leaves most of the GPU idle, and its duration is
-// the serial work of one link.  Up to SMALL_VH links per colour launch the staple of a link
-// is split over six wavefronts (update_links_split): 8^4 overrelaxation 8.0 us a launch and
-// heatbath 11.9 us between two events, of which about 6 us are the launch itself (four lanes
-// per link: 8.9 and 13.4 us; one lane: 10 and 20 us).  From 16^4 on (32768 links) the launch
-// fills the GPU and one lane per link is as fast or faster (16^4: 11.5 against 12.8 us; 32^4:
-// 96 against 124 us).
-#ifndef LT_SMALL_VH
-#define LT_SMALL_VH 16384
-#endif
-constexpr int SMALL_VH = LT_SMALL_VH;
-
-template <bool HEATBATH>
-__global__ void __launch_bounds__(SPLIT_BS) __attribute__((amdgpu_waves_per_eu(3)))
-split_cb2_kernel(double2* __restrict__ U, Geom g, int mu, int par, double prefactor, uint64_t seed, uint64_t counter,
+__global__ void __launch_bounds__(64 * CB2_WAVES)
+__attribute__((amdgpu_waves_per_eu(split_eu(HEATBATH, SPLIT_WILSON, CB2_WAVES))))
+sweep_cb2_kernel(double2* __restrict__ U, Geom g, int mu, int par, double prefactor, uint64_t seed, uint64_t counter,
                  const uint64_t* __restrict__ state, int k, SplitMap map)
 {
-    __shared__ SplitShared<HEATBATH> sh;
+    __shared__ SplitShared<HEATBATH, CB2_WAVES> sh;
     if (HEATBATH && state) counter = state[0] + (uint64_t)k;
     int c[4] = {0, 0, 0, 0}, s = 0;
     const int i = split_index(map, xcd_block_dir(blockIdx.x, gridDim.x, par));
     if (i >= 0) s = site_of_cb(g, i, par, c);
-    update_links_split<HEATBATH, SPLIT_WILSON>(U, g, mu, i >= 0, s, c, prefactor, seed, counter, 1.0, 0.0, sh);
+    update_links_split<HEATBATH, SPLIT_WILSON, CB2_WAVES>(U, g, mu, i >= 0, s, c, prefactor, seed, counter, 1.0, 0.0, sh);
 }
 
 // PlaquetteSum of the captured update: per-block sums (the block tree of the HMC
@@ -127,46 +99,26 @@ __global__ void LT_LINK_KERNEL staple_field_kernel(const double2* __restrict__ U
     st_link(out, g, s, mu, par, staple(U, g, s, c, mu));
 }
 
-// The colour launches chunk the y tiles by LinkMap::ycs (by default all y tiles of an x
-// step in one chunk: with the alternating walk (rev) 2 % faster per HB + 4 OR update at
-// 32^4 than the two-tile chunks the Jacobi kernels keep; the RK3 flow stage is 1.5 %
-// slower with one chunk).  The tile order never changes a result.
-LinkMap sweep_map(const LinkMap& m)
-{
-    LinkMap r = m;
-    r.yc = r.ycs;
-    finish_map(r);
-    return r;
-}
-
 template <bool HEATBATH>
-void split_cb2(lt_field u, const char* name, int mu, int par, double prefactor, uint64_t counter, const uint64_t* state,
+void cb2_colour(lt_field u, const char* name, int mu, int par, double prefactor, uint64_t counter, const uint64_t* state,
                int k)
 {
     const SplitMap m = split_map(u->g, 2);
-    launch(u->ctx, name, split_cb2_kernel<HEATBATH>, dim3(split_blocks(u->g, m)), dim3(SPLIT_BS), 0, u->d, u->g, mu, par,
-           prefactor, u->seed, counter, state, k, m);
+    launch(u->ctx, name, sweep_cb2_kernel<HEATBATH>, dim3(split_blocks(u->g, m)), dim3(64 * CB2_WAVES),
+           0, u->d, u->g, mu, par, prefactor, u->seed, counter, state, k, m);
 }
 
 // n sweeps; the four-colour ones (split) expect the field in the split order
 template <bool HEATBATH>
 void sweep_launches(lt_field u, int n, int schedule, double prefactor, const char* name)
 {
-    lt_ctx ctx = u->ctx;
-    const Geom& g = u->g;
     for (int k = 0; k < n; ++k) {
         uint64_t counter = HEATBATH ? u->counter++ : 0;
         for (int mu = 0; mu < 4; ++mu) {
             if (schedule == LT_CB4) {
                 for (int col = 0; col < 4; ++col) k_cb4_colour(u, HEATBATH, mu, col, prefactor, counter, name);
-            } else if (g.Vh <= SMALL_VH) {
-                for (int par = 0; par < 2; ++par)
-                    split_cb2<HEATBATH>(u, name, mu, par, prefactor, counter, nullptr, 0);
             } else {
-                const LinkMap m = sweep_map(u->map);
-                for (int par = 0; par < 2; ++par)
-                    launch(ctx, name, sweep_cb2_kernel<HEATBATH>, dim3(map_blocks(m)), dim3(m.nthreads), 0, u->d, g, m, mu,
-                           par, prefactor, u->seed, counter, par);
+                for (int par = 0; par < 2; ++par) cb2_colour<HEATBATH>(u, name, mu, par, prefactor, counter, nullptr, 0);
             }
         }
     }
@@ -269,18 +221,12 @@ namespace {
 void enqueue_update(lt_field u, UpdateGraph& G, double prefactor)
 {
     lt_ctx ctx = u->ctx;
-    const Geom& g = u->g;
-    const LinkMap m = sweep_map(u->map);
     for (int k = 0; k < G.n_hb; ++k)
         for (int mu = 0; mu < 4; ++mu) {
             if (G.schedule == LT_CB4) {
                 for (int col = 0; col < 4; ++col) k_cb4_colour_graph_hb(u, mu, col, prefactor, G.state, k);
-            } else if (g.Vh <= SMALL_VH) {
-                for (int par = 0; par < 2; ++par) split_cb2<true>(u, "hb_cb2", mu, par, prefactor, 0, G.state, k);
             } else {
-                for (int par = 0; par < 2; ++par)
-                    launch(ctx, "hb_cb2", hb_cb2_graph_kernel, dim3(map_blocks(m)), dim3(m.nthreads), 0, u->d, g, m,
-                           mu, par, prefactor, u->seed, (const uint64_t*)G.state, k, par);
+                for (int par = 0; par < 2; ++par) cb2_colour<true>(u, "hb_cb2", mu, par, prefactor, 0, G.state, k);
             }
         }
     sweep_launches<false>(u, G.n_or, G.schedule, 0.0, G.schedule == LT_CB4 ? "or_cb4" : "or_cb2");
@@ -289,7 +235,7 @@ void enqueue_update(lt_field u, UpdateGraph& G, double prefactor)
             k_cb4_plaq_partials(u, G.part);
         else
             launch(ctx, "plaquette", upd_plaq_kernel, dim3(8 * map_blocks(u->map)), dim3(u->map.nthreads), 0,
-                   (const double2*)u->d, g, u->map, G.part);
+                   (const double2*)u->d, u->g, u->map, G.part);
         launch(ctx, "reduce_finish", upd_plaq_finish_kernel, dim3(1), dim3(RBS), 0, (const double*)G.part, (int)G.nb,
                (const uint64_t*)G.state, G.plaq);
     }

@@ -95,8 +95,8 @@ def test_overrelaxation_keeps_action_and_schedule_check(la, lto, gpu_ctx):
 
 
 # extents: whole and partial blocks of 64 links, one and several timeslices per chunk, the
-# smallest lattice; actions with and without the rectangle
-@pytest.mark.parametrize("shape", [(4, 4, 4, 4), (4, 12, 8, 4), (16, 4, 8, 8), (8, 12, 4, 20)])
+# smallest lattice, rows of 32 z; actions with and without the rectangle
+@pytest.mark.parametrize("shape", [(4, 4, 4, 4), (4, 12, 8, 4), (16, 4, 8, 8), (8, 12, 4, 20), (4, 8, 4, 32)])
 @pytest.mark.parametrize("c_rect", [-1.0 / 12.0, 0.0])
 def test_split_staple_sweeps_match_oracle(la, lto, gpu_ctx, shape, c_rect):
     """One overrelaxation and one heatbath sweep from identical links: per link 1e-12 and

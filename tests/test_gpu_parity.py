@@ -337,8 +337,8 @@ def one_rounding(U):
 
 
 # split colour launches: whole and partial blocks of 64 links, one and several timeslices per
-# chunk, both sides of the switch to one lane per link (32768 links of rows of 32, 16384 links
-# with two colours); beta = 0.7 rejects most draws, so third and later attempts occur
+# chunk, rows of 32 z and others (three and six wavefronts per block); beta = 0.7 rejects most
+# draws, so third and later attempts occur
 @pytest.mark.parametrize("schedule,shape", [(2, (2, 2, 2, 2)), (2, (6, 10, 4, 14)), (2, (16, 4, 8, 4)), (2, (8, 16, 16, 18)),
                                             (4, (4, 4, 4, 4)), (4, (16, 12, 4, 20)), (4, (4, 4, 8, 32)),
                                             (4, (20, 16, 16, 32))])
