@@ -48,21 +48,21 @@ __device__ __forceinline__ int rep_of(const int* __restrict__ pre, int n, int b)
 __global__ void LT_LINK_KERNEL bk_momentum(double2* __restrict__ P, BatchGrid bg, const uint64_t* __restrict__ counter)
 {
     LT_BATCH_LINK_PROLOGUE
-    body_momentum(P + off, g, m, lb, bg.reps[r].seed, counter[r]);
+    body_momentum<true>(P + off, g, m, lb, bg.reps[r].seed, counter[r]);
 }
 
 __global__ void LT_LINK_KERNEL bk_force_update(const double2* __restrict__ U, double2* __restrict__ P,
                                                const double2* __restrict__ F, BatchGrid bg, double a, double bf)
 {
     LT_BATCH_LINK_PROLOGUE
-    body_force_update(U + off, P + off, F ? F + off : nullptr, g, m, lb, a, bf);
+    body_force_update<true>(U + off, P + off, F ? F + off : nullptr, g, m, lb, a, bf);
 }
 
 __global__ void LT_LINK_KERNEL bk_field_update(double2* __restrict__ U, const double2* __restrict__ P, BatchGrid bg,
                                                double eps)
 {
     LT_BATCH_LINK_PROLOGUE
-    body_field_update(U + off, P + off, g, m, lb, eps);
+    body_field_update<true>(U + off, P + off, g, m, lb, eps);
 }
 
 __global__ void LT_LINK_KERNEL bk_stout_tape(const double2* __restrict__ Uin, double2* __restrict__ Uout,
@@ -151,7 +151,18 @@ __global__ void __launch_bounds__(RBS) bk_kinetic(const double2* __restrict__ P,
     const int r = rep_of(bg.kb, bg.n, blockIdx.x);
     const Geom g = bg.reps[r].g;
     const int i = (blockIdx.x - bg.kb[r]) * RBS + threadIdx.x;
-    block_sum(i < 8 * g.Vh ? body_kinetic_link(P + bg.reps[r].off, g, i) : 0.0, part + blockIdx.x);
+    block_sum(i < 8 * g.Vh ? body_kinetic_link<true>(P + bg.reps[r].off, g, i) : 0.0, part + blockIdx.x);
+}
+
+// P += a F, momenta in 8 reals
+__global__ void __launch_bounds__(RBS) bk_momentum_kick(double2* __restrict__ P, const double2* __restrict__ F,
+                                                        BatchGrid bg, double a)
+{
+    const int r = rep_of(bg.kb, bg.n, blockIdx.x);
+    const Geom g = bg.reps[r].g;
+    const long long off = bg.reps[r].off;
+    const int i = (blockIdx.x - bg.kb[r]) * RBS + threadIdx.x;
+    if (i < 8 * g.Vh) body_momentum_entry<false>(P + off, F + off, g, i, a);
 }
 
 // block r: ordered sum of replica r's partials (same order as the single-lattice finish)
@@ -431,6 +442,11 @@ void kb_kinetic(lt_ctx ctx, const BatchGrid& bg, int total_kb, const double2* P,
 {
     launch(ctx, "batch_kinetic", bk_kinetic, dim3(total_kb), dim3(RBS), 0, P, bg, part);
     launch(ctx, "batch_finish", bk_finish, dim3(bg.n), dim3(RBS), 0, (const double*)part, bg.kb, 1, out);
+}
+
+void kb_momentum_kick(lt_ctx ctx, const BatchGrid& bg, int total_kb, double2* P, const double2* F, double a)
+{
+    launch(ctx, "batch_momentum_kick", bk_momentum_kick, dim3(total_kb), dim3(RBS), 0, P, F, bg, a);
 }
 
 void kb_dvdq(lt_ctx ctx, const BatchGrid& bg, const BatchState& st, const DevBias& bias, int sample_index)

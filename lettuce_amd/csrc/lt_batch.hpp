@@ -85,6 +85,7 @@ void kb_stout_recursion_run(lt_ctx ctx, const BatchGrid& bg, int total_lb, const
 void kb_plaquette(lt_ctx ctx, const BatchGrid& bg, int total_sb, const double2* U, double* part, double* out);
 void kb_kinetic(lt_ctx ctx, const BatchGrid& bg, int total_kb, const double2* P, double* part, double* out);
 // scalar stages (one thread per replica)
+void kb_momentum_kick(lt_ctx ctx, const BatchGrid& bg, int total_kb, double2* P, const double2* F, double a);
 void kb_dvdq(lt_ctx ctx, const BatchGrid& bg, const BatchState& st, const DevBias& bias, int sample_index);
 void kb_h0(lt_ctx ctx, const BatchGrid& bg, const BatchState& st, const DevBias& bias, double beta);
 void kb_h1_accept(lt_ctx ctx, const BatchGrid& bg, const BatchState& st, const DevBias& bias, double beta,

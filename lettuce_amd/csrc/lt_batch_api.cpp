@@ -186,7 +186,7 @@ void enqueue_step(lt_batch b, const StepKey& p, int n_sub)
             else if (kick == lt::KICK_GAUGE)   // UpdateGaugeMomenta (:464-477)
                 lt::kb_force_update(ctx, bg, b->total_lb, b->U, b->P, nullptr, e * p.beta / 6.0, 0.0);
             else   // UpdateMetadynamicsMomenta (:479-491)
-                lt::k_axpy(ctx, b->F, b->P, e, (size_t)b->total);
+                lt::kb_momentum_kick(ctx, bg, b->total_kb, b->P, b->F, e);
         },
         [&](double e) { lt::kb_field_update(ctx, bg, b->total_lb, b->U, b->P, e); });
     forward(b, bg);

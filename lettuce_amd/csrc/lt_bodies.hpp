@@ -15,9 +15,14 @@ namespace lt {
 
 // ---------------------------------------------------------------- HMC
 
+// Momenta are anti-hermitian and traceless wherever the trajectory functions made them, and
+// are kept in 8 reals then (ALG: ld_ah8, st_ah8, the first four of the nine slots): 64 bytes a
+// link instead of 144.  The momenta a caller hands over are general matrices.
+
 // P = 1/2 * A with A the anti-hermitian combination of the eight generators used
 // by the reference's RandomMomentum; phi_1..phi_8 come from Philox stream
 // RNG_MOMENTUM, draw blocks k = 0..3 (Box-Muller pairs).
+template <bool ALG>
 __device__ __forceinline__ void body_momentum(double2* __restrict__ P, const Geom& g, const LinkMap& m, int b,
                                               uint64_t seed, uint64_t counter)
 {
@@ -43,20 +48,44 @@ __device__ __forceinline__ void body_momentum(double2* __restrict__ P, const Geo
     A.m[6] = cd{-phi[5], phi[4]};
     A.m[7] = cd{-phi[7], phi[6]};
     A.m[8] = cd{0.0, -2.0 * phi[8] / s3};
-    st_link(P, g, s, mu, par, scale(0.5, A));
+    A = scale(0.5, A);
+    if (ALG)
+        st_ah8(P, g, s, mu, par, ah_tri(A));
+    else
+        st_link(P, g, s, mu, par, A);
 }
 
-// P += a * Algebra(st U^+) + bf * F   (F optional: metadynamics force)
+// x += a y
+__device__ __forceinline__ void axpy_tri(Tri& x, double a, const Tri& y)
+{
+    x.d0 += a * y.d0;
+    x.d1 += a * y.d1;
+    x.r01 += a * y.r01;
+    x.r02 += a * y.r02;
+    x.r12 += a * y.r12;
+}
+
+// P += a * Algebra(st U^+) + bf * F   (F optional: metadynamics force, whole matrices)
+template <bool ALG>
 __device__ __forceinline__ void body_force_update(const double2* __restrict__ U, double2* __restrict__ P,
                                                   const double2* __restrict__ F, const Geom& g, const LinkMap& m, int b,
                                                   double a, double bf)
 {
     int mu, par, c[4], s;
     if (!map_link_b(g, m, b, mu, par, c, s)) return;
-    // 16^3 x 32: 60.8 us a launch, 63 with the plain staple
+    // 16^3 x 32, whole matrices: 60.8 us a launch, 63 with the plain staple
     Raw6 own;
     const M3 st = staple_pipelined(U, g, s, c, mu, par, own);
     M3 A = algebra(mul_nd(st, su3_of(own)));
+    if (ALG) {
+        Raw4 r;
+        ld_ah8(P, g, s, mu, par, r);
+        Tri p = her_of(r);
+        axpy_tri(p, a, ah_tri(A));
+        if (F) axpy_tri(p, bf, ah_tri(ld(F, g, s, mu, par)));
+        st_ah8(P, g, s, mu, par, p);
+        return;
+    }
     M3 p = ld(P, g, s, mu, par);
     if (F) {
         M3 f = ld(F, g, s, mu, par);
@@ -70,12 +99,22 @@ __device__ __forceinline__ void body_force_update(const double2* __restrict__ U,
 }
 
 // U <- exp(eps P) U, Gram-Schmidt (local per link, in place)
+template <bool ALG>
 __device__ __forceinline__ void body_field_update(double2* __restrict__ U, const double2* __restrict__ P, const Geom& g,
                                                   const LinkMap& m, int b, double eps)
 {
     int mu, par, c[4], s;
     if (!map_link_b(g, m, b, mu, par, c, s)) return;
-    M3 W = mul(exp_ah(ld(P, g, s, mu, par), eps), ldu(U, g, s, mu, par));
+    M3 E;
+    if (ALG) {
+        Raw4 r;
+        ld_ah8(P, g, s, mu, par, r);
+        const Tri p = her_of(r);
+        E = exp_alg8(Alg8{p.d0, p.d1, p.r01, p.r02, p.r12}, eps);
+    } else {
+        E = exp_ah(ld(P, g, s, mu, par), eps);
+    }
+    M3 W = mul(E, ldu(U, g, s, mu, par));
     gram_schmidt(W);
     stu(U, g, s, mu, par, W);
 }
@@ -83,14 +122,49 @@ __device__ __forceinline__ void body_field_update(double2* __restrict__ U, const
 // -Re tr(P P) of entry i of the 8 Vh entries (mu, parity, cb): lanes walk one array, and no
 // coordinates are needed (one lane per (site, mu) in lexicographic order takes four times the
 // L1 accesses; 16^3 x 32: 16.5 -> 15 us between events, the launch itself about 6)
+template <bool ALG>
 __device__ __forceinline__ double body_kinetic_link(const double2* __restrict__ P, const Geom& g, int i)
 {
     const int a = i / g.Vh;
     const double2* q = P + slot_base(g, a, 9, i - a * g.Vh);
+    if (ALG) {
+        Raw4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r.v[e] = q[(size_t)e * slot_stride(g)];
+        const Tri p = her_of(r);
+        return -retr_ah(p, p);
+    }
     M3 p;
 #pragma unroll
     for (int e = 0; e < 9; ++e) p.m[e] = cd{q[(size_t)e * slot_stride(g)].x, q[(size_t)e * slot_stride(g)].y};
     return -retr_mul(p, p);
+}
+
+// entry i of the 8 Vh entries: P += a F with P in 8 reals and F whole matrices, or (a = 0, no
+// F) P written out as whole matrices
+template <bool WHOLE>
+__device__ __forceinline__ void body_momentum_entry(double2* __restrict__ P, const double2* __restrict__ F, const Geom& g,
+                                                    int i, double a)
+{
+    const int k = i / g.Vh;
+    const size_t o = slot_base(g, k, 9, i - k * g.Vh), st = slot_stride(g);
+    double2* q = P + o;
+    if (WHOLE) {
+        Raw4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r.v[e] = q[(size_t)e * st];
+        const M3 p = add_ah(m3_zero(), her_of(r));
+#pragma unroll
+        for (int e = 0; e < 9; ++e) q[(size_t)e * st] = make_double2(p.m[e].re, p.m[e].im);
+    } else {
+        const double2* f = F + o;
+        q[0] = make_double2(q[0].x + a * f[0].y, q[0].y + a * f[4 * st].y);
+#pragma unroll
+        for (int e = 1; e < 4; ++e) {
+            const double2 v = f[(size_t)(e == 3 ? 5 : e) * st];
+            q[(size_t)e * st] = make_double2(q[(size_t)e * st].x + a * v.x, q[(size_t)e * st].y + a * v.y);
+        }
+    }
 }
 
 // ------------------------------------------------- collective variable
@@ -397,7 +471,7 @@ __device__ __forceinline__ void body_lambda(double2* __restrict__ Sig, const dou
 // Lambda buffer this launch reads: other lanes still read their neighbours' entries there).
 // SIGMA_KICK (the last level of the recursion inside a metadynamics momentum update): the
 // result is the bias force at level 0, and instead of storing it the kernel applies
-// UpdateMomenta to the link, P += a Algebra(st U^+) + bf * force, with the staple it
+// UpdateMomenta to the link (momenta in 8 reals), P += a Algebra(st U^+) + bf * force, with the staple it
 // already holds -- body_force_update's formula, without the force field's store and
 // load and the staple formed again (the momenta agree with the separate update to
 // rounding, not bit for bit: the products are contracted into fused multiply-adds
@@ -476,10 +550,9 @@ __device__ __forceinline__ void body_sigma_all(const double2* __restrict__ U, do
     }
     Raw4 y;
     ld_ah8(Sig, g, s, mu, par, y);
-    M3 p;
-    Raw4 tape;
+    Raw4 tape, p;
     if (MODE == SIGMA_LAMBDA) ld_raw4(next.T, g, s, mu, par, tape);
-    if (MODE == SIGMA_KICK) p = ld(kick.P, g, s, mu, par);
+    if (MODE == SIGMA_KICK) ld_ah8(kick.P, g, s, mu, par, p);
     fence();
     M3 cl = m3_zero();   // st^+ Lambda - the six-term sum
     mul_tri_acc<false, 1>(cl, dag(park_load(st_slot, n)), her_of(rl));
@@ -494,9 +567,10 @@ __device__ __forceinline__ void body_sigma_all(const double2* __restrict__ U, do
         lambda_link(sig, her_of(tape), Sig, next.Lam, g, s, mu, par);
     } else {
         const M3 A = algebra(mul_nd(park_load(st_slot, n), L));
-#pragma unroll
-        for (int e = 0; e < 9; ++e) p.m[e] += kick.a * A.m[e] + kick.bf * sig.m[e];
-        st_link(kick.P, g, s, mu, par, p);
+        Tri q8 = her_of(p);
+        axpy_tri(q8, kick.a, ah_tri(A));
+        axpy_tri(q8, kick.bf, ah_tri(sig));
+        st_ah8(kick.P, g, s, mu, par, q8);
     }
 }
 

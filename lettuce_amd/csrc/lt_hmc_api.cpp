@@ -15,11 +15,14 @@
 #include "lt_internal.hpp"
 
 namespace lt {
-void k_random_momentum(lt_field P, uint64_t seed, uint64_t counter);
-void k_force_update(lt_field U, lt_field P, const double2* F, double a, double b);
-void k_field_update(lt_field U, lt_field P, double eps);
+// alg: momenta in 8 reals instead of whole matrices
+void k_random_momentum(lt_field P, uint64_t seed, uint64_t counter, bool alg);
+void k_force_update(lt_field U, lt_field P, const double2* F, double a, double b, bool alg);
+void k_field_update(lt_field U, lt_field P, double eps, bool alg);
 double k_plaquette_sum(lt_field U);
-double k_kinetic(lt_field P);
+double k_kinetic(lt_field P, bool alg);
+void k_momentum_kick(lt_ctx ctx, const Geom& g, double2* P, const double2* F, double a);
+void k_momentum_whole(lt_field P);
 void k_stout_tape(lt_ctx ctx, const Geom& g, const LinkMap& m, const double2* in, double2* out, double2* tape,
                   double rho, double2* keep = nullptr);
 double k_clover_charge(lt_ctx ctx, const Geom& g, const double2* U, double2* C);
@@ -272,10 +275,10 @@ void integrate(int kind, double tau, int n_step, const std::function<void(double
     lt::hmc_schedule(kind, tau, n_step, P, U);
 }
 
-double hamiltonian(lt_field U, lt_field P, double beta)
+double hamiltonian(lt_field U, lt_field P, double beta, bool alg)
 {
     const double S = beta * (6.0 * (double)U->g.V - lt::k_plaquette_sum(U) / 3.0);
-    return S + lt::k_kinetic(P);
+    return S + lt::k_kinetic(P, alg);
 }
 
 void copy_field(lt_field dst, lt_field src)
@@ -360,7 +363,7 @@ double cv_charge(lt_cv cv, lt_field U)
 }
 
 // The molecular dynamics of HMCMetaDKernel (Integrator(*this, ...), hmc_metadynamics.hpp:374-524)
-// on the momenta in P; F is force scratch; the CVs of the sampling kicks are appended to samples.
+// on the momenta in P (8 reals); F is force scratch; the CVs of the sampling kicks are appended to samples.
 void metad_integrate(lt_field U, lt_field P, lt_field F, lt_cv cv, lt_bias bias, double beta, int integrator,
                      double tau, int n_step, std::vector<double>& samples)
 {
@@ -380,13 +383,13 @@ void metad_integrate(lt_field U, lt_field P, lt_field F, lt_cv cv, lt_bias bias,
                 cv_backward(cv, bias->derivative(q), F->d);
             }
             if (kick == lt::KICK_BOTH)   // UpdateMomenta (:441-459)
-                lt::k_force_update(U, P, F->d, e * beta / 6.0, e);
+                lt::k_force_update(U, P, F->d, e * beta / 6.0, e, true);
             else if (kick == lt::KICK_GAUGE)   // UpdateGaugeMomenta (:464-477)
-                lt::k_force_update(U, P, nullptr, e * beta / 6.0, 0.0);
+                lt::k_force_update(U, P, nullptr, e * beta / 6.0, 0.0, true);
             else   // UpdateMetadynamicsMomenta (:479-491)
-                lt::k_axpy(U->ctx, F->d, P->d, e, (size_t)72 * P->g.Vh);
+                lt::k_momentum_kick(U->ctx, P->g, P->d, F->d, e);
         },
-        [&](double e) { lt::k_field_update(U, P, e); });
+        [&](double e) { lt::k_field_update(U, P, e, true); });
 }
 
 }  // namespace
@@ -404,7 +407,7 @@ int lt_hmc_random_momentum(lt_field P, uint64_t seed, uint64_t counter)
 {
     if (!P) return fail(LT_EINVAL, "null field");
     return guarded([&] {
-        lt::k_random_momentum(P, seed, counter);
+        lt::k_random_momentum(P, seed, counter, false);
         P->su3 = false;
         return LT_OK;
     });
@@ -414,7 +417,7 @@ int lt_hmc_update_momenta(lt_field U, lt_field P, double eps, double beta)
 {
     if (!U || !P || !same_shape(U->g, P->g)) return fail(LT_EINVAL, "lt_hmc_update_momenta: bad fields");
     return guarded([&] {
-        lt::k_force_update(U, P, nullptr, eps * beta / 6.0, 0.0);
+        lt::k_force_update(U, P, nullptr, eps * beta / 6.0, 0.0, false);
         return LT_OK;
     });
 }
@@ -423,7 +426,7 @@ int lt_hmc_update_fields(lt_field U, lt_field P, double eps)
 {
     if (!U || !P || !same_shape(U->g, P->g)) return fail(LT_EINVAL, "lt_hmc_update_fields: bad fields");
     return guarded([&] {
-        lt::k_field_update(U, P, eps);
+        lt::k_field_update(U, P, eps, false);
         return LT_OK;
     });
 }
@@ -432,7 +435,7 @@ int lt_hmc_hamiltonian(lt_field U, lt_field P, double beta, double* H)
 {
     if (!U || !P || !H || !same_shape(U->g, P->g)) return fail(LT_EINVAL, "lt_hmc_hamiltonian: bad arguments");
     return guarded([&] {
-        *H = hamiltonian(U, P, beta);
+        *H = hamiltonian(U, P, beta, false);
         return LT_OK;
     });
 }
@@ -443,8 +446,8 @@ int lt_hmc_integrate(lt_field U, lt_field P, double beta, int integrator, double
         return fail(LT_EINVAL, "lt_hmc_integrate: bad arguments");
     return guarded([&] {
         integrate(
-            integrator, tau, n_step, [&](double e, bool) { lt::k_force_update(U, P, nullptr, e * beta / 6.0, 0.0); },
-            [&](double e) { lt::k_field_update(U, P, e); });
+            integrator, tau, n_step, [&](double e, bool) { lt::k_force_update(U, P, nullptr, e * beta / 6.0, 0.0, false); },
+            [&](double e) { lt::k_field_update(U, P, e, false); });
         return LT_OK;
     });
 }
@@ -459,13 +462,14 @@ int lt_hmc_trajectory(lt_field U, lt_field P, lt_field U_copy, double beta, int 
         // HMCKernel::operator() (hmc_gauge.hpp:549-583)
         const uint64_t counter = U->counter++;
         copy_field(U_copy, U);
-        lt::k_random_momentum(P, U->seed, counter);
+        lt::k_random_momentum(P, U->seed, counter, true);
         P->su3 = false;
-        const double H0 = hamiltonian(U, P, beta);
+        const double H0 = hamiltonian(U, P, beta, true);
         integrate(
-            integrator, tau, n_step, [&](double e, bool) { lt::k_force_update(U, P, nullptr, e * beta / 6.0, 0.0); },
-            [&](double e) { lt::k_field_update(U, P, e); });
-        const double H1 = hamiltonian(U, P, beta);
+            integrator, tau, n_step, [&](double e, bool) { lt::k_force_update(U, P, nullptr, e * beta / 6.0, 0.0, true); },
+            [&](double e) { lt::k_field_update(U, P, e, true); });
+        const double H1 = hamiltonian(U, P, beta, true);
+        lt::k_momentum_whole(P);
         const double d = H1 - H0;
         int acc = 1;
         if (metropolis) {
@@ -486,17 +490,18 @@ int lt_hmc_reversibility_test(lt_field U, lt_field P, double beta, int integrato
         return fail(LT_EINVAL, "lt_hmc_reversibility_test: bad arguments");
     return guarded([&] {
         // HMCKernel::ReversibilityTest (hmc_gauge.hpp:585-599)
-        lt::k_random_momentum(P, U->seed, U->counter++);
+        lt::k_random_momentum(P, U->seed, U->counter++, true);
         P->su3 = false;
-        const double H0 = hamiltonian(U, P, beta);
+        const double H0 = hamiltonian(U, P, beta, true);
         for (int pass = 0; pass < 2; ++pass) {
             if (pass) lt::k_scale(U->ctx, P->d, -1.0, (size_t)72 * P->g.Vh);   // ReverseMomenta
             integrate(
                 integrator, tau, n_step,
-                [&](double e, bool) { lt::k_force_update(U, P, nullptr, e * beta / 6.0, 0.0); },
-                [&](double e) { lt::k_field_update(U, P, e); });
+                [&](double e, bool) { lt::k_force_update(U, P, nullptr, e * beta / 6.0, 0.0, true); },
+                [&](double e) { lt::k_field_update(U, P, e, true); });
         }
-        const double H1 = hamiltonian(U, P, beta);
+        const double H1 = hamiltonian(U, P, beta, true);
+        lt::k_momentum_whole(P);
         if (H_old) *H_old = H0;
         if (H_new) *H_new = H1;
         return LT_OK;
@@ -731,17 +736,18 @@ int lt_metad_hmc_trajectory(lt_field U, lt_field P, lt_field U_copy, lt_field F,
     return guarded([&] {
         const uint64_t counter = U->counter++;
         copy_field(U_copy, U);
-        lt::k_random_momentum(P, U->seed, counter);
+        lt::k_random_momentum(P, U->seed, counter, true);
         P->su3 = false;
         F->su3 = false;
         const double cv_old = cv_charge(cv, U);
-        const double H0 = hamiltonian(U, P, beta) + bias->potential(cv_old);
+        const double H0 = hamiltonian(U, P, beta, true) + bias->potential(cv_old);
         std::vector<double> samples;
         samples.reserve(n_step);
         metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, samples);
         cv->path = samples;
         const double cv1 = cv_charge(cv, U);
-        const double H1 = hamiltonian(U, P, beta) + bias->potential(cv1);
+        const double H1 = hamiltonian(U, P, beta, true) + bias->potential(cv1);
+        lt::k_momentum_whole(P);
         const double d = H1 - H0;
         int acc = 1;
         if (metropolis) {
@@ -799,15 +805,16 @@ int lt_metad_reversibility_test(lt_field U, lt_field P, lt_field F, lt_cv cv, lt
         return fail(LT_EINVAL, "lt_metad_reversibility_test: bad arguments");
     return guarded([&] {
         // HMCMetaDKernel::ReversibilityTest (hmc_metadynamics.hpp:657-674)
-        lt::k_random_momentum(P, U->seed, U->counter++);
+        lt::k_random_momentum(P, U->seed, U->counter++, true);
         P->su3 = false;
         F->su3 = false;
-        const double H0 = hamiltonian(U, P, beta) + bias->potential(cv_charge(cv, U));
+        const double H0 = hamiltonian(U, P, beta, true) + bias->potential(cv_charge(cv, U));
         std::vector<double> samples;
         metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, samples);
         lt::k_scale(U->ctx, P->d, -1.0, (size_t)72 * P->g.Vh);   // ReverseMomenta
         metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, samples);
-        const double H1 = hamiltonian(U, P, beta) + bias->potential(cv_charge(cv, U));
+        const double H1 = hamiltonian(U, P, beta, true) + bias->potential(cv_charge(cv, U));
+        lt::k_momentum_whole(P);
         if (H_old) *H_old = H0;
         if (H_new) *H_new = H1;
         return LT_OK;
