@@ -165,17 +165,21 @@ __global__ void __launch_bounds__(RBS) bk_momentum_kick(double2* __restrict__ P,
     if (i < 8 * g.Vh) body_momentum_entry<false>(P + off, F + off, g, i, a);
 }
 
+__device__ __forceinline__ void replica_sum(const double* __restrict__ part, const int* __restrict__ pre, int per, int r,
+                                            double* out)
+{
+    const double* p = part + (size_t)per * pre[r];
+    const int cnt = per * (pre[r + 1] - pre[r]);
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < cnt; i += RBS) acc += p[i];
+    block_sum(acc, out);
+}
 // block r: ordered sum of replica r's partials (same order as the single-lattice finish)
 // (per: partials per block of the prefix)
 __global__ void __launch_bounds__(RBS) bk_finish(const double* __restrict__ part, const int* __restrict__ pre, int per,
                                                  double* out)
 {
-    const int r = blockIdx.x;
-    const double* p = part + (size_t)per * pre[r];
-    const int cnt = per * (pre[r + 1] - pre[r]);
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < cnt; i += RBS) acc += p[i];
-    block_sum(acc, out + r);
+    replica_sum(part, pre, per, blockIdx.x, out + blockIdx.x);
 }
 
 // ------------------------------------------------------------- scalar stages
@@ -213,14 +217,19 @@ __device__ __forceinline__ double charge_of(double raw)
 
 __device__ __forceinline__ double strength_of(const BatchState& st, int r) { return st.strength[st.label[r]]; }
 
-__global__ void __launch_bounds__(SBS) bk_dvdq(BatchGrid bg, BatchState st, DevBias bias, int sample_index)
+// block r: replica r's charge from its partials (as bk_finish; none: the charge is there), its
+// path sample and dV/dQ; one launch where a sum and one block over all replicas took two of
+// about 6 us each
+__global__ void __launch_bounds__(RBS) bk_dvdq(BatchGrid bg, BatchState st, DevBias bias, const double* __restrict__ part,
+                                               int sample_index)
 {
 #pragma clang fp contract(off)
-    for (int r = threadIdx.x; r < bg.n; r += SBS) {
-        const double q = charge_of(st.qraw[r]);
-        if (sample_index >= 0) st.samples[(size_t)r * st.n_sub + sample_index] = q;
-        st.dvdq[r] = strength_of(st, r) * bias_derivative(bias, q);
-    }
+    const int r = blockIdx.x;
+    if (part) replica_sum(part, bg.sb, 3, r, st.qraw + r);
+    if (threadIdx.x) return;
+    const double q = charge_of(st.qraw[r]);
+    if (sample_index >= 0) st.samples[(size_t)r * st.n_sub + sample_index] = q;
+    st.dvdq[r] = strength_of(st, r) * bias_derivative(bias, q);
 }
 
 // H = beta (6V - plaq/3) + kinetic + strength * V(Q)   (hmc_gauge.hpp:525-541, hmc_metadynamics.hpp:557-559)
@@ -391,7 +400,7 @@ void kb_clover_charge(lt_ctx ctx, const BatchGrid& bg, int total_sb, const doubl
                       double* qraw)
 {
     launch(ctx, "batch_clover_store", bk_clover_charge, dim3(3 * total_sb), dim3(RBS), 0, U, C, bg, part);
-    launch(ctx, "batch_finish", bk_finish, dim3(bg.n), dim3(RBS), 0, (const double*)part, bg.sb, 3, qraw);
+    if (qraw) launch(ctx, "batch_finish", bk_finish, dim3(bg.n), dim3(RBS), 0, (const double*)part, bg.sb, 3, qraw);
 }
 
 void kb_clover_deriv(lt_ctx ctx, const BatchGrid& bg, int total_lb, const double2* U, const double2* C, double2* F,
@@ -449,9 +458,10 @@ void kb_momentum_kick(lt_ctx ctx, const BatchGrid& bg, int total_kb, double2* P,
     launch(ctx, "batch_momentum_kick", bk_momentum_kick, dim3(total_kb), dim3(RBS), 0, P, F, bg, a);
 }
 
-void kb_dvdq(lt_ctx ctx, const BatchGrid& bg, const BatchState& st, const DevBias& bias, int sample_index)
+void kb_dvdq(lt_ctx ctx, const BatchGrid& bg, const BatchState& st, const DevBias& bias, const double* part,
+             int sample_index)
 {
-    launch(ctx, "batch_dvdq", bk_dvdq, dim3(1), dim3(SBS), 0, bg, st, bias, sample_index);
+    launch(ctx, "batch_dvdq", bk_dvdq, dim3(bg.n), dim3(RBS), 0, bg, st, bias, part, sample_index);
 }
 
 void kb_h0(lt_ctx ctx, const BatchGrid& bg, const BatchState& st, const DevBias& bias, double beta)

@@ -72,7 +72,7 @@ void kb_force_update(lt_ctx ctx, const BatchGrid& bg, int total_lb, const double
 void kb_field_update(lt_ctx ctx, const BatchGrid& bg, int total_lb, double2* U, const double2* P, double eps);
 void kb_stout_tape(lt_ctx ctx, const BatchGrid& bg, int total_lb, const double2* in, double2* out, double2* tape,
                    double rho);
-// clover planes, charge-density partials and per-replica finish into qraw
+// clover planes, charge-density partials and (qraw not null) per-replica finish into qraw
 void kb_clover_charge(lt_ctx ctx, const BatchGrid& bg, int total_sb, const double2* U, double2* C, double* part,
                       double* qraw);
 // next: go on with the Lambda of the top stout level (see k_clover_deriv)
@@ -84,9 +84,13 @@ void kb_stout_recursion_run(lt_ctx ctx, const BatchGrid& bg, int total_lb, const
                             const MomentumKick* kick = nullptr, bool top_lambda_done = false);
 void kb_plaquette(lt_ctx ctx, const BatchGrid& bg, int total_sb, const double2* U, double* part, double* out);
 void kb_kinetic(lt_ctx ctx, const BatchGrid& bg, int total_kb, const double2* P, double* part, double* out);
-// scalar stages (one thread per replica)
+// P += a F, momenta in 8 reals
 void kb_momentum_kick(lt_ctx ctx, const BatchGrid& bg, int total_kb, double2* P, const double2* F, double a);
-void kb_dvdq(lt_ctx ctx, const BatchGrid& bg, const BatchState& st, const DevBias& bias, int sample_index);
+// the replicas' charges from the partials of kb_clover_charge (null: already in st.qraw), then
+// the bias derivatives
+void kb_dvdq(lt_ctx ctx, const BatchGrid& bg, const BatchState& st, const DevBias& bias, const double* part,
+             int sample_index);
+// scalar stages (one thread per replica)
 void kb_h0(lt_ctx ctx, const BatchGrid& bg, const BatchState& st, const DevBias& bias, double beta);
 void kb_h1_accept(lt_ctx ctx, const BatchGrid& bg, const BatchState& st, const DevBias& bias, double beta,
                   int metropolis);

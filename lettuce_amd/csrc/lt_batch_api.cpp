@@ -135,12 +135,14 @@ void ensure_samples(lt_batch b, int n_sub)
     b->n_sub_cap = n_sub;
 }
 
-// CV forward for all replicas: stout levels with tapes, clover planes, raw charge sums
-void forward(lt_batch b, const lt::BatchGrid& bg)
+// CV forward for all replicas: stout levels with tapes, clover planes, raw charge sums (finish)
+// or only their partials
+void forward(lt_batch b, const lt::BatchGrid& bg, bool finish)
 {
     for (int k = 0; k < b->n_levels; ++k)
         lt::kb_stout_tape(b->ctx, bg, b->total_lb, b->levels[k], b->levels[k + 1], b->tapes[k], b->rho);
-    lt::kb_clover_charge(b->ctx, bg, b->total_sb, b->levels[b->n_levels], b->clover, b->part, b->st.qraw);
+    lt::kb_clover_charge(b->ctx, bg, b->total_sb, b->levels[b->n_levels], b->clover, b->part,
+                         finish ? b->st.qraw : nullptr);
 }
 
 // One PT-MetaD step (HMCMetaDKernel::operator(), hmc_metadynamics.hpp:552-655, per replica;
@@ -155,18 +157,22 @@ void enqueue_step(lt_batch b, const StepKey& p, int n_sub)
 
     lt::k_copy(ctx, b->U, b->Ucopy, (size_t)b->total);
     lt::kb_momentum(ctx, bg, b->total_lb, b->P, st.counter);
-    forward(b, bg);
+    forward(b, bg, true);
     lt::kb_plaquette(ctx, bg, b->total_sb, b->U, b->part, st.plaq);
     lt::kb_kinetic(ctx, bg, b->total_kb, b->P, b->part, st.kin);
     lt::kb_h0(ctx, bg, st, bias, p.beta);
     int isub = 0;
+    bool moved = false;   // links updated since the last forward pass
     lt::metad_schedule(
         p.integrator, p.tau, p.n_step,
         [&](double e, bool sub, int kick) {
             if (kick & lt::KICK_BIAS) {
-                // CalculateTopologicalForce (hmc_metadynamics.hpp:374-436)
-                forward(b, bg);
-                lt::kb_dvdq(ctx, bg, st, bias, sub ? isub++ : -1);
+                // CalculateTopologicalForce (hmc_metadynamics.hpp:374-436); a forward pass is made
+                // only where a field update lies between it and the one before: the first kick
+                // takes H0's, and the charges of H1 are the last kick's
+                if (moved) forward(b, bg, false);
+                lt::kb_dvdq(ctx, bg, st, bias, moved ? b->part : nullptr, sub ? isub++ : -1);
+                moved = false;
                 const int n = b->n_levels;
                 // the clover derivative goes on with the Lambda of the top level
                 const lt::SigmaNext top{n > 0 ? b->tapes[n - 1] : nullptr, b->lambda[0]};
@@ -188,8 +194,11 @@ void enqueue_step(lt_batch b, const StepKey& p, int n_sub)
             else   // UpdateMetadynamicsMomenta (:479-491)
                 lt::kb_momentum_kick(ctx, bg, b->total_kb, b->P, b->F, e);
         },
-        [&](double e) { lt::kb_field_update(ctx, bg, b->total_lb, b->U, b->P, e); });
-    forward(b, bg);
+        [&](double e) {
+            lt::kb_field_update(ctx, bg, b->total_lb, b->U, b->P, e);
+            moved = true;
+        });
+    if (moved) forward(b, bg, true);
     lt::kb_plaquette(ctx, bg, b->total_sb, b->U, b->part, st.plaq);
     lt::kb_kinetic(ctx, bg, b->total_kb, b->P, b->part, st.kin);
     lt::kb_h1_accept(ctx, bg, st, bias, p.beta, p.metropolis);

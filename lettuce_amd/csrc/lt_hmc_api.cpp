@@ -363,16 +363,21 @@ double cv_charge(lt_cv cv, lt_field U)
 }
 
 // The molecular dynamics of HMCMetaDKernel (Integrator(*this, ...), hmc_metadynamics.hpp:374-524)
-// on the momenta in P (8 reals); F is force scratch; the CVs of the sampling kicks are appended to samples.
+// on the momenta in P (8 reals); F is force scratch; the CVs of the sampling kicks are appended to
+// samples.  q: the CV of U before (cv's last forward pass was over U) and after.  A forward pass
+// is made only where a field update lies between it and the one before: the first kick takes
+// H0's, and the CV after the last kick is that kick's.
 void metad_integrate(lt_field U, lt_field P, lt_field F, lt_cv cv, lt_bias bias, double beta, int integrator,
-                     double tau, int n_step, std::vector<double>& samples)
+                     double tau, int n_step, double& q, std::vector<double>& samples)
 {
+    bool moved = false;   // links updated since the last forward pass
     lt::metad_schedule(
         integrator, tau, n_step,
         [&](double e, bool sub, int kick) {
             if (kick & lt::KICK_BIAS) {
                 // CalculateTopologicalForce (hmc_metadynamics.hpp:374-436)
-                const double q = cv_forward(cv, U);
+                if (moved) q = cv_forward(cv, U);
+                moved = false;
                 if (sub) samples.push_back(q);
                 if (kick == lt::KICK_BOTH && cv->n_levels > 0) {
                     // UpdateMomenta applied by the last kernel of the force (on level 0 = U)
@@ -389,7 +394,11 @@ void metad_integrate(lt_field U, lt_field P, lt_field F, lt_cv cv, lt_bias bias,
             else   // UpdateMetadynamicsMomenta (:479-491)
                 lt::k_momentum_kick(U->ctx, P->g, P->d, F->d, e);
         },
-        [&](double e) { lt::k_field_update(U, P, e, true); });
+        [&](double e) {
+            lt::k_field_update(U, P, e, true);
+            moved = true;
+        });
+    if (moved) q = cv_charge(cv, U);
 }
 
 }  // namespace
@@ -743,9 +752,9 @@ int lt_metad_hmc_trajectory(lt_field U, lt_field P, lt_field U_copy, lt_field F,
         const double H0 = hamiltonian(U, P, beta, true) + bias->potential(cv_old);
         std::vector<double> samples;
         samples.reserve(n_step);
-        metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, samples);
+        double cv1 = cv_old;
+        metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, cv1, samples);
         cv->path = samples;
-        const double cv1 = cv_charge(cv, U);
         const double H1 = hamiltonian(U, P, beta, true) + bias->potential(cv1);
         lt::k_momentum_whole(P);
         const double d = H1 - H0;
@@ -808,12 +817,13 @@ int lt_metad_reversibility_test(lt_field U, lt_field P, lt_field F, lt_cv cv, lt
         lt::k_random_momentum(P, U->seed, U->counter++, true);
         P->su3 = false;
         F->su3 = false;
-        const double H0 = hamiltonian(U, P, beta, true) + bias->potential(cv_charge(cv, U));
+        double q = cv_charge(cv, U);
+        const double H0 = hamiltonian(U, P, beta, true) + bias->potential(q);
         std::vector<double> samples;
-        metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, samples);
+        metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, q, samples);
         lt::k_scale(U->ctx, P->d, -1.0, (size_t)72 * P->g.Vh);   // ReverseMomenta
-        metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, samples);
-        const double H1 = hamiltonian(U, P, beta, true) + bias->potential(cv_charge(cv, U));
+        metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, q, samples);
+        const double H1 = hamiltonian(U, P, beta, true) + bias->potential(q);
         lt::k_momentum_whole(P);
         if (H_old) *H_old = H0;
         if (H_new) *H_new = H1;
