@@ -88,12 +88,12 @@ bool make_linkmap(const Geom& g, int tt, int tx, int ty, int tz, LinkMap& m)
 // factors of two: 12^4, 20^4, 24^4), a linear map of 128 consecutive checkerboard sites
 // per block (measured at 20^4: overrelaxation colour launch 82 -> 25 us, HB + 4 OR update
 // 3.3 -> 1.0 ms; 24^4: 1.72 -> 1.50 ms).
-LinkMap default_linkmap(const Geom& g)
+LinkMap default_linkmap(const Geom& g, int threads)
 {
     LinkMap m{};
     const int ext[4] = {g.L[0], g.L[1], g.L[2], g.L[3] / 2};
     int T[4] = {1, 1, 1, 1};
-    int want = 128;
+    int want = threads;
     const int order[4] = {3, 2, 1, 0};
     for (int k = 0; k < 4 && want > 1; ++k) {
         int i = order[k];
@@ -112,8 +112,9 @@ LinkMap default_linkmap(const Geom& g)
     }
     // rows cut into pieces of 8 or more (z/2 = 24 at 48^4): a box of whole rows whose
     // thread count is a multiple of 64 (48^4: 1 x 1 x 8 x 24, HB + OR sweeps -4 %, RK3
-    // stage -5 % against 1 x 1 x 16 x 8), most y rows first
-    if (want == 1 && T[3] >= 8 && T[3] < ext[3] && ext[3] <= 32) {
+    // stage -5 % against 1 x 1 x 16 x 8), most y rows first; not for the force's small blocks,
+    // where 1 x 1 x 8 x 8 is the faster one (recursion level 252 -> 220 us at 16^3 x 48)
+    if (threads > FORCE_BLOCK && want == 1 && T[3] >= 8 && T[3] < ext[3] && ext[3] <= 32) {
         int bestn = 0, B[4] = {0, 0, 0, 0};
         for (int ty = ext[2]; ty >= 1; --ty) {
             if (ext[2] % ty) continue;
@@ -135,7 +136,7 @@ LinkMap default_linkmap(const Geom& g)
         if (bestn >= 128 && make_linkmap(g, B[0], B[1], B[2], B[3], m)) return m;
     }
     if (want == 1 && (T[3] >= 8 || T[3] == ext[3]) && make_linkmap(g, T[0], T[1], T[2], T[3], m)) return m;
-    if (make_linkmap(g, 0, 0, 0, 128, m)) return m;
+    if (make_linkmap(g, 0, 0, 0, threads, m)) return m;
     // extents without enough factors of two: the largest dividing tile of at most
     // 256 threads, z-major
     int best = 0, bt[4] = {1, 1, 1, 1};

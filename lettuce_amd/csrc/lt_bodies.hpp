@@ -466,6 +466,7 @@ __device__ __forceinline__ void body_lambda(double2* __restrict__ Sig, const dou
 // Lambda are loaded a half ahead, the link's own after the last half.  Between events, levels
 // with a Lambda and the last one: 16 x 8^4 90 -> 84.7 us, 16^4 106 -> 98 us with Y instead of
 // Sigma' and the early loads; loading every operand two products ahead spills 68 registers.
+// Blocks of one wave (FORCE_BLOCK) take that to 78 and 80 us.
 // MODE SIGMA_STORE stores the result in Sig.  SIGMA_LAMBDA goes on with the Lambda of the
 // level below for the same link, with that level's tape and Lambda buffer in next (not the
 // Lambda buffer this launch reads: other lanes still read their neighbours' entries there).

@@ -45,7 +45,7 @@ void k_clover_deriv(lt_ctx ctx, const Geom& g, const LinkMap& m, const double2* 
 struct lt_cv_s {
     lt_ctx ctx = nullptr;
     lt::Geom g{};
-    lt::LinkMap map{};
+    lt::LinkMap map{}, back{};   // stout levels with tape; clover derivative and recursion
     int n_levels = 0;
     double rho = 0.0;
     int interval = 0;               // 0: full storage, else checkpoint interval k
@@ -331,18 +331,18 @@ void cv_backward(lt_cv cv, double dvdq, double2* F, const lt::MomentumKick* kick
     const int n = cv->n_levels;
     if (cv->interval == 0) {
         if (n == 0) {
-            lt::k_clover_deriv(cv->ctx, cv->g, cv->map, cv->levels[0], cv->clover, F, dvdq);
+            lt::k_clover_deriv(cv->ctx, cv->g, cv->back, cv->levels[0], cv->clover, F, dvdq);
             return;
         }
         // the clover derivative goes on with the Lambda of the top level
         const lt::SigmaNext top{cv->tapes[n - 1], cv->lambda[0]};
-        lt::k_clover_deriv(cv->ctx, cv->g, cv->map, cv->levels[n], cv->clover, F, dvdq, &top);
+        lt::k_clover_deriv(cv->ctx, cv->g, cv->back, cv->levels[n], cv->clover, F, dvdq, &top);
         lt::k_stout_recursion_run(
-            cv->ctx, cv->g, cv->map, [&](int j) -> const double2* { return cv->levels[j]; },
+            cv->ctx, cv->g, cv->back, [&](int j) -> const double2* { return cv->levels[j]; },
             [&](int j) -> const double2* { return cv->tapes[j]; }, n, 0, F, cv->lambda, cv->rho, kick, true);
         return;
     }
-    lt::k_clover_deriv(cv->ctx, cv->g, cv->map, n ? cv->top : cv->input, cv->clover, F, dvdq);
+    lt::k_clover_deriv(cv->ctx, cv->g, cv->back, n ? cv->top : cv->input, cv->clover, F, dvdq);
     const int k = cv->interval;
     for (int a = ((n - 1) / k) * k; a >= 0 && n > 0; a -= k) {
         const int b = std::min(a + k, n);
@@ -351,7 +351,7 @@ void cv_backward(lt_cv cv, double dvdq, double2* F, const lt::MomentumKick* kick
         for (int j = a + 1; j <= b; ++j)
             lt::k_stout_tape(cv->ctx, cv->g, cv->map, level(j - 1), cv->seg[j - a], cv->tapes[j - a - 1], cv->rho);
         lt::k_stout_recursion_run(
-            cv->ctx, cv->g, cv->map, level, [&](int j) -> const double2* { return cv->tapes[j - a]; }, b, a, F,
+            cv->ctx, cv->g, cv->back, level, [&](int j) -> const double2* { return cv->tapes[j - a]; }, b, a, F,
             cv->lambda, cv->rho, a == 0 ? kick : nullptr);
     }
 }
@@ -530,6 +530,7 @@ int lt_cv_create_checkpointed(lt_ctx ctx, int nt, int nx, int ny, int nz, int n_
         cv->ctx = ctx;
         cv->g = lt::make_geom(nt, nx, ny, nz);
         cv->map = lt::default_linkmap(cv->g);
+        cv->back = lt::default_linkmap(cv->g, lt::FORCE_BLOCK);
         cv->n_levels = n_levels;
         cv->rho = rho;
         cv->interval = interval > 0 ? std::min(interval, std::max(n_levels, 1)) : 0;

@@ -272,7 +272,15 @@ inline bool valid_metad_integrator(int k)
 Geom make_geom(int nt, int nx, int ny, int nz);
 // tile map with extents (tt, tx, ty, tz) over (t, x, y, z/2); returns false if they do not divide
 bool make_linkmap(const Geom& g, int tt, int tx, int ty, int tz, LinkMap& m);
-LinkMap default_linkmap(const Geom& g);
+// Block of the clover derivative and of the stout-force recursion.  Their launches hold few
+// waves per CU for long: with blocks of one wave a CU whose block is done gets the next one at
+// once, with 128 threads it waits for both waves and the last blocks go on alone (recursion
+// level 128 -> 64 threads: 16^4 90 -> 80 us, 16^3 x 32 157 -> 150, 24^4 374 -> 365, 32^4 1139 ->
+// 1121, z = 48 252 -> 220 at 16^3 x 48; clover derivative -1 to -4 %, 12 x 8 x 10 x 14 34 -> 27;
+// 256 threads: 24^4 380, 8^4 23.4 against 21.2).  The tape launches before them keep 128: two
+// waves of a block share the links of their neighbours (32^4 526 -> 569 us with 64).
+constexpr int FORCE_BLOCK = 64;
+LinkMap default_linkmap(const Geom& g, int threads = 128);
 // same block shape and site order
 inline bool same_map(const LinkMap& a, const LinkMap& b)
 {

@@ -190,6 +190,23 @@ def test_cv_force_stout_weights(la, lto, gpu_ctx, rho):
     cv.close()
 
 
+# blocks of 64 links: rows of z cut in three, one block that is not full, a partial last block
+@pytest.mark.parametrize("shape", [(2, 2, 8, 48), (2, 2, 2, 2), (2, 6, 2, 10)])
+def test_cv_force_small_blocks(la, lto, gpu_ctx, shape):
+    """The clover derivative and two recursion levels: the bars of one level above."""
+    flush(f"cv blocks {shape}")
+    U0 = lto.stout(lto.haar(shape, 6), shape, 0.1, 1)
+    U = gauge(la, gpu_ctx, shape, U0)
+    F = matrix(la, gpu_ctx, shape)
+    cv = la.CollectiveVariable(gpu_ctx, shape, 2, 0.12)
+    Q = cv.forward(U)
+    cv.backward(0.7, F)
+    Qr, Fr = lto.cv_force(U0, shape, 0.12, 2, 0.7)
+    assert abs(Q - Qr) <= 1e-12 * max(1.0, abs(Qr))
+    assert rel_err(F.download(), Fr) <= 1e-11
+    cv.close()
+
+
 def test_cv_force_golden16(la, lto, golden, gpu_ctx):
     flush("cv golden 16^4")
     U0 = lto.stout(lto.haar(G16, 0), G16, 0.1, 3)
