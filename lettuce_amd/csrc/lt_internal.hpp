@@ -277,10 +277,20 @@ bool make_linkmap(const Geom& g, int tt, int tx, int ty, int tz, LinkMap& m);
 // once, with 128 threads it waits for both waves and the last blocks go on alone (recursion
 // level 128 -> 64 threads: 16^4 90 -> 80 us, 16^3 x 32 157 -> 150, 24^4 374 -> 365, 32^4 1139 ->
 // 1121, z = 48 252 -> 220 at 16^3 x 48; clover derivative -1 to -4 %, 12 x 8 x 10 x 14 34 -> 27;
-// 256 threads: 24^4 380, 8^4 23.4 against 21.2).  The tape launches before them keep 128: two
-// waves of a block share the links of their neighbours (32^4 526 -> 569 us with 64).
+// 256 threads: 24^4 380, 8^4 23.4 against 21.2).  The tape launches before them keep the default: two
+// waves of a block share the links of their neighbours (32^4 526 -> 569 us with 64), except on
+// small lattices (below).
 constexpr int FORCE_BLOCK = 64;
-LinkMap default_linkmap(const Geom& g, int threads = 128);
+// Lattices of up to this volume get blocks of one wave in every link kernel: their 4V links are at
+// most one wave per SIMD, and blocks of two waves leave CUs empty while others hold two blocks.
+// 128 -> 64 threads: four stout levels 8^4 32.0 -> 30.1 us, 10^4 53.1 -> 39.3, 12 x 8 x 10 x 14
+// 57.6 -> 43.7, 16 x 8 x 8 x 16 57.1 -> 46.6; RK3 x 2 48.4 -> 45.6, 79.2 -> 60.8, 83.1 -> 65.5,
+// 82.4 -> 68.5; an OMF2 trajectory of 8 steps 270 -> 260, 368 -> 310, 386 -> 334, 390 -> 347.  Beyond it nothing is left (12^4, 18 x 12 x 10 x 14 and 16^4
+// within 2 % either way), and from 16^3 x 32 on the links that two waves share count (RK3 x 2
+// 387 -> 407, 32^4 2980 -> 3121).
+constexpr int SMALL_VOLUME = 16384;
+// threads: block size, 0 for the default of the lattice's volume
+LinkMap default_linkmap(const Geom& g, int threads = 0);
 // same block shape and site order
 inline bool same_map(const LinkMap& a, const LinkMap& b)
 {

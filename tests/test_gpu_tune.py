@@ -115,3 +115,35 @@ def test_read_rate_probe(la, gpu_ctx):
     for bad in (3 << 20, 1 << 10, 1 << 31):
         with pytest.raises(la.LettuceError):
             gpu_ctx.read_rate(bad)
+
+
+# blocks of one wave by default up to 16384 sites, of two beyond: fewer links than a wave, partial
+# last blocks, rows of z cut in three, the largest small lattice and the smallest shape after it
+@pytest.mark.parametrize("shape, threads", [((2, 2, 2, 2), 64), ((12, 8, 10, 14), 64), ((8, 18, 14, 4), 64), ((4, 4, 8, 48), 64),
+                                            ((16, 8, 8, 16), 64), ((18, 10, 8, 12), 128)])
+def test_default_block_keeps_results(la, lto, gpu_ctx, shape, threads):
+    """Flow, smearing and the update's links are the same bits with the default blocks and with
+    linear ones of 256; the plaquette, summed in another order, to rounding."""
+    flush(f"default block {shape}")
+    U0 = lto.haar(shape, 3)
+    out = []
+    for tile in (None, (0, 0, 0, 256)):
+        U, V, W = (la.GaugeField(gpu_ctx, shape) for _ in range(3))
+        if tile:
+            for f in (U, V, W):
+                f.set_tile(*tile)
+        else:
+            assert np.prod([n for n in U.get_tile() if n]) == threads
+        U.upload(U0)
+        U.set_rng(4, 0)
+        p = la.UpdateSweeps(U, 6.0, 1, 1, 1, 2)
+        la.StoutSmearingN(U, V, 2, 0.12)
+        fl = la.GradientFlowKernel(U, W, "rk3", 0.01)
+        fl(1)
+        fl.close()
+        out.append((p, U.download(), V.download(), W.download()))
+        for f in (U, V, W):
+            f.close()
+    assert abs(out[0][0] - out[1][0]) <= 1e-13 * max(1.0, abs(out[0][0]))
+    for a, b in zip(out[0][1:], out[1][1:]):
+        assert np.array_equal(a, b)
