@@ -270,8 +270,10 @@ __device__ __forceinline__ double body_plaq_link(const double2* __restrict__ U, 
     if (mu < 2) v += plaq_plane(U, g, s, c, par, mu, mu + 2);
     return v;
 }
-// sum of v over the n lanes of a link-map block into *out: a butterfly in each wavefront, then
-// the n / 64 wavefront sums in wave order (sh: LT_LINK_BS / 64 doubles)
+// sum of v over a link-map block of n lanes into *out: a butterfly in each wavefront, then the
+// wavefront sums in wave order (sh: LT_LINK_BS / 64 doubles).  A map's block may end in a part of
+// a wavefront (96 lanes for whole rows of 24 z): such a kernel is launched with whole ones
+// (sum_block), whose further lanes have no site and bring zero.
 __device__ __forceinline__ void link_block_sum(double v, int n, double* sh, double* out)
 {
 #pragma unroll
@@ -279,7 +281,7 @@ __device__ __forceinline__ void link_block_sum(double v, int n, double* sh, doub
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < (n >> 6); ++w) v += sh[w];
+        for (int w = 1; w < ((n + 63) >> 6); ++w) v += sh[w];
         *out = v;
     }
 }

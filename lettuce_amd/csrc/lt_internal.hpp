@@ -219,6 +219,8 @@ inline unsigned map_blocks(const LinkMap& m)
         throw LtError{LT_ESTATE, "invalid thread-block tile for the link kernels"};
     return (unsigned)(m.N[0] * m.N[1] * m.N[2] * m.N[3]);
 }
+// block of the link launches that end in link_block_sum: the map's, in whole wavefronts
+inline dim3 sum_block(const LinkMap& m) { return dim3((unsigned)(m.nthreads + 63) & ~63u); }
 
 // The momentum / field update sequence of Integrators::HMC::{Leapfrog, OMF_2, OMF_4}
 // (LettuceGauge/updates/hmc_gauge.hpp:48-75,155-190,241-295).  P(eps, sub) is a

@@ -340,7 +340,7 @@ double k_wilson_loop(lt_field u, lt_field chain, int n0, int n1, int reset)
     launch(ctx, "wilson_chain", wchain_kernel, dim3(nb), dim3(m.nthreads), 0, (const double2*)u->d, chain->d, g, m, n0, n1,
            reset);
     double* part = ctx->scratch_for((size_t)nb + 1);
-    launch(ctx, "wilson_loop", wloop_kernel, dim3(nb), dim3(m.nthreads), 0, (const double2*)chain->d, g, m, n1, part);
+    launch(ctx, "wilson_loop", wloop_kernel, dim3(nb), sum_block(m), 0, (const double2*)chain->d, g, m, n1, part);
     double w;
     sum_parts(ctx, part, nb, 1, &w);
     return w;

@@ -234,7 +234,7 @@ void enqueue_update(lt_field u, UpdateGraph& G, double prefactor)
         if (G.schedule == LT_CB4)
             k_cb4_plaq_partials(u, G.part);
         else
-            launch(ctx, "plaquette", upd_plaq_kernel, dim3(8 * map_blocks(u->map)), dim3(u->map.nthreads), 0,
+            launch(ctx, "plaquette", upd_plaq_kernel, dim3(8 * map_blocks(u->map)), sum_block(u->map), 0,
                    (const double2*)u->d, u->g, u->map, G.part);
         launch(ctx, "reduce_finish", upd_plaq_finish_kernel, dim3(1), dim3(RBS), 0, (const double*)G.part, (int)G.nb,
                (const uint64_t*)G.state, G.plaq);
@@ -319,7 +319,7 @@ double k_plaquette_planes(lt_field u)
     lt_ctx ctx = u->ctx;
     const unsigned nb = plaq_parts(u->map);
     double* part = ctx->scratch_for((size_t)nb + 1);
-    launch(ctx, "plaquette", upd_plaq_kernel, dim3(8 * map_blocks(u->map)), dim3(u->map.nthreads), 0,
+    launch(ctx, "plaquette", upd_plaq_kernel, dim3(8 * map_blocks(u->map)), sum_block(u->map), 0,
            (const double2*)u->d, u->g, u->map, part);
     launch(ctx, "plaquette_sum", plaq_sum_kernel, dim3(1), dim3(RBS), 0, (const double*)part, (int)nb, part + nb);
     double* h = ctx->host_for(1);

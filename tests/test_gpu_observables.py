@@ -135,3 +135,32 @@ def test_plaquette_sum(la, lto, gpu_ctx, shape, tiles):
     f.SetToIdentity()
     assert la.PlaquetteSum(f) == 18.0 * lto.volume(shape)
     f.close()
+
+
+# blocks that are not whole wavefronts: less than one, and a part of the second, third and fourth
+@pytest.mark.parametrize("shape,tiles,schedules", [
+    ((4, 4, 8, 24), [(1, 1, 8, 12), (1, 1, 4, 12), (1, 1, 1, 1)], (2, 4)),
+    ((4, 6, 10, 20), [(1, 3, 5, 10), (1, 2, 10, 10), (2, 1, 5, 10)], (2,))])
+def test_sums_over_part_wavefronts(la, lto, gpu_ctx, shape, tiles, schedules):
+    """WilsonLoop, PlaquetteSum and the plaquette of an update under tiles whose blocks end in a
+    part of a wavefront, against the oracle to 1e-12 as under every other tile."""
+    U = lto.stout(lto.haar(shape, 6), shape, 0.1, 2)
+    chain = lto.new_field(shape)
+    loops = [(0, 1, True), (1, 3, False)]
+    ref = [lto.plaquette_sum(U, shape)] + [lto.wilson_loop(U, chain, shape, *n) for n in loops]
+    for tile in tiles:
+        flush(f"part wavefronts {shape} {tile}")
+        f = la.GaugeField(gpu_ctx, shape)
+        f.upload(U)
+        f.set_rng(3, 0)
+        f.set_tile(*tile)
+        ch = la.MatrixField(gpu_ctx, shape)
+        got = [la.PlaquetteSum(f)] + [la.WilsonLoop(*n, f, ch) for n in loops]
+        for a, b in zip(got, ref):
+            assert abs(a - b) <= 1e-12 * max(1.0, abs(b)), (tile, got, ref)
+        for schedule in schedules:
+            p = la.UpdateSweeps(f, 6.0, 1, 1, 2, schedule)
+            want = lto.plaquette_sum(f.download(), shape)
+            assert abs(p[1] - want) <= 1e-12 * abs(want), (tile, schedule, p[1], want)
+        f.close()
+        ch.close()
