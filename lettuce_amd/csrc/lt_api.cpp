@@ -176,8 +176,8 @@ double* lt_ctx_s::scratch_for(size_t n)
         if (scratch) LT_HIP_CHECK(hipFree(scratch));
         scratch = nullptr;
         scratch_doubles = 0;
-        if (hipMalloc(&scratch, n * sizeof(double)) != hipSuccess)
-            throw lt::LtError{LT_ENOMEM, "scratch allocation failed"};
+        scratch = (double*)device_alloc(n * sizeof(double));
+        if (!scratch) throw lt::LtError{LT_ENOMEM, "scratch allocation failed"};
         scratch_doubles = n;
     }
     return scratch;
@@ -385,8 +385,9 @@ int lt_ctx_read_rate(lt_ctx ctx, size_t footprint_bytes, double* bytes_per_s)
             if (e1) (void)hipEventDestroy(e1);
         };
         try {
-            LT_HIP_CHECK(hipMalloc(&buf, footprint_bytes));
-            LT_HIP_CHECK(hipMalloc(&out, (size_t)lanes * sizeof(double2)));
+            buf = (double2*)ctx->device_alloc(footprint_bytes);
+            out = (double2*)ctx->device_alloc((size_t)lanes * sizeof(double2));
+            if (!buf || !out) throw lt::LtError{LT_EHIP, "read-rate buffer allocation failed"};
             LT_HIP_CHECK(hipMemsetAsync(buf, 0, footprint_bytes, ctx->stream));
             LT_HIP_CHECK(hipEventCreate(&e0));
             LT_HIP_CHECK(hipEventCreate(&e1));

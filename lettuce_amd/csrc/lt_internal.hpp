@@ -79,9 +79,10 @@ struct lt_ctx_s {
     // second link buffer of multi-level smearing, grown on demand and kept: allocating and
     // freeing 382 MB in every call took 9 ms where two stout levels of that field take 0.65 ms.
     // One buffer per context, of the largest field smeared so far; given back with the
-    // context's last handle, and when another allocation of the context fails.  A caller
-    // holds links_mutex while it enqueues the launches that use the buffer (they are ordered
-    // by the stream), so threads sharing a context do not interleave on it.
+    // context's last handle, and when another allocation of the library on this context fails
+    // (all of them go through device_alloc).  A caller holds links_mutex while it enqueues the
+    // launches that use the buffer (they are ordered by the stream), so threads sharing a context
+    // do not interleave on it.
     std::mutex links_mutex;
     double2* links = nullptr;
     size_t links_n = 0;

@@ -48,9 +48,9 @@ std::string hex_of(uint64_t v)
 
 struct DeviceBuf {
     void* p = nullptr;
-    explicit DeviceBuf(size_t bytes)
+    DeviceBuf(lt_ctx ctx, size_t bytes)
     {
-        if (bytes && hipMalloc(&p, bytes) != hipSuccess) throw lt::LtError{LT_ENOMEM, "BMW staging allocation failed"};
+        if (bytes && !(p = ctx->device_alloc(bytes))) throw lt::LtError{LT_ENOMEM, "BMW staging allocation failed"};
     }
     ~DeviceBuf() { (void)hipFree(p); }
 };
@@ -88,7 +88,7 @@ uint64_t pack_pass(lt_field f, int K, std::FILE* out)
     const long long V = f->g.V, slab = slab_sites(f->g, K);
     const size_t slab_bytes = (size_t)slab * 4 * K * sizeof(uint64_t);
     const long long nb = (slab + BS - 1) / BS;
-    DeviceBuf d_out(out ? slab_bytes : 0), d_part(2 * nb * sizeof(uint64_t));
+    DeviceBuf d_out(ctx, out ? slab_bytes : 0), d_part(ctx, 2 * nb * sizeof(uint64_t));
     PinnedBuf h_out(out ? slab_bytes : 0), h_part(2 * nb * sizeof(uint64_t));
     uint64_t A = 0, B = 0;
     for (long long n0 = 0; n0 < V; n0 += slab) {
@@ -182,7 +182,7 @@ int lt_field_load_bmw(lt_field f, const char* path, int full_rows, int* checksum
         const long long V = f->g.V, slab = slab_sites(f->g, K);
         const size_t slab_bytes = (size_t)slab * 4 * K * sizeof(uint64_t);
         const long long nb = (slab + BS - 1) / BS;
-        DeviceBuf d_in(slab_bytes), d_part(2 * nb * sizeof(uint64_t)), d_dev(nb * sizeof(double));
+        DeviceBuf d_in(ctx, slab_bytes), d_part(ctx, 2 * nb * sizeof(uint64_t)), d_dev(ctx, nb * sizeof(double));
         PinnedBuf h_in(slab_bytes), h_part(2 * nb * sizeof(uint64_t)), h_dev(nb * sizeof(double));
         uint64_t A = 0, B = 0;
         double dev_row2 = 0.0;

@@ -248,10 +248,10 @@ LinkMap tune(lt_ctx ctx, const std::vector<LinkMap>& cands, const LinkMap& incum
 
 namespace {
 
-double2* scratch_links(size_t n)
+double2* scratch_links(lt_ctx ctx, size_t n)
 {
-    double2* p = nullptr;
-    if (hipMalloc(&p, n * sizeof(double2)) != hipSuccess) throw lt::LtError{LT_ENOMEM, "tuner scratch allocation failed"};
+    auto* p = (double2*)ctx->device_alloc(n * sizeof(double2));
+    if (!p) throw lt::LtError{LT_ENOMEM, "tuner scratch allocation failed"};
     return p;
 }
 
@@ -271,7 +271,7 @@ extern "C" int lt_autotune_field(lt_field f, int family, const char* cache_path,
             lt_ctx ctx = f->ctx;
             const size_t nl = (size_t)72 * f->g.Vh;
             // work on scratch copies: the field itself is not modified
-            double2* a = scratch_links(nl);
+            double2* a = scratch_links(ctx, nl);
             double2* b = nullptr;
             double2* z = nullptr;
             try {
@@ -292,8 +292,8 @@ extern "C" int lt_autotune_field(lt_field f, int family, const char* cache_path,
                     m = lt::tune(ctx, lt::tile_candidates(f->g, 0), d, run, ms, 3);
                     m = lt::tune(ctx, lt::order_candidates(m), m, run, ms, 3);
                 } else {
-                    b = scratch_links(nl);
-                    z = scratch_links((size_t)32 * f->g.Vh);
+                    b = scratch_links(ctx, nl);
+                    z = scratch_links(ctx, (size_t)32 * f->g.Vh);
                     auto run = [&](const lt::LinkMap& c) {
                         lt::k_flow_stage(ctx, f->g, c, a, b, z, 0.0, 0.01, 0.25, 0, 1);
                     };

@@ -250,8 +250,12 @@ void k_update_graph(lt_field u, double beta, int n_hb, int n_or, int schedule, i
     if (!u->ug) u->ug = new UpdateGraph();
     UpdateGraph& G = *u->ug;
     const int with_plaq = plaq_host ? 1 : 0;
-    if (!G.state && hipMalloc(&G.state, 2 * sizeof(uint64_t)) != hipSuccess)
-        throw LtError{LT_ENOMEM, "update graph allocation failed"};
+    auto alloc = [&](size_t bytes) {
+        void* p = ctx->device_alloc(bytes);
+        if (!p) throw LtError{LT_ENOMEM, "update graph allocation failed"};
+        return p;
+    };
+    if (!G.state) G.state = (uint64_t*)alloc(2 * sizeof(uint64_t));
     // plaquette partials: one per block of the field's present link map
     const unsigned np = plaq_parts(u->map);
     if (np > G.part_cap) {
@@ -259,8 +263,7 @@ void k_update_graph(lt_field u, double beta, int n_hb, int n_or, int schedule, i
         if (G.part) LT_HIP_CHECK(hipFree(G.part));
         G.part = nullptr;
         G.part_cap = 0;
-        if (hipMalloc(&G.part, (size_t)np * sizeof(double)) != hipSuccess)
-            throw LtError{LT_ENOMEM, "update graph allocation failed"};
+        G.part = (double*)alloc((size_t)np * sizeof(double));
         G.part_cap = np;
     }
     G.nb = np;
@@ -269,8 +272,7 @@ void k_update_graph(lt_field u, double beta, int n_hb, int n_or, int schedule, i
         if (G.plaq) LT_HIP_CHECK(hipFree(G.plaq));
         G.plaq = nullptr;
         G.cap = 0;
-        if (hipMalloc(&G.plaq, (size_t)n_update * sizeof(double)) != hipSuccess)
-            throw LtError{LT_ENOMEM, "update graph allocation failed"};
+        G.plaq = (double*)alloc((size_t)n_update * sizeof(double));
         G.cap = (size_t)n_update;
     }
     if (!G.exec || G.d != u->d || !same_map(G.m, u->map) || G.seed != u->seed || G.beta != beta || G.n_hb != n_hb ||

@@ -1,0 +1,72 @@
+"""Host paths of the library without a GPU: the HIP runtime is replaced by tests/cpp/host_hip.cpp,
+which keeps device memory on the host under a limit and counts kernels instead of running them.
+Each case runs in a process of its own, where the replacement is loaded before the library."""
+import ctypes
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+L16 = (16, 16, 16, 16)
+
+
+@pytest.fixture(scope="module")
+def host_hip(tmp_path_factory):
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    so = str(tmp_path_factory.mktemp("host") / "host_hip.so")
+    subprocess.run([hipcc, "-x", "hip", "--offload-host-only", "-std=c++17", "-O1", "-w", "-shared", "-fPIC",
+                    os.path.join(ROOT, "tests", "cpp", "host_hip.cpp"), "-o", so], check=True, timeout=300)
+    return so
+
+
+# ---------------------------------------------------------------- the cases, in a process of their own
+
+def check_memory(h, la, call):
+    """A context that keeps a smearing buffer gives it back to the call that needs its memory."""
+    ctx = la.Context(0)
+    a, b = la.GaugeField(ctx, L16), la.GaugeField(ctx, L16)
+    before = h.host_used()
+    la.StoutSmearingN(a, b, 2, 0.12)
+    kept = h.host_used() - before
+    spare = 0
+    if call == "scratch":
+        run = lambda: la.TopChargeCloverDensity(a)
+    elif call == "read_rate":
+        run = lambda: ctx.read_rate(1 << 16)
+    elif call == "tune_sweep":
+        run, spare = lambda: a.autotune("sweep"), kept // 2
+    elif call == "tune_flow":
+        run, spare = lambda: a.autotune("flow"), 3 * kept // 2
+    elif call == "update":
+        run = lambda: la.UpdateSweeps(a, 6.0, 1, 1, 2)
+    elif call == "checksum":
+        run = lambda: a.bmw_checksum()
+    h.host_limit(h.host_used() + spare)
+    run()
+
+
+CASES = {f"memory_{c}": (lambda h, la, c=c: check_memory(h, la, c))
+         for c in ("scratch", "read_rate", "tune_sweep", "tune_flow", "update", "checksum")}
+
+
+@pytest.mark.parametrize("case", sorted(CASES))
+def test_host_path(host_hip, case):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), host_hip, case], capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+if __name__ == "__main__":
+    h = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+    h.host_used.restype = ctypes.c_size_t
+    h.host_limit.argtypes = [ctypes.c_size_t]
+    h.host_copies_to_host.restype = ctypes.c_long
+    h.host_launches.restype = ctypes.c_long
+    sys.path.insert(0, ROOT)
+    import lettuce_amd
+    CASES[sys.argv[2]](h, lettuce_amd)
