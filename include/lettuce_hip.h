@@ -118,7 +118,7 @@ int lt_field_get_rng(lt_field f, uint64_t *seed, uint64_t *counter);
  * (tt, tx, ty, tz) in (t, x, y, z/2), which must divide the lattice, or, with
  * tt = tx = ty = 0, tz consecutive checkerboard sites (tz = 64, 128, 192 or 256);
  * results do not depend on it (no reference counterpart: the reference's OpenMP
- * schedule) */
+ * schedule).  get: the tile that was set or tuned last. */
 int lt_field_set_tile(lt_field f, int tt, int tx, int ty, int tz);
 int lt_field_get_tile(lt_field f, int tile[4]);
 
@@ -404,9 +404,10 @@ int lt_batch_results(lt_batch b, double *dH, int *accepted, double *cv, int *lab
  * have no launch shape).  Times the candidate thread-block tiles of the link
  * kernels on scratch copies and keeps the fastest; results are bit-identical for
  * every tile.  cache_path (may be NULL) is a JSON file of tuned tiles keyed by GPU
- * architecture, extents and kernel family; a cached entry is applied without timing. */
+ * architecture, extents and kernel family; a cached entry is applied without timing.
+ * Each family has a tile of its own in the field, lt_field_set_tile sets both. */
 #define LT_TUNE_SWEEP 1   /* the plaquette pass of an update (its colour launches have a fixed shape) */
-#define LT_TUNE_FLOW  2   /* stout / Wilson-flow stage kernels */
+#define LT_TUNE_FLOW  2   /* every other link kernel; times the stout / Wilson-flow stage */
 int lt_autotune_field(lt_field f, int family, const char *cache_path, int tile_out[4], double *best_ms);
 /* per distinct replica extent: the tile of the batched MetaD force kernels */
 int lt_batch_autotune(lt_batch b, const char *cache_path);

@@ -163,14 +163,16 @@ class GaugeField:
         call("lt_field_set_tile", self._h, tt, tx, ty, tz)
 
     def get_tile(self):
+        """The tile that was set or tuned last."""
         t = (ctypes.c_int * 4)()
         call("lt_field_get_tile", self._h, t)
         return tuple(t)
 
     def autotune(self, family="sweep", cache=None):
-        """Time the candidate tiles of the sweep or flow kernels on scratch copies of this
-        field, apply the fastest; cache: optional JSON file of tuned tiles.
-        Returns (tile, ms per launch)."""
+        """Time the candidate tiles on scratch copies of this field, apply the fastest: of the
+        plaquette pass of an update ("sweep"; its colour launches have a fixed shape) or of the
+        other link kernels by the flow stage ("flow"), each leaving the other's tile alone.
+        cache: optional JSON file of tuned tiles.  Returns (tile, ms per launch)."""
         t = (ctypes.c_int * 4)()
         ms = ctypes.c_double()
         code = {"sweep": 1, "flow": 2}[family]

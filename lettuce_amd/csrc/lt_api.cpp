@@ -449,7 +449,7 @@ int lt_field_create(lt_ctx ctx, int nt, int nx, int ny, int nz, lt_field* out)
         auto* f = new lt_field_s();
         f->ctx = ctx;
         f->g = lt::make_geom(nt, nx, ny, nz);
-        f->map = lt::default_linkmap(f->g);
+        f->set_map(lt::default_linkmap(f->g));
         try {
             f->d = alloc_links(ctx, f->g);
         } catch (...) {
@@ -612,14 +612,15 @@ int lt_field_set_tile(lt_field f, int tt, int tx, int ty, int tz)
     lt::LinkMap m{};
     if (!lt::make_linkmap(f->g, tt, tx, ty, tz, m))
         return fail(LT_EINVAL, "lt_field_set_tile: tile must divide (Nt, Nx, Ny, Nz/2) with 1..1024 threads");
-    f->map = m;
+    f->set_map(m);
     return LT_OK;
 }
 
 int lt_field_get_tile(lt_field f, int tile[4])
 {
     if (!f || !tile) return fail(LT_EINVAL, "null argument");
-    for (int i = 0; i < 4; ++i) tile[i] = f->map.lin && i < 3 ? 0 : f->map.T[i];
+    const lt::LinkMap& m = f->last_map();
+    for (int i = 0; i < 4; ++i) tile[i] = m.lin && i < 3 ? 0 : m.T[i];
     return LT_OK;
 }
 

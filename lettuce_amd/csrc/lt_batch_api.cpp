@@ -336,7 +336,7 @@ int lt_batch_create(lt_ctx ctx, int n_rep, const int* shapes, int n_levels, doub
                 auto* v = new lt_field_s();
                 v->ctx = ctx;
                 v->g = b->reps[r].g;
-                v->map = lt::default_linkmap(v->g);
+                v->set_map(lt::default_linkmap(v->g));
                 v->su3 = true;
                 v->view = true;
                 v->d = b->U + b->reps[r].off;
@@ -533,7 +533,7 @@ int lt_batch_autotune(lt_batch b, const char* cache_path)
                 lt::store_tile(cache_path, key, best, ms);
             }
             apply(best);
-            for (int q : same) b->views[q]->map = best;
+            for (int q : same) b->views[q]->set_map(best);
         }
         LT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
         return LT_OK;

@@ -136,8 +136,8 @@ void k_cb4_colour_action(lt_field u, bool heatbath, int mu, int colour, double p
 
 void k_cb4_plaq_partials(lt_field u, double* part)
 {
-    launch(u->ctx, "plaquette", cb4_plaq_kernel, dim3(8 * map_blocks(u->map)), sum_block(u->map), 0,
-           (const double2*)u->d, u->g, u->map, part);
+    launch(u->ctx, "plaquette", cb4_plaq_kernel, dim3(8 * map_blocks(u->plaq_map)), sum_block(u->plaq_map), 0,
+           (const double2*)u->d, u->g, u->plaq_map, part);
 }
 
 }  // namespace lt

@@ -103,13 +103,22 @@ struct UpdateGraph;   // captured local-update loop body of a field (lt_update_s
 struct lt_field_s {
     lt_ctx ctx = nullptr;
     lt::Geom g{};
-    lt::LinkMap map{};         // thread -> site tiling of the per-parity link kernels
+    // thread -> site tiling of the per-parity link kernels, and of the plaquette pass, which
+    // tuning the sweeps sets alone (the other kernels gain nothing from what suits that pass)
+    lt::LinkMap map{}, plaq_map{};
+    bool plaq_map_last = false;   // the tile set or tuned last is the plaquette pass's
     bool su3 = true;           // rows 0,1 stored, row 2 implied (false: general 3x3 matrices)
     bool view = false;         // d belongs to a replica batch (not freed, not swappable)
     double2* d = nullptr;      // 4 * 2 * 9 * Vh complex doubles
     uint64_t seed = 0;
     uint64_t counter = 0;
     lt::UpdateGraph* ug = nullptr;
+    void set_map(const lt::LinkMap& m)
+    {
+        map = plaq_map = m;
+        plaq_map_last = false;
+    }
+    const lt::LinkMap& last_map() const { return plaq_map_last ? plaq_map : map; }
     size_t bytes() const { return (size_t)72 * g.Vh * sizeof(double2); }
 };
 
@@ -328,7 +337,7 @@ void k_cb4_colour(lt_field u, bool heatbath, int mu, int colour, double prefacto
 void k_cb4_colour_graph_hb(lt_field u, int mu, int colour, double prefactor, const uint64_t* state, int k);
 void k_cb4_colour_action(lt_field u, bool heatbath, int mu, int colour, double prefactor, uint64_t counter,
                          double c_plaq, double c_rect, const char* name);
-void k_cb4_plaq_partials(lt_field u, double* part);   // one partial per block of u->map's launch
+void k_cb4_plaq_partials(lt_field u, double* part);   // one partial per block of u->plaq_map's launch
 // n_update x (n_hb heatbath + n_or overrelaxation sweeps) as one graph replayed per
 // update, PlaquetteSum after each into plaq_host (may be null); and its teardown
 void k_update_graph(lt_field u, double beta, int n_hb, int n_or, int schedule, int n_update, double* plaq_host);
@@ -347,6 +356,8 @@ void k_observables(lt_field u, double* host_out);
 // sum over sites and planes of Re tr P, the planes of a site spread over its links (the HMC
 // Hamiltonian keeps k_plaquette_sum, a plane pair per lane, which the replica batch repeats)
 double k_plaquette_planes(lt_field u);
+// its pass over the field alone: block sums into the context's scratch, whose number is returned
+unsigned k_plaquette_partials(lt_field u);
 // per-site clover charge density (V doubles, lexicographic order) into host memory
 void k_topcharge_density(lt_field u, double* host_q);
 // the fixed observables scratch of lt_observables_noalloc: its address on `device`

@@ -283,11 +283,12 @@ extern "C" int lt_autotune_field(lt_field f, int family, const char* cache_path,
                 // shape; the field's default map is the incumbent
                 const lt::LinkMap d = lt::default_linkmap(f->g);
                 if (family == LT_TUNE_SWEEP) {
-                    // the colour launches have their own block shape and order; the
-                    // plaquette pass of an update runs over the map
+                    // the colour launches have their own block shape and order; what of an
+                    // update runs over a map is the plaquette pass, timed without its sum's
+                    // way to the host
                     auto run = [&](const lt::LinkMap& c) {
-                        tmp.map = c;
-                        (void)lt::k_plaquette_planes(&tmp);
+                        tmp.plaq_map = c;
+                        (void)lt::k_plaquette_partials(&tmp);
                     };
                     m = lt::tune(ctx, lt::tile_candidates(f->g, 0), d, run, ms, 3);
                     m = lt::tune(ctx, lt::order_candidates(m), m, run, ms, 3);
@@ -311,7 +312,8 @@ extern "C" int lt_autotune_field(lt_field f, int family, const char* cache_path,
                 if (p) (void)hipFree(p);
             lt::store_tile(cache_path, key, m, ms);
         }
-        f->map = m;
+        f->plaq_map_last = family == LT_TUNE_SWEEP;
+        (f->plaq_map_last ? f->plaq_map : f->map) = m;
         if (tile_out)
             for (int i = 0; i < 4; ++i) tile_out[i] = m.lin && i < 3 ? 0 : m.T[i];
         if (best_ms) *best_ms = ms;

@@ -234,8 +234,8 @@ void enqueue_update(lt_field u, UpdateGraph& G, double prefactor)
         if (G.schedule == LT_CB4)
             k_cb4_plaq_partials(u, G.part);
         else
-            launch(ctx, "plaquette", upd_plaq_kernel, dim3(8 * map_blocks(u->map)), sum_block(u->map), 0,
-                   (const double2*)u->d, u->g, u->map, G.part);
+            launch(ctx, "plaquette", upd_plaq_kernel, dim3(8 * map_blocks(u->plaq_map)), sum_block(u->plaq_map), 0,
+                   (const double2*)u->d, u->g, u->plaq_map, G.part);
         launch(ctx, "reduce_finish", upd_plaq_finish_kernel, dim3(1), dim3(RBS), 0, (const double*)G.part, (int)G.nb,
                (const uint64_t*)G.state, G.plaq);
     }
@@ -256,8 +256,8 @@ void k_update_graph(lt_field u, double beta, int n_hb, int n_or, int schedule, i
         return p;
     };
     if (!G.state) G.state = (uint64_t*)alloc(2 * sizeof(uint64_t));
-    // plaquette partials: one per block of the field's present link map
-    const unsigned np = plaq_parts(u->map);
+    // plaquette partials: one per block of the pass's present map
+    const unsigned np = plaq_parts(u->plaq_map);
     if (np > G.part_cap) {
         G.drop_exec();
         if (G.part) LT_HIP_CHECK(hipFree(G.part));
@@ -275,11 +275,11 @@ void k_update_graph(lt_field u, double beta, int n_hb, int n_or, int schedule, i
         G.plaq = (double*)alloc((size_t)n_update * sizeof(double));
         G.cap = (size_t)n_update;
     }
-    if (!G.exec || G.d != u->d || !same_map(G.m, u->map) || G.seed != u->seed || G.beta != beta || G.n_hb != n_hb ||
+    if (!G.exec || G.d != u->d || !same_map(G.m, u->plaq_map) || G.seed != u->seed || G.beta != beta || G.n_hb != n_hb ||
         G.n_or != n_or || G.schedule != schedule || G.with_plaq != with_plaq) {
         G.drop_exec();
         G.d = u->d;
-        G.m = u->map;
+        G.m = u->plaq_map;
         G.seed = u->seed;
         G.beta = beta;
         G.n_hb = n_hb;
@@ -316,13 +316,19 @@ void k_update_graph(lt_field u, double beta, int n_hb, int n_or, int schedule, i
     LT_HIP_CHECK(hipStreamSynchronize(ctx->stream));
 }
 
+unsigned k_plaquette_partials(lt_field u)
+{
+    const unsigned nb = plaq_parts(u->plaq_map);
+    launch(u->ctx, "plaquette", upd_plaq_kernel, dim3(nb), sum_block(u->plaq_map), 0, (const double2*)u->d, u->g,
+           u->plaq_map, u->ctx->scratch_for((size_t)nb + 1));
+    return nb;
+}
+
 double k_plaquette_planes(lt_field u)
 {
     lt_ctx ctx = u->ctx;
-    const unsigned nb = plaq_parts(u->map);
-    double* part = ctx->scratch_for((size_t)nb + 1);
-    launch(ctx, "plaquette", upd_plaq_kernel, dim3(8 * map_blocks(u->map)), sum_block(u->map), 0,
-           (const double2*)u->d, u->g, u->map, part);
+    const unsigned nb = k_plaquette_partials(u);
+    double* part = ctx->scratch;
     launch(ctx, "plaquette_sum", plaq_sum_kernel, dim3(1), dim3(RBS), 0, (const double*)part, (int)nb, part + nb);
     double* h = ctx->host_for(1);
     LT_HIP_CHECK(hipMemcpyAsync(h, part + nb, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));

@@ -2,6 +2,7 @@
 which keeps device memory on the host under a limit and counts kernels instead of running them.
 Each case runs in a process of its own, where the replacement is loaded before the library."""
 import ctypes
+import json
 import os
 import shutil
 import subprocess
@@ -50,8 +51,36 @@ def check_memory(h, la, call):
     run()
 
 
+def check_tune_sweep(h, la):
+    """Tuning the sweeps sets the tile of the plaquette pass alone, tuning the flow that of the
+    other link kernels; nothing comes to the host while the pass is timed."""
+    ctx = la.Context(0)
+    a, b = la.GaugeField(ctx, L16), la.GaugeField(ctx, L16)
+    cache = os.path.join(os.path.dirname(sys.argv[1]), "tiles.json")
+
+    def blocks():
+        la.StoutSmearingN(a, b, 1, 0.12)
+        la.PlaquetteSum(a)
+        la.UpdateSweeps(a, 6.0, 1, 1, 1, 4)
+        return [h.host_block(k) for k in (b"stout_kernel", b"upd_plaq_kernel", b"cb4_plaq_kernel")]
+
+    assert blocks() == [128, 128, 128]
+    with open(cache, "w") as f:
+        json.dump({"gfx950|16x16x16x16|sweep": [2, 2, 4, 4, 1.0], "gfx950|16x16x16x16|flow": [1, 2, 16, 8, 1.0]}, f)
+    assert a.autotune("sweep", cache)[0] == a.get_tile() == (2, 2, 4, 4)
+    assert blocks() == [128, 64, 64]
+    assert a.autotune("flow", cache)[0] == a.get_tile() == (1, 2, 16, 8)
+    assert blocks() == [256, 64, 64]
+    a.set_tile(1, 1, 8, 8)
+    assert a.get_tile() == (1, 1, 8, 8) and blocks() == [64, 64, 64]
+    n = h.host_copies_to_host()
+    a.autotune("sweep")
+    assert h.host_copies_to_host() == n
+
+
 CASES = {f"memory_{c}": (lambda h, la, c=c: check_memory(h, la, c))
          for c in ("scratch", "read_rate", "tune_sweep", "tune_flow", "update", "checksum")}
+CASES["tune_sweep"] = check_tune_sweep
 
 
 @pytest.mark.parametrize("case", sorted(CASES))
