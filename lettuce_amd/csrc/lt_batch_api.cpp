@@ -533,7 +533,6 @@ int lt_batch_autotune(lt_batch b, const char* cache_path)
                 lt::store_tile(cache_path, key, best, ms);
             }
             apply(best);
-            for (int q : same) b->views[q]->set_map(best);
         }
         LT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
         return LT_OK;

@@ -78,9 +78,19 @@ def check_tune_sweep(h, la):
     assert h.host_copies_to_host() == n
 
 
+def check_batch_views(h, la):
+    """Tuning a batch leaves the tiles of its replicas' fields alone: it tries only blocks of the
+    batch's own size, the single-lattice kernels have another on large lattices."""
+    b = la.ReplicaBatch(la.Context(0), [L16, (8, 8, 8, 8)], 2, 0.12)
+    before = [b.field(r).get_tile() for r in range(2)]
+    b.autotune()
+    assert [b.field(r).get_tile() for r in range(2)] == before
+
+
 CASES = {f"memory_{c}": (lambda h, la, c=c: check_memory(h, la, c))
          for c in ("scratch", "read_rate", "tune_sweep", "tune_flow", "update", "checksum")}
 CASES["tune_sweep"] = check_tune_sweep
+CASES["batch_views"] = check_batch_views
 
 
 @pytest.mark.parametrize("case", sorted(CASES))
