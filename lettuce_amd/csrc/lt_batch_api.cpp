@@ -510,10 +510,13 @@ int lt_batch_autotune(lt_batch b, const char* cache_path)
                 upload(b->d_reps, b->reps.data(), sizeof(lt::BatchRep) * b->n);
             };
             // the replica's block range was sized for the map in use: a new map must need the
-            // same number of blocks (fewer would leave links out)
+            // same number of blocks (fewer would leave links out) of at most as many threads (a
+            // linear map of more gives a small lattice as many blocks, and its lanes' LDS slots lie
+            // that many apart, past the LDS of the launched block)
             const lt::LinkMap cur = b->reps[same[0]].m;
             const unsigned nb = lt::map_blocks(cur);
-            if (!lt::cached_tile(cache_path, key, g, best, ms) || lt::map_blocks(best) != nb) {
+            if (!lt::cached_tile(cache_path, key, g, best, ms) || lt::map_blocks(best) != nb ||
+                best.nthreads > cur.nthreads) {
                 const lt::BatchGrid bg = b->grid();
                 auto run = [&](const lt::LinkMap& m) {
                     apply(m);

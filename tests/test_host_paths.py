@@ -87,10 +87,26 @@ def check_batch_views(h, la):
     assert [b.field(r).get_tile() for r in range(2)] == before
 
 
+def check_batch_cache(h, la):
+    """A cached tile of more threads than the batch launches is not taken: its kernels would reach
+    past the LDS of their block."""
+    cache = os.path.join(os.path.dirname(sys.argv[1]), "batch.json")
+    key = "gfx950|2x2x2x2|batch64"
+    for entry in ([0, 0, 0, 128, 1.0], [0, 0, 0, 256, 1.0]):
+        with open(cache, "w") as f:
+            json.dump({key: entry}, f)
+        b = la.ReplicaBatch(la.Context(0), [(2, 2, 2, 2)], 2, 0.12)
+        b.autotune(cache)
+        with open(cache) as f:
+            tile = json.load(f)[key][:4]
+        assert tile == [0, 0, 0, 64], tile
+
+
 CASES = {f"memory_{c}": (lambda h, la, c=c: check_memory(h, la, c))
          for c in ("scratch", "read_rate", "tune_sweep", "tune_flow", "update", "checksum")}
 CASES["tune_sweep"] = check_tune_sweep
 CASES["batch_views"] = check_batch_views
+CASES["batch_cache"] = check_batch_cache
 
 
 @pytest.mark.parametrize("case", sorted(CASES))
