@@ -46,7 +46,7 @@ bool make_linkmap(const Geom& g, int tt, int tx, int ty, int tz, LinkMap& m)
         m.T[3] = tz;
         m.N[0] = (g.Vh + tz - 1) / tz;
         m.N[1] = m.N[2] = m.N[3] = 1;
-        m.tc = m.yc = m.ycs = 1;
+        m.tc = m.yc = 1;
         m.xr = LT_XCD_REMAP;
         finish_map(m);
         return true;
@@ -76,7 +76,6 @@ bool make_linkmap(const Geom& g, int tt, int tx, int ty, int tz, LinkMap& m)
 #if LT_YCHUNK > 0
     if (m.N[2] % LT_YCHUNK == 0) m.yc = LT_YCHUNK;
 #endif
-    m.ycs = m.N[2];
     m.xr = LT_XCD_REMAP;
     finish_map(m);
     return true;

@@ -1258,7 +1258,6 @@ struct LinkMap {
     int tc;       // t tiles per chunk (divides N[0])
     int yc;       // y tiles per chunk (divides N[2]) of the Jacobi kernels (flow, stout, MetaD)
     int lin;      // linear map: block b covers checkerboard sites [b * nthreads, (b + 1) * nthreads)
-    int ycs;      // kept with a tuned map's file entry; orders nothing
     int xr;       // spread the block index over the XCDs (xcd_block)
     // divisions of map_site_b, from the numbers above (finish_map)
     Div dtx, dty, dtz, dtc, dnz, dyc, dnx, dny;

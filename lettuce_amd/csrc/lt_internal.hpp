@@ -225,7 +225,7 @@ inline unsigned split_blocks(const Geom& g, const SplitMap& m) { return (unsigne
 inline unsigned map_blocks(const LinkMap& m)
 {
     if (m.nthreads < 1 || m.nthreads > LT_LINK_BS || m.T[0] * m.T[1] * m.T[2] * m.T[3] != m.nthreads || m.tc < 1
-        || m.N[0] % m.tc || m.yc < 1 || m.N[2] % m.yc || m.ycs < 1 || m.N[2] % m.ycs)
+        || m.N[0] % m.tc || m.yc < 1 || m.N[2] % m.yc)
         throw LtError{LT_ESTATE, "invalid thread-block tile for the link kernels"};
     return (unsigned)(m.N[0] * m.N[1] * m.N[2] * m.N[3]);
 }
@@ -308,8 +308,7 @@ inline bool same_map(const LinkMap& a, const LinkMap& b)
 {
     for (int i = 0; i < 4; ++i)
         if (a.T[i] != b.T[i] || a.N[i] != b.N[i]) return false;
-    return a.nthreads == b.nthreads && a.tc == b.tc && a.yc == b.yc && a.lin == b.lin && a.ycs == b.ycs &&
-           a.xr == b.xr;
+    return a.nthreads == b.nthreads && a.tc == b.tc && a.yc == b.yc && a.lin == b.lin && a.xr == b.xr;
 }
 
 // kernel launchers (defined in the .hip translation units)

@@ -109,9 +109,9 @@ std::string tune_key(int device, const Geom& g, const char* family)
 }
 
 // Cache file: one JSON object, "key": [tt, tx, ty, tz, ms, tc, yc, ycs, xr] per entry (tt =
-// tx = ty = 0: a linear map of tz consecutive checkerboard sites per block; tc, yc, ycs, xr:
-// the site order, see order_candidates; ycs belonged to colour kernels on the map and orders
-// nothing now; entries of five numbers keep the default order).
+// tx = ty = 0: a linear map of tz consecutive checkerboard sites per block; tc, yc, xr: the site
+// order, see order_candidates; ycs, the y chunk of colour kernels that ran over the map, orders
+// nothing but still has to divide; entries of five numbers keep the default order).
 static std::map<std::string, std::array<double, 9>> read_cache(const char* path)
 {
     std::map<std::string, std::array<double, 9>> m;
@@ -164,13 +164,13 @@ bool cached_tile(const char* path, const std::string& key, const Geom& g, LinkMa
     if (it == c.end()) return false;
     const auto& v = it->second;
     if (!make_linkmap(g, (int)v[0], (int)v[1], (int)v[2], (int)v[3], m)) return false;
-    if (v[5] >= 0.0) {   // site order: t chunk, y chunks (Jacobi, sweeps), XCD spread
+    if (v[5] >= 0.0) {   // site order: t chunk, y chunk, XCD spread
         LinkMap o = m;
         o.tc = (int)v[5];
         o.yc = (int)v[6];
-        o.ycs = (int)v[7];
         o.xr = (int)v[8];
-        if (o.tc < 1 || o.N[0] % o.tc || o.yc < 1 || o.N[2] % o.yc || o.ycs < 1 || o.N[2] % o.ycs) return false;
+        const int ycs = (int)v[7];
+        if (o.tc < 1 || o.N[0] % o.tc || o.yc < 1 || o.N[2] % o.yc || ycs < 1 || o.N[2] % ycs) return false;
         finish_map(o);
         m = o;
     }
@@ -183,7 +183,7 @@ void store_tile(const char* path, const std::string& key, const LinkMap& m, doub
     if (!path || !*path) return;
     auto c = read_cache(path);
     c[key] = {m.lin ? 0.0 : (double)m.T[0], m.lin ? 0.0 : (double)m.T[1], m.lin ? 0.0 : (double)m.T[2], (double)m.T[3], ms,
-              (double)m.tc, (double)m.yc, (double)m.ycs, (double)m.xr};
+              (double)m.tc, (double)m.yc, (double)m.N[2], (double)m.xr};
     write_cache(path, c);
 }
 
