@@ -158,7 +158,7 @@ int lt_update_sweeps(lt_field u, double beta, int n_hb, int n_or, int schedule, 
 /* ---- observables ---------------------------------------------------------- */
 /* PlaquetteSum (plaquette.hpp:26-43): sum over sites and the six planes of Re tr P, one
  * link (x, mu) per GPU lane with the planes (mu, mu+1 mod 4) and, for mu < 2, (mu, mu+2),
- * in the tile order of the field's link kernels; agrees with the plaquette of
+ * in the order of the pass's tile; agrees with the plaquette of
  * lt_observables to rounding */
 int lt_plaquette_sum(lt_field u, double *out);
 /* WilsonAction::Action / Rectangular<1>::Action (wilson_action.hpp:23-41) */

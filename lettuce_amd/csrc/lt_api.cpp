@@ -610,7 +610,7 @@ int lt_field_set_tile(lt_field f, int tt, int tx, int ty, int tz)
     if (!f) return fail(LT_EINVAL, "null field");
     lt::LinkMap m{};
     if (!lt::make_linkmap(f->g, tt, tx, ty, tz, m))
-        return fail(LT_EINVAL, "lt_field_set_tile: tile must divide (Nt, Nx, Ny, Nz/2) with 1..1024 threads");
+        return fail(LT_EINVAL, "lt_field_set_tile: tile must divide (Nt, Nx, Ny, Nz/2) with 1..256 threads");
     f->set_map(m);
     return LT_OK;
 }

@@ -31,7 +31,8 @@ constexpr int RBS = 256;
 // ones by the memory behind the L2.
 // Rectangle staple: one lane per link with the sum parked in LDS ran about 9500 FP64
 // instructions in a row at two waves per SIMD, 186 us per overrelaxation launch at 24^4 and 322
-// us at 32^4; now 81.6 and 199 us (heatbath 195 -> 92 us at 24^4).  About half of its lines miss
+// us at 32^4; now 81.6 and 199 us (heatbath 195 -> 92 us at 24^4: three wavefronts per SIMD with 22
+// registers, 60 bytes a lane, spilled; two without spills are no faster).  About half of its lines miss
 // the L2: 385 MB a launch at 24^4, 53 us at the rate at which the memory-side cache reads.
 template <bool HEATBATH, int KIND, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(split_eu(HEATBATH, KIND, WAVES))))

@@ -26,8 +26,8 @@
 #define LT_TCHUNK 1
 #endif
 // y tiles per chunk (LinkMap::yc; 0: all y tiles in one chunk).  Two y tiles per
-// chunk at 32^4 (8 tiles in flight per x step in each XCD): OR sweep -2 %, RK3 flow
-// step -1 % against one chunk; one y tile per chunk is slower.
+// chunk at 32^4 (8 tiles in flight per x step in each XCD): RK3 flow step -1 % against
+// one chunk; one y tile per chunk is slower.
 #ifndef LT_YCHUNK
 #define LT_YCHUNK 2
 #endif
@@ -722,7 +722,7 @@ __device__ __forceinline__ void gauss2(double u0, double u1, double& g0, double&
 // exceeds n / d by less than 1/d and the quotient is exact.  A division by a kernel argument
 // is about twenty VALU instructions otherwise, also where the operands are uniform; the maps
 // from a thread to its site take eight to ten of them (OR + HB updates of a 16^4 lattice 462 ->
-// 448 us, four colours at 20^4 2025 -> 1968 us, the heatbath launch at 32^4 128 -> 124 us).
+// 448 us, four colours at 28 x 20 x 12 x 36 2025 -> 1968 us, the heatbath launch at 32^4 128 -> 124 us).
 struct Div {
     uint32_t m;
     int sh;

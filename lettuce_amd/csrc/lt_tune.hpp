@@ -12,8 +12,7 @@ namespace lt {
 // tiles of `threads` threads (0: 64, 128 and 256; whole-row boxes: any multiple of 64 up
 // to 256) that divide the extents, z-major, linear maps, and the default map
 std::vector<LinkMap> tile_candidates(const Geom& g, int threads);
-// site orders (t / y chunking, XCD spread) of one block shape, for the colour sweeps
-// (sweeps = true) or the Jacobi kernels
+// site orders (t / y chunking, XCD spread) of one block shape
 std::vector<LinkMap> order_candidates(const LinkMap& base);
 // "<arch>|<Nt>x<Nx>x<Ny>x<Nz>|<family>"
 std::string tune_key(int device, const Geom& g, const char* family);
