@@ -77,7 +77,7 @@ struct lt_ctx_s {
     std::map<std::string, lt::ProfEntry> prof;
 
     // second link buffer of multi-level smearing, grown on demand and kept: allocating and
-    // freeing 382 MB in every call took 9 ms where two stout levels of that field take 0.65 ms.
+    // freeing 382 MB in every call took 6 to 9 ms where two stout levels of that field take 0.65 ms.
     // One buffer per context, of the largest field smeared so far; given back with the
     // context's last handle, and when another allocation of the library on this context fails
     // (all of them go through device_alloc).  A caller holds links_mutex while it enqueues the
