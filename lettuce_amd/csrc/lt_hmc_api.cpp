@@ -281,6 +281,23 @@ double hamiltonian(lt_field U, lt_field P, double beta, bool alg)
     return S + lt::k_kinetic(P, alg);
 }
 
+// f on momenta that are in 8 reals; they are whole matrices afterwards, also where f throws (out of
+// memory, say: a caller may go on with them)
+template <typename F>
+void with_momenta8(lt_field P, F f)
+{
+    try {
+        f();
+    } catch (...) {
+        try {
+            lt::k_momentum_whole(P);
+        } catch (...) {
+        }
+        throw;
+    }
+    lt::k_momentum_whole(P);
+}
+
 void copy_field(lt_field dst, lt_field src)
 {
     lt::k_copy(dst->ctx, src->d, dst->d, (size_t)72 * dst->g.Vh);
@@ -473,12 +490,15 @@ int lt_hmc_trajectory(lt_field U, lt_field P, lt_field U_copy, double beta, int 
         copy_field(U_copy, U);
         lt::k_random_momentum(P, U->seed, counter, true);
         P->su3 = false;
-        const double H0 = hamiltonian(U, P, beta, true);
-        integrate(
-            integrator, tau, n_step, [&](double e, bool) { lt::k_force_update(U, P, nullptr, e * beta / 6.0, 0.0, true); },
-            [&](double e) { lt::k_field_update(U, P, e, true); });
-        const double H1 = hamiltonian(U, P, beta, true);
-        lt::k_momentum_whole(P);
+        double H0 = 0.0, H1 = 0.0;
+        with_momenta8(P, [&] {
+            H0 = hamiltonian(U, P, beta, true);
+            integrate(
+                integrator, tau, n_step,
+                [&](double e, bool) { lt::k_force_update(U, P, nullptr, e * beta / 6.0, 0.0, true); },
+                [&](double e) { lt::k_field_update(U, P, e, true); });
+            H1 = hamiltonian(U, P, beta, true);
+        });
         const double d = H1 - H0;
         int acc = 1;
         if (metropolis) {
@@ -501,16 +521,18 @@ int lt_hmc_reversibility_test(lt_field U, lt_field P, double beta, int integrato
         // HMCKernel::ReversibilityTest (hmc_gauge.hpp:585-599)
         lt::k_random_momentum(P, U->seed, U->counter++, true);
         P->su3 = false;
-        const double H0 = hamiltonian(U, P, beta, true);
-        for (int pass = 0; pass < 2; ++pass) {
-            if (pass) lt::k_scale(U->ctx, P->d, -1.0, (size_t)72 * P->g.Vh);   // ReverseMomenta
-            integrate(
-                integrator, tau, n_step,
-                [&](double e, bool) { lt::k_force_update(U, P, nullptr, e * beta / 6.0, 0.0, true); },
-                [&](double e) { lt::k_field_update(U, P, e, true); });
-        }
-        const double H1 = hamiltonian(U, P, beta, true);
-        lt::k_momentum_whole(P);
+        double H0 = 0.0, H1 = 0.0;
+        with_momenta8(P, [&] {
+            H0 = hamiltonian(U, P, beta, true);
+            for (int pass = 0; pass < 2; ++pass) {
+                if (pass) lt::k_scale(U->ctx, P->d, -1.0, (size_t)72 * P->g.Vh);   // ReverseMomenta
+                integrate(
+                    integrator, tau, n_step,
+                    [&](double e, bool) { lt::k_force_update(U, P, nullptr, e * beta / 6.0, 0.0, true); },
+                    [&](double e) { lt::k_field_update(U, P, e, true); });
+            }
+            H1 = hamiltonian(U, P, beta, true);
+        });
         if (H_old) *H_old = H0;
         if (H_new) *H_new = H1;
         return LT_OK;
@@ -749,15 +771,16 @@ int lt_metad_hmc_trajectory(lt_field U, lt_field P, lt_field U_copy, lt_field F,
         lt::k_random_momentum(P, U->seed, counter, true);
         P->su3 = false;
         F->su3 = false;
-        const double cv_old = cv_charge(cv, U);
-        const double H0 = hamiltonian(U, P, beta, true) + bias->potential(cv_old);
         std::vector<double> samples;
-        samples.reserve(n_step);
-        double cv1 = cv_old;
-        metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, cv1, samples);
-        cv->path = samples;
-        const double H1 = hamiltonian(U, P, beta, true) + bias->potential(cv1);
-        lt::k_momentum_whole(P);
+        double cv_old = 0.0, cv1 = 0.0, H0 = 0.0, H1 = 0.0;
+        with_momenta8(P, [&] {
+            samples.reserve(n_step);
+            cv1 = cv_old = cv_charge(cv, U);
+            H0 = hamiltonian(U, P, beta, true) + bias->potential(cv_old);
+            metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, cv1, samples);
+            cv->path = samples;
+            H1 = hamiltonian(U, P, beta, true) + bias->potential(cv1);
+        });
         const double d = H1 - H0;
         int acc = 1;
         if (metropolis) {
@@ -818,14 +841,16 @@ int lt_metad_reversibility_test(lt_field U, lt_field P, lt_field F, lt_cv cv, lt
         lt::k_random_momentum(P, U->seed, U->counter++, true);
         P->su3 = false;
         F->su3 = false;
-        double q = cv_charge(cv, U);
-        const double H0 = hamiltonian(U, P, beta, true) + bias->potential(q);
-        std::vector<double> samples;
-        metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, q, samples);
-        lt::k_scale(U->ctx, P->d, -1.0, (size_t)72 * P->g.Vh);   // ReverseMomenta
-        metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, q, samples);
-        const double H1 = hamiltonian(U, P, beta, true) + bias->potential(q);
-        lt::k_momentum_whole(P);
+        double H0 = 0.0, H1 = 0.0;
+        with_momenta8(P, [&] {
+            double q = cv_charge(cv, U);
+            H0 = hamiltonian(U, P, beta, true) + bias->potential(q);
+            std::vector<double> samples;
+            metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, q, samples);
+            lt::k_scale(U->ctx, P->d, -1.0, (size_t)72 * P->g.Vh);   // ReverseMomenta
+            metad_integrate(U, P, F, cv, bias, beta, integrator, tau, n_step, q, samples);
+            H1 = hamiltonian(U, P, beta, true) + bias->potential(q);
+        });
         if (H_old) *H_old = H0;
         if (H_new) *H_new = H1;
         return LT_OK;

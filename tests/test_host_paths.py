@@ -102,8 +102,31 @@ def check_batch_cache(h, la):
         assert tile == [0, 0, 0, 64], tile
 
 
+def check_momenta(h, la, call):
+    """A trajectory that runs out of memory leaves its momenta as whole matrices, as one that ends:
+    in the 8 reals that it keeps them in, a caller that goes on with them would read other ones."""
+    ctx = la.Context(0)
+    U, V, P, F = la.GaugeField(ctx, L16), la.GaugeField(ctx, L16), la.MatrixField(ctx, L16), la.MatrixField(ctx, L16)
+    cv = la.CollectiveVariable(ctx, L16, 1, 0.12)
+    bias = la.MetaBiasPotential(-8.0, 8.0, 80, 1.5, 0.3, 10.0, 1000.0, well_tempered=False)
+    run = {"hmc": lambda: la.HMCKernel(U, V, P, "omf2", 6.0, 1.0)(2, False),
+           "hmc_reversibility": lambda: la.HMCKernel(U, V, P, "omf2", 6.0, 1.0).ReversibilityTest(2),
+           "metad": lambda: la.HMCMetaDKernel(U, V, P, F, bias, cv, "omf2", 6.0, 1.0)(2, False),
+           "metad_reversibility": lambda: la.HMCMetaDKernel(U, V, P, F, bias, cv, "omf2", 6.0, 1.0).ReversibilityTest(2)}[call]
+    h.host_limit(h.host_used())
+    try:
+        run()
+    except la.LettuceError as e:
+        assert "allocation failed" in str(e), e
+    else:
+        raise AssertionError("no scratch to be had, and no error")
+    assert h.host_launches(b"15momentum_kernelILb1E") == 1 and h.host_launches(b"momentum_entry_kernelILb1E") == 1
+
+
 CASES = {f"memory_{c}": (lambda h, la, c=c: check_memory(h, la, c))
          for c in ("scratch", "read_rate", "tune_sweep", "tune_flow", "update", "checksum")}
+CASES.update({f"momenta_{c}": (lambda h, la, c=c: check_momenta(h, la, c))
+              for c in ("hmc", "hmc_reversibility", "metad", "metad_reversibility")})
 CASES["tune_sweep"] = check_tune_sweep
 CASES["batch_views"] = check_batch_views
 CASES["batch_cache"] = check_batch_cache
